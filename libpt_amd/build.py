@@ -23,7 +23,9 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(ROOT, "_build", "obj")
 LIB = os.path.join(HERE, "libpt_amd.so")
 
-SOURCES = ["pt_kernel.hip", "pt_noalloc.hip", "pt_host.cpp", "pt_terms.cpp"]
+SOURCES = ["pt_tiles_fp64.hip", "pt_tiles_fp32.hip", "pt_tiles_bf16x3.hip",
+           "pt_tiles_f16x3.hip", "pt_kernel.hip", "pt_noalloc.hip",
+           "pt_host.cpp", "pt_terms.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

@@ -33,42 +33,42 @@ enum pt_kind { PT_AAA = 0, PT_AAB = 1 };
 enum pt_role { PT_ROLE_A = 0, PT_ROLE_B = 1, PT_ROLE_C = 2 };
 
 #define PT_MAX_TERMS 40
-#define PT_MAX_BUFS 24
+#define PT_MAX_BUFS 26
 
-/* kappa per group of the packed Q operands: one group of one (u, w) pair
- * is 32 bytes: 4 FP64, 8 FP32, or 8 split (hi, lo) pairs stored as
- * hi 2q, hi 2q+1, lo 2q, lo 2q+1 for q = 0 .. 3 */
+/* kappa per fragment of the packed Q operands: a fragment is 1 KB, 16 rows
+ * of 64 bytes (8 FP64, 16 FP32, or 16 split values: per 4 kappa hi 0-3 and
+ * lo 0-3), in the lane order of the MFMA operand: lane 16 g + row holds
+ * the row's g-th quarter */
+#define PT_FRAG 1024
 static inline int
 pt_kc(int form)
 {
-	return form == 0 ? 4 : 8;
+	return form == 0 ? 8 : 16;
 }
 
-static inline int
-pt_group_bytes(int form)
-{
-	(void)form;
-	return 32;
-}
-
-/* groups per packed slab of K kappa (zero padded), rounded up to an even
- * count: a step over a 16-wide w range takes two groups */
+/* kappa chunks of a slab of K kappa (zero padded) */
 static inline int64_t
-pt_kgroups(int form, int64_t K)
+pt_chunks(int form, int64_t K)
 {
-	const int64_t kc = pt_kc(form);
-	return 2 * ((K + 2 * kc - 1) / (2 * kc));
+	return (K + pt_kc(form) - 1) / pt_kc(form);
+}
+
+/* fragments of a packed slab [row block of 16][chunk][column]: rows and
+ * columns of the plane; tri: the pairs row > column of a square plane,
+ * block b holding its columns 0 .. 16 (b + 1) - 1 */
+static inline int64_t
+pt_slab_frags(int form, int64_t K, int64_t rows, int64_t cols, int tri)
+{
+	const int64_t nb = (rows + 15) / 16;
+	return pt_chunks(form, K) * (tri ? 8 * nb * (nb + 1) : nb * cols);
 }
 
 /* Workgroup geometry (the kernel's Geo): NW = 4 waves, tile 32 a x 32 b x
- * TC c with TC = 16 for FP64 (whose 16 x 16 x 16 accumulator block per
- * wave fills 128 registers) and 32 for FP32 and the split forms (FP32
- * accumulators), two workgroups per CU; or NW = 8 waves, tile 32 a x 32 b
- * x 32 c, one
- * workgroup per CU with four staging slots.  Each wave owns 16 a x 16 b x
- * CW c (CW = TC for four waves, 16 for eight).  (fT) forms its two W sets
- * one after the other in the same registers, so the geometry does not
- * depend on the W-set count. */
+ * TC c with TC = 16 for FP64 and 32 for FP32 and the split forms (128
+ * accumulator registers per lane either way), two workgroups per CU; or
+ * NW = 8 waves, tile 32 a x 32 b x 32 c, one workgroup per CU.  (fT) forms
+ * its two W sets one after the other in the same registers, so the
+ * geometry does not depend on the W-set count. */
 #define PT_TA 32
 #define PT_TB 32
 
@@ -96,23 +96,27 @@ pt_cw(int form, int nset, int nw)
 }
 
 /*
- * S operands are read in the API layout (kappa contiguous).  Q operands
- * [slab][kappa][plane] are read from packed copies
- * [slab][kappa / KC][plane][kappa % KC] (zero padded in kappa), so the KC
- * values of one (u, w) pair form one contiguous group.
+ * S operands are read in the API layout (kappa contiguous; the split forms
+ * from hi | lo << 16 copies), Q operands from packed copies (PT_FRAG).  The
+ * pair (u, w) is the two indices that S does not carry, in a, b, c order;
+ * the packed rows are u and the columns w, or (tr) rows w and columns u.
  */
 struct pt_term {
 	int64_t s_off[3];  /* S base offset (elements) = s_off . (i, j, k) */
-	int64_t q_off[3];  /* Q slab offset: in the API layout (elements) when
-	                      built, in bytes of the packed copy when launched */
+	int64_t q_off[3];  /* Q slab offset (bytes of the packed copy) */
 	int64_t s_st;      /* stride of the single index s (kappa stride 1) */
-	int64_t q_k;       /* plane size of Q (kappa stride in the API layout) */
-	int64_t q_st[3];   /* strides of a, b, c in the Q plane (S role unused) */
+	int64_t cols;      /* columns of the packed plane */
 	int32_t s_buf, q_buf;
 	int32_t role, set, sign, K;
-	int32_t packed;    /* Q pair (u > w) is a packed triangle u(u-1)/2 + w */
-	int32_t ufast;     /* u is the contiguous Q index (else w) */
+	int32_t nch;       /* kappa chunks */
+	int32_t tri;       /* packed triangle u > w (pt_slab_frags) */
+	int32_t tr;
+	int32_t pad_;
 };
+
+/* terms of one W set of a spin case */
+#define PT_TERMS_SAME 18
+#define PT_TERMS_MIXED 16
 
 /* epilogue inputs (element type: double, or float for PT_FORM_FP32) */
 struct pt_epi {
@@ -179,8 +183,12 @@ pt_ft_chunk(int form, int nw)
 	return ((int64_t)4 << 30) / pt_wsave_bytes(form, 2, nw);
 }
 
-/* kernel launchers (pt_kernel.hip); return hipError_t as int */
+/* kernel launchers (pt_tiles_*.hip, pt_kernel.hip); return hipError_t as int */
 int pt_launch_tiles(int form, const struct pt_launch *p, void *stream);
+int pt_launch_tiles_fp64(const struct pt_launch *p, void *stream);
+int pt_launch_tiles_fp32(const struct pt_launch *p, void *stream);
+int pt_launch_tiles_bf16x3(const struct pt_launch *p, void *stream);
+int pt_launch_tiles_f16x3(const struct pt_launch *p, void *stream);
 /* out[s] = fixed-order sum of segment s's partials (as pt_launch_reduce) */
 int pt_launch_reduce_batch(const struct pt_launch *segs,
     const int64_t *begin, int nseg, double *out, void *stream);
@@ -189,11 +197,12 @@ int pt_launch_segsum(const double *x, int64_t nseg, int64_t seglen,
     double *out, void *stream);
 int pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
     double scale, void *stream);
-/* [R][K][PL] -> [R][ceil(K/KC)][PL][KC] (mode 0 FP64, 1 FP32) or
- * [R][ceil(K/KC)][PL][hi KC][lo KC] halves (mode 2 BF16, 3 FP16, of x*scale);
- * P1 > 0: the plane [P1][PL / P1] is stored transposed */
+/* [R slabs][K][plane] -> packed slabs (pt_slab_frags) of the plane's rows
+ * and columns; the source plane is [rows][cols], [cols][rows] (tr), or the
+ * packed pairs row > column (tri); the split forms store hi and lo of
+ * x * scale */
 int pt_launch_pack(const void *src, void *dst, int64_t R, int64_t K,
-    int64_t nkb, int64_t PL, int KC, int mode, double scale, int64_t P1,
+    int64_t rows, int64_t cols, int tri, int tr, int form, double scale,
     void *stream);
 int pt_launch_absmax(const double *src, int64_t n, double *out, void *stream);
 int pt_launch_copy(const double *src, double *dst, int64_t n, void *stream);

@@ -307,11 +307,13 @@ struct libpt_amd_plan {
 	                               measured 10 % ahead of 1 for FP64 and
 	                               4 % for split-BF16 at o=45, v=477 (2, 8
 	                               and 16 within 1 % of 4) */
-	bool vct = true;            /* VC packed a second time, transposed */
+	bool copies = true;         /* transposed operand copies (pt_term.tr
+	                               is set without them) */
 	bool fixed_geometry = false; /* a batch's plan: its launches are
 	                                recorded, so the tuner keeps nw */
 	bool unusable = false;      /* a geometry or order change failed half
 	                               way: the tile lists are not whole */
+	bool no_room = false;       /* an allocation did not fit */
 	bool persist = false;       /* persistent grid (LIBPT_AMD_PERSISTENT) */
 	uint32_t *d_ctr = nullptr;  /* its 8 item counters */
 	int64_t oa = 0, va = 0, ob = 0, vb = 0;
@@ -370,6 +372,7 @@ dev_alloc(void **p, size_t bytes)
 	hipError_t e = hipMalloc(p, bytes ? bytes : 256);
 	if (e != hipSuccess) {
 		set_err("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+		(void)hipGetLastError(); /* a later launch check would see it */
 		*p = nullptr;
 		return false;
 	}
@@ -388,7 +391,9 @@ plan_alloc(libpt_amd_plan *pl, void **p, size_t bytes)
 		if (need > a.cap - a.used) {
 			set_err("the call needs more than the %zu bytes of static "
 			    "scratch of the allocation-free entry point (%zu in use, "
-			    "%zu more requested)", a.cap, a.used, need);
+			    "%zu more requested)", (size_t)LIBPT_AMD_NOALLOC_SCRATCH,
+			    a.used, need);
+			pl->no_room = true;
 			return false;
 		}
 		*p = a.base + a.used;
@@ -399,8 +404,10 @@ plan_alloc(libpt_amd_plan *pl, void **p, size_t bytes)
 		set_err("too many device buffers in one plan");
 		return false;
 	}
-	if (!dev_alloc(p, bytes))
+	if (!dev_alloc(p, bytes)) {
+		pl->no_room = true;
 		return false;
+	}
 	pl->owned.push_back(*p);
 	return true;
 }
@@ -609,18 +616,9 @@ case_finish(libpt_amd_plan *pl, Case &c, int form, int kind, int nset,
 	L.tcw = pt_tcw(form, nset, pl->nw);
 	for (int s = 0; s < nset; ++s) {
 		if (kind == PT_AAA)
-			pt_terms_same(c.terms, s, oa, va);
+			pt_terms_same(c.terms, form, s, oa, va, pl->copies);
 		else
-			pt_terms_mixed(c.terms, s, oa, va, ob, vb, pl->vct);
-	}
-	/* Q slab offsets: API elements (K q_k per slab) -> bytes of the
-	 * packed copy (pt_kgroups q_k groups per slab) */
-	for (pt_term &t : c.terms) {
-		const int64_t slab = (int64_t)t.K * t.q_k;
-		const int64_t pslab = pt_kgroups(form, t.K) * t.q_k *
-		    pt_group_bytes(form);
-		for (int x = 0; x < 3; ++x)
-			t.q_off[x] = t.q_off[x] / slab * pslab;
+			pt_terms_mixed(c.terms, form, s, oa, va, ob, vb, pl->copies);
 	}
 	L.nterm1 = pt_terms_order(c.terms, &L.nterm_a);
 	L.nterm2 = (int32_t)c.terms.size() / nset - L.nterm1;
@@ -742,6 +740,21 @@ plan_set_geometry(libpt_amd_plan *pl, int nw)
 	return true;
 }
 
+int64_t noalloc_need(const libpt_amd_plan &pl);
+
+/* does a spin case of these sizes have any triples? */
+bool
+case_same(int64_t o, int64_t v)
+{
+	return o >= 3 && v >= 3;
+}
+
+bool
+case_mixed(int64_t o1, int64_t v1, int64_t o2, int64_t v2)
+{
+	return o1 >= 2 && v1 >= 2 && o2 >= 1 && v2 >= 1;
+}
+
 /* Stages the operands and work lists of one call into pl, which comes
  * with its arena (or none) and, when pl->own_stream is false, its stream.
  * own_wsave: allocate the (fT) save areas now, so that runs allocate
@@ -766,11 +779,7 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 	if (const char *g = getenv("LIBPT_AMD_KGROUP"))
 		pl->kgrp = std::max(1, std::min(64, atoi(g)));
 	if (const char *t = getenv("LIBPT_AMD_VC_TRANSPOSED"))
-		pl->vct = atoi(t) != 0;
-	/* the static scratch of the allocation-free call holds more systems
-	 * without the second copy of the mixed ovvv block */
-	if (pl->arena)
-		pl->vct = false;
+		pl->copies = pl->copies && atoi(t) != 0;
 	if (const char *t = getenv("LIBPT_AMD_PERSISTENT"))
 		pl->persist = atoi(t) != 0;
 	pl->call = call;
@@ -790,6 +799,12 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		PFAIL((hipEventCreate(&pl->ev0) == hipSuccess &&
 		    hipEventCreate(&pl->ev1) == hipSuccess) ||
 		    (set_err("hipEventCreate failed"), false));
+	}
+	if (pl->arena && noalloc_need(*pl) > (int64_t)LIBPT_AMD_NOALLOC_SCRATCH) {
+		set_err("the call needs more than the %zu bytes of static scratch of "
+		    "the allocation-free entry point (%lld)",
+		    (size_t)LIBPT_AMD_NOALLOC_SCRATCH, (long long)noalloc_need(*pl));
+		return false;
 	}
 	PFAIL(plan_alloc(pl, (void **)&pl->d_out, 4 * sizeof(double)));
 	PFAIL(plan_alloc(pl, (void **)&pl->d_ctr, 8 * sizeof(uint32_t)));
@@ -812,31 +827,35 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		famT[0] = 4; famO[0] = 8; famV[0] = 9;
 		famT[1] = 3; famO[1] = 6; famV[1] = 7;
 	}
-	const int KC = pt_kc(form), GB = pt_group_bytes(form);
 	const int nblk = restricted ? 2 : 4;
 	const double t_prep = now_s();
 
-	/* block geometry [R slabs][K kappa][PL plane] and element offsets,
-	 * src/pt.c:460-467 (restricted) and :487-512 (unrestricted) */
+	/* block geometry [R slabs][K kappa][plane rows x cols, or the pairs
+	 * row > column] and element offsets, src/pt.c:460-467 (restricted) and
+	 * :487-512 (unrestricted) */
 	struct Geo {
-		int64_t R, K, PL, off;
+		int64_t R, K, rows, cols;
+		int tri;
+		int64_t off;
 	};
 	auto geo = [&](int fam, int blk) {
-		const int64_t PA = va * (va - 1) / 2, PB = vb * (vb - 1) / 2;
 		Geo g[4];
 		if (fam == 0) {        /* t2-like [o][o][v][v] */
-			g[0] = {oa, oa, va * va, 0};
-			g[1] = {oa, ob, va * vb, 0};
-			g[2] = {ob, ob, vb * vb, 0};
-			g[3] = {ob, oa, vb * va, 0};
+			g[0] = {oa, oa, va, va, 0, 0};
+			g[1] = {oa, ob, va, vb, 0, 0};
+			g[2] = {ob, ob, vb, vb, 0, 0};
+			g[3] = {ob, oa, vb, va, 0, 0};
 		} else {               /* ovvv [o][v][v][v], same spin packed */
-			g[0] = {oa, va, PA, 0};
-			g[1] = {oa, vb, va * vb, 0};
-			g[2] = {ob, vb, PB, 0};
-			g[3] = {ob, va, vb * va, 0};
+			g[0] = {oa, va, va, va, 1, 0};
+			g[1] = {oa, vb, va, vb, 0, 0};
+			g[2] = {ob, vb, vb, vb, 1, 0};
+			g[3] = {ob, va, vb, va, 0, 0};
 		}
-		for (int b = 1; b < 4; ++b)
-			g[b].off = g[b - 1].off + g[b - 1].R * g[b - 1].K * g[b - 1].PL;
+		for (int b = 1; b < 4; ++b) {
+			const Geo &h = g[b - 1];
+			g[b].off = h.off + h.R * h.K * (h.tri ?
+			    h.rows * (h.rows - 1) / 2 : h.rows * h.cols);
+		}
 		return g[blk];
 	};
 
@@ -877,51 +896,53 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		sT[s] = out2[0];
 		sO[s] = out2[1];
 	}
-	/* Q operands: packed copies of every amplitude and ovvv block */
-	Blocks qT[2], qV[2];
+	/* Q operands: packed copies of every amplitude and ovvv block (fam 0
+	 * and 1), and the transposed copies: every amplitude block, and the
+	 * mixed ovvv blocks as the mixed-spin case reads its VC operand
+	 * (VC[k, d, c, b] with (u, w) = (b or a, c)) */
+	Blocks qT[2] = {}, qV[2] = {}, qTt[2] = {}, qVt[2] = {};
+	/* blocks that a spin case with any triples reads */
+	const bool sa = case_same(oa, va), sb = case_same(ob, vb);
+	const bool mx = case_mixed(oa, va, ob, vb) ||
+	    case_mixed(ob, vb, oa, va);
+	const bool used[4] = {sa || mx, mx, sb || mx, mx};
+	const bool used_t[4] = {sa, mx, sb, mx};   /* transposed */
+	auto pack = [&](int s, int fam, int b, bool tr, const char **out) {
+		const Geo g = geo(fam, b);
+		const int64_t rows = tr ? g.cols : g.rows;
+		const int64_t cols = tr ? g.rows : g.cols;
+		const int api = fam == 0 ? famT[s] : famV[s];
+		void *dst;
+		if (!plan_alloc(pl, &dst, (size_t)(g.R * pt_slab_frags(form, g.K,
+		    rows, cols, g.tri)) * PT_FRAG))
+			return false;
+		const char *src = (const char *)arr[api] + esz * (size_t)g.off;
+		if (pt_launch_pack(src, dst, g.R, g.K, rows, cols, g.tri, tr, form,
+		    pl->scale[2 * s + fam], pl->stream) != 0) {
+			set_err("pack launch failed");
+			return false;
+		}
+		*out = (const char *)dst;
+		return true;
+	};
 	for (int s = 0; s < nset_; ++s) {
 		for (int fam = 0; fam < 2; ++fam) {
-			const int api = fam == 0 ? famT[s] : famV[s];
-			const double sc = pl->scale[2 * s + (fam == 0 ? 0 : 1)];
-			Blocks &dstb = fam == 0 ? qT[s] : qV[s];
+			Blocks &q = fam == 0 ? qT[s] : qV[s];
+			Blocks &qt = fam == 0 ? qTt[s] : qVt[s];
 			for (int b = 0; b < nblk; ++b) {
-				const Geo g = geo(fam, b);
-				const int64_t nkb = pt_kgroups(form, g.K);
-				void *dst;
-				PFAIL(plan_alloc(pl, &dst, (size_t)(g.R * nkb * g.PL) * GB));
-				const char *src = (const char *)arr[api] + esz * (size_t)g.off;
-				PFAIL(pt_launch_pack(src, dst, g.R, g.K, nkb, g.PL, KC, form,
-				    sc, 0, pl->stream) == 0 ||
-				    (set_err("pack launch failed"), false));
-				dstb.p[b] = (const char *)dst;
+				if (used[b])
+					PFAIL(pack(s, fam, b, false, &q.p[b]));
+				qt.p[b] = q.p[b];
+				if (used_t[b] && pl->copies && (fam == 0 || (b & 1)))
+					PFAIL(pack(s, fam, b, true, &qt.p[b]));
 			}
 			if (restricted) {
-				dstb.p[2] = dstb.p[0];
-				dstb.p[3] = dstb.p[1];
+				q.p[2] = q.p[0];
+				q.p[3] = q.p[1];
+				qt.p[2] = qt.p[0];
+				qt.p[3] = qt.p[1];
 			}
 		}
-	}
-	/* the mixed ovvv blocks as the mixed-spin case reads its VC operand
-	 * (VC[k, d, c, b] with (u, w) = (b or a, c)): packed again with the
-	 * plane transposed, so that the 32 w of a DMA row are contiguous
-	 * (abab plane [va][vb], baba [vb][va]) */
-	Blocks qVt[2];
-	for (int s = 0; s < nset_ && pl->vct; ++s) {
-		const double sc = pl->scale[2 * s + 1];
-		for (int b = 1; b < (restricted ? 2 : 4); b += 2) {
-			const Geo g = geo(1, b);
-			const int64_t nkb = pt_kgroups(form, g.K);
-			void *dst;
-			PFAIL(plan_alloc(pl, &dst, (size_t)(g.R * nkb * g.PL) * GB));
-			const char *src = (const char *)arr[famV[s]] + esz *
-			    (size_t)g.off;
-			PFAIL(pt_launch_pack(src, dst, g.R, g.K, nkb, g.PL, KC, form, sc,
-			    b == 1 ? va : vb, pl->stream) == 0 ||
-			    (set_err("pack launch failed"), false));
-			qVt[s].p[b] = (const char *)dst;
-		}
-		if (restricted)
-			qVt[s].p[3] = qVt[s].p[1];
 	}
 	PFAIL(hipStreamSynchronize(pl->stream) == hipSuccess ||
 	    (set_err("operand preparation failed"), false));
@@ -1006,7 +1027,7 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		int64_t o1 = sp == 0 ? oa : ob, v1 = sp == 0 ? va : vb;
 		int64_t o2 = sp == 0 ? ob : oa, v2 = sp == 0 ? vb : va;
 		for (int s = 0; s < nset; ++s) {
-			const int sl = 12 * s;
+			const int sl = PT_SET_BUFS * s;
 			c.L.buf[sl + 0] = opT[s].p[same];
 			c.L.buf[sl + 1] = opT[s].p[mixB];
 			c.L.buf[sl + 2] = opT[s].p[mixC];
@@ -1015,10 +1036,11 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 			c.L.buf[sl + 5] = opO[s].p[mixC];
 			c.L.buf[sl + 6] = qV[s].p[same];
 			c.L.buf[sl + 7] = qV[s].p[mixB];
-			c.L.buf[sl + 8] = pl->vct ? qVt[s].p[mixC] : qV[s].p[mixC];
+			c.L.buf[sl + 8] = qVt[s].p[mixC];
 			c.L.buf[sl + 9] = qT[s].p[same];
 			c.L.buf[sl + 10] = qT[s].p[mixB];
-			c.L.buf[sl + 11] = qT[s].p[mixC];
+			c.L.buf[sl + 11] = qTt[s].p[mixC];
+			c.L.buf[sl + 12] = qTt[s].p[same];
 			c.L.inv_scale[s] = 1.0 / (pl->scale[2 * s] * pl->scale[2 * s + 1]);
 		}
 		pt_epi &e = c.L.epi;
@@ -1035,12 +1057,12 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		c.factor = fac;
 		bool empty;
 		if (cs.kind == PT_AAA) {
-			empty = o1 < 3 || v1 < 3;
+			empty = !case_same(o1, v1);
 			if (!empty)
 				PFAIL(case_finish(pl, c, form, PT_AAA, nset, o1, v1, o1,
 				    v1));
 		} else {
-			empty = o1 < 2 || v1 < 2 || o2 < 1 || v2 < 1;
+			empty = !case_mixed(o1, v1, o2, v2);
 			if (!empty)
 				PFAIL(case_finish(pl, c, form, PT_AAB, nset, o1, v1, o2,
 				    v2));
@@ -1063,12 +1085,18 @@ plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 {
 	if (!dev_init())
 		return nullptr;
-	libpt_amd_plan *pl = new libpt_amd_plan;
-	if (!plan_init(pl, call, form, oa, va, ob, vb, arr, own_wsave)) {
+	/* without the transposed copies where they leave too little memory */
+	for (int copies = 1; copies >= 0; --copies) {
+		libpt_amd_plan *pl = new libpt_amd_plan;
+		pl->copies = copies != 0;
+		if (plan_init(pl, call, form, oa, va, ob, vb, arr, own_wsave))
+			return pl;
+		const bool again = copies && pl->no_room;
 		plan_free(pl);
-		return nullptr;
+		if (!again)
+			break;
 	}
-	return pl;
+	return nullptr;
 }
 
 } /* namespace */
@@ -1872,6 +1900,66 @@ pt_set_error(const char *msg)
 		g_err[0] = 0;
 }
 
+namespace {
+
+/* The part of an allocation-free call's scratch that decides whether the
+ * call is taken (LIBPT_AMD_NOALLOC_SCRATCH): the operand copies in the sizes
+ * of their arrays with kappa padded to whole chunks, the lists, energies
+ * and term tables, and one (fT) save area.  The packed rows' padding and
+ * the transposed copies come on top of it, out of the rest of the static
+ * array. */
+int64_t
+noalloc_need(const libpt_amd_plan &pl)
+{
+	const int64_t oa = pl.oa, va = pl.va, ob = pl.ob, vb = pl.vb;
+	const int form = pl.form, nw = pl.nw;
+	const bool ft = pl.call == LIBPT_AMD_RFT || pl.call == LIBPT_AMD_UFT;
+	const bool restricted = pl.call == LIBPT_AMD_RPT ||
+	    pl.call == LIBPT_AMD_RFT;
+	const int nset = ft ? 2 : 1;
+	const int64_t el = form == PT_FORM_FP64 ? 8 : 4;
+	auto r = [](int64_t b) { return (b + 255) / 256 * 256; };
+	int64_t n[10], need = 512;
+	(void)api_sizes(pl.call, oa, va, ob, vb, n);
+	const int64_t R[4] = {oa, oa, ob, ob}, KT[4] = {oa, ob, ob, oa};
+	const int64_t KV[4] = {va, vb, vb, va};
+	const int64_t T[4] = {va * va, va * vb, vb * vb, vb * va};
+	const int64_t V[4] = {va * (va - 1) / 2, va * vb, vb * (vb - 1) / 2,
+	    vb * va};
+	for (int s = 0; s < nset; ++s) {
+		if (form == PT_FORM_BF16X3 || form == PT_FORM_F16X3)
+			need += r(4 * n[3]) + r(4 * n[ft ? 6 : 4]);
+		for (int b = 0; b < (restricted ? 2 : 4); ++b)
+			need += r(R[b] * pt_chunks(form, KT[b]) * pt_kc(form) * T[b] *
+			    el) + r(R[b] * pt_chunks(form, KV[b]) * pt_kc(form) * V[b] *
+			    el);
+	}
+	for (int sp = 0; sp < (restricted ? 1 : 2); ++sp)
+		for (int same = 0; same < 2; ++same) {
+			const int64_t o1 = sp ? ob : oa, v1 = sp ? vb : va;
+			const int64_t o2 = sp ? oa : ob, v2 = sp ? va : vb;
+			if (!(same ? case_same(o1, v1) : case_mixed(o1, v1, o2, v2)))
+				continue;
+			Case c;
+			c.same = same;
+			c.nA = (int)((v1 + PT_TA - 1) / PT_TA);
+			c.tcw = pt_tcw(form, nset, nw);
+			c.nC = (int)(((same ? v1 : v2) + c.tcw - 1) / c.tcw);
+			int64_t nt = 0;
+			(void)tile_order(c, c.block, [&](int, int, int) { ++nt; });
+			const int64_t nijk = same ? o1 * (o1 - 1) * (o1 - 2) / 6 :
+			    o1 * (o1 - 1) / 2 * o2;
+			need += r(120 * nset * (same ? PT_TERMS_SAME :
+			    PT_TERMS_MIXED)) + r(12 * nijk) + r(12 * nt) +
+			    r(8 * nijk * nt);
+		}
+	if (ft)
+		need += pt_wsave_bytes(form, 2, nw);
+	return need;
+}
+
+} /* namespace */
+
 /*
  * The body of libpt_amd_energy_noalloc (pt_noalloc.hip): one call on
  * device-resident inputs whose every device buffer -- packed operands,
@@ -1887,23 +1975,31 @@ pt_noalloc_energy(int call, int form, size_t oa, size_t va, size_t ob,
 {
 	if (!dev_init())
 		return NAN;
-	Arena ar;
-	ar.base = (char *)scratch;
-	ar.cap = cap;
-	libpt_amd_plan pl;
-	pl.arena = &ar;
-	pl.own_stream = false;
-	pl.stream = (hipStream_t)stream;
-	double e = NAN;
-	if (plan_init(&pl, call, form, oa, va, ob, vb, dev_arrays, true)) {
-		bool ok = true;
-		for (int sc = 0; sc < pl.cases.size() && ok; ++sc)
-			ok = libpt_amd_plan_run(&pl, sc, 0, pl.cases[sc].n_ijk) == 0;
-		if (ok)
-			e = libpt_amd_plan_energy(&pl);
+	/* without the transposed copies where they do not fit */
+	for (int copies = 1; copies >= 0; --copies) {
+		Arena ar;
+		ar.base = (char *)scratch;
+		ar.cap = cap;
+		libpt_amd_plan pl;
+		pl.arena = &ar;
+		pl.own_stream = false;
+		pl.stream = (hipStream_t)stream;
+		pl.copies = copies != 0;
+		double e = NAN;
+		if (plan_init(&pl, call, form, oa, va, ob, vb, dev_arrays, true)) {
+			bool ok = true;
+			for (int sc = 0; sc < pl.cases.size() && ok; ++sc)
+				ok = libpt_amd_plan_run(&pl, sc, 0, pl.cases[sc].n_ijk) ==
+				    0;
+			if (ok)
+				e = libpt_amd_plan_energy(&pl);
+		}
+		const bool again = copies && pl.no_room;
+		plan_release(&pl);
+		if (!again)
+			return e;
 	}
-	plan_release(&pl);
-	return e;
+	return NAN;
 }
 
 namespace {

@@ -1,0 +1,1072 @@
+/*
+ * CDNA4 (gfx950) tile kernel of the perturbative-triples engine, one
+ * translation unit per arithmetic form (pt_tiles_*.hip).
+ *
+ * k_tiles: one workgroup = one ijk item x one (A, B, C) tile of 32 a x 32 b
+ * x TC c.  W of the tile stays in MFMA accumulators and never goes to
+ * memory:
+ *
+ *   phase 1 -- accumulator layout [a][b]@c (16 x 16 blocks, one c each);
+ *       wave w of NW owns the whole a, b range at c = C0 + NW x + w:
+ *       terms whose single index is a  (A = S rows a,  B = Q[.][b][c])
+ *       terms whose single index is b  (A = Q[.][a][c], B = S rows b)
+ *   transpose through LDS to layout [a][c]@b; wave w owns b = B0 + NW y + w
+ *   phase 2 -- terms whose single index is c
+ *       (A = Q[.][a][b], B = S rows c)
+ *   epilogue -- for every (a, b, c) of the reference's triangle:
+ *       disconnected term Z, denominator Dn, energy W (W - Z) / Dn
+ *       ((fT): (W_L - Z_L) W_R / Dn), compensated FP64 sum per lane,
+ *       one deterministic reduction per workgroup into partial[item];
+ *       the Z and Dn operands that depend on b are staged in LDS once
+ *       per item, those of a and c alone held in registers per lane.
+ *
+ * Operands go from the packed copies straight into the registers of the
+ * wave that multiplies them.  A packed Q slab is a sequence of fragments of
+ * 1 KB, 16 rows (u) x PT_KC kappa in the lane order of the MFMA operand, so
+ * a fragment is one coalesced 16-byte load per lane, and since each wave
+ * owns its own w (c in phase 1, b in phase 2) and the full range of the
+ * other two indices, every Q fragment of a tile is loaded by exactly one
+ * wave and used by both 16-row blocks of S.  There is nothing to share
+ * through LDS, hence no barrier in the step loop: the two waves of a SIMD
+ * drift apart and fill each other's waits, and each fragment register is
+ * reloaded for the next step right after its MFMAs, one whole step ahead.
+ * Against the kernel that staged the operands in LDS (two slots, a barrier
+ * per step, one wave per 16 a x 16 b x TC c): MFMA pipe 84 % busy instead of
+ * 67 % at rpt v=477 in FP64, where the card's clock then falls from 2.2 to
+ * 1.95 GHz (a share of the triples: 289 -> 270 ms); rpt o=20 v=120 331 ->
+ * 239 ms, FP32 upt 24/200/20/204 292 -> 196 ms, split-BF16 rpt v=477 253 ->
+ * 233 ms, a batch of 8 systems of v 40 to 160 198 -> 120 ms.  Bound by the
+ * MFMA pipe and power in FP64 and FP32, by L2 and HBM bandwidth in the split
+ * forms.
+ *
+ * Forms: FP64 (v_mfma_f64_16x16x4_f64), FP32 (v_mfma_f32_16x16x4_f32),
+ * split BF16 / FP16 (hi+lo pairs, hi*hi + lo*hi + hi*lo packed into the
+ * k slots of v_mfma_f32_16x16x32_{bf16,f16}, FP32 accumulation, FP64
+ * epilogue).
+ *
+ * MFMA lane layouts (checked on gfx950): A[m][k] lane m + 16*(k/KL),
+ * B[k][n] lane n + 16*(k/KL) (KL = 1 for x4, 8 consecutive k for x32);
+ * D[m][n] lane n + 16*(m/4) reg m%4 for f32 results, but
+ * lane n + 16*(m%4) reg m/4 for v_mfma_f64_16x16x4_f64.
+ */
+#ifndef LIBPT_AMD_PT_TILES_H
+#define LIBPT_AMD_PT_TILES_H
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "pt_engine.h"
+
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+namespace {
+
+template <int F> struct Form;
+
+template <> struct Form<PT_FORM_FP64> {
+	typedef double G;   /* S element in HBM */
+	typedef double AE;  /* accumulator element */
+	typedef v4d ACC;
+	typedef double ER;  /* epilogue real */
+	static constexpr int KC = 8;    /* kappa per fragment */
+	static constexpr bool ROW_F64 = true, SPLIT = false;
+};
+
+template <> struct Form<PT_FORM_FP32> {
+	typedef float G;
+	typedef float AE;
+	typedef v4f ACC;
+	typedef float ER;
+	static constexpr int KC = 16;
+	static constexpr bool ROW_F64 = false, SPLIT = false;
+};
+
+template <> struct Form<PT_FORM_BF16X3> {
+	typedef uint32_t G;  /* hi in bits 0-15, lo in bits 16-31 */
+	typedef float AE;
+	typedef v4f ACC;
+	typedef double ER;
+	static constexpr int KC = 16;
+	static constexpr bool ROW_F64 = false, SPLIT = true;
+};
+
+template <> struct Form<PT_FORM_F16X3> : Form<PT_FORM_BF16X3> {};
+
+/* ---------------------------------------------------------------- MFMA */
+
+__device__ __forceinline__ v4d
+mma(double a, double b, v4d c)
+{
+	return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ v4f
+mma(float a, float b, v4f c)
+{
+	return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+/* one K=32 bf16 / f16 MFMA (v_mfma_f32_16x16x32_{bf16,f16}, full rate on
+ * gfx950) on operands of four 32-bit words (eight 16-bit values) per lane.
+ * A and B fill their eight slots of each lane group with the same
+ * (kappa, hi/lo) pattern, so each slot contributes one product of the
+ * same kappa whatever the instruction's k order within the lane group. */
+template <int F>
+__device__ __forceinline__ v4f
+mma32(v4u a, v4u b, v4f c)
+{
+	if constexpr (F == PT_FORM_BF16X3)
+		return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+		    __builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0,
+		    0, 0);
+	else
+		return __builtin_amdgcn_mfma_f32_16x16x32_f16(
+		    __builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0,
+		    0);
+}
+
+/* ---------------------------------------------------------- S operand */
+
+/* the S fragment of a step as its MFMAs take it.  FP64, FP32: the loaded
+ * words.  Split: Q fragments hold, per lane, hi k0 k1, hi k2 k3, lo k0 k1,
+ * lo k2 k3 and go to the MFMA as they are; S comes as (hi, hi) for
+ * hi*hi + lo*hi and (lo, 0) for hi*lo. */
+template <int F>
+struct SFrag {
+	v4u w;
+	__device__ __forceinline__ void set(v4u e, uint32_t sgn)
+	{
+		if constexpr (F == PT_FORM_FP64) {
+			w = v4u{e[0], e[1] ^ sgn, e[2], e[3] ^ sgn};
+		} else if constexpr (F == PT_FORM_FP32) {
+			w = v4u{e[0] ^ sgn, e[1] ^ sgn, e[2] ^ sgn, e[3] ^ sgn};
+		} else {
+			/* API words hi | lo << 16 of kappa 0 .. 3 -> hi 01, hi 23,
+			 * lo 01, lo 23 */
+			const uint32_t s2 = sgn | (sgn >> 16);
+			w = v4u{__builtin_amdgcn_perm(e[1], e[0], 0x05040100u) ^ s2,
+			    __builtin_amdgcn_perm(e[3], e[2], 0x05040100u) ^ s2,
+			    __builtin_amdgcn_perm(e[1], e[0], 0x07060302u) ^ s2,
+			    __builtin_amdgcn_perm(e[3], e[2], 0x07060302u) ^ s2};
+		}
+	}
+};
+
+/* an accumulator block as one register tuple: without it the compiler splits
+ * the blocks at control flow into their elements (because they start as
+ * constants or are put together from LDS reads) and copies them there */
+template <class ACC>
+__device__ __forceinline__ void
+pin(ACC &x)
+{
+	__asm__ volatile("" : "+v"(x));
+}
+
+/* NMF MFMAs add one Q fragment times one S fragment; part p of them.  QA:
+ * Q is the A operand (rows of D), else B. */
+template <int F> constexpr int NMF = F == PT_FORM_FP32 ? 4 : 2;
+
+template <int F, bool QA>
+__device__ __forceinline__ typename Form<F>::ACC
+mma_part(int p, v4u q, const SFrag<F> &s, typename Form<F>::ACC c)
+{
+	if constexpr (F == PT_FORM_FP64) {
+		const v2d x = __builtin_bit_cast(v2d, q), y = __builtin_bit_cast(v2d,
+		    s.w);
+		return QA ? mma(x[p], y[p], c) : mma(y[p], x[p], c);
+	} else if constexpr (F == PT_FORM_FP32) {
+		const v4f x = __builtin_bit_cast(v4f, q), y = __builtin_bit_cast(v4f,
+		    s.w);
+		return QA ? mma(x[p], y[p], c) : mma(y[p], x[p], c);
+	} else {
+		const v4u y = p ? v4u{s.w[2], s.w[3], 0u, 0u} :
+		    v4u{s.w[0], s.w[1], s.w[0], s.w[1]};
+		return QA ? mma32<F>(q, y, c) : mma32<F>(y, q, c);
+	}
+}
+
+/* ---------------------------------------------------------- epilogue */
+
+__device__ __forceinline__ void
+kahan(double &s, double &cmp, double x)
+{
+	double y = x - cmp;
+	double t = s + y;
+	cmp = (t - s) - y;
+	s = t;
+}
+
+/*
+ * Energy terms of one lane's NB elements (a, b0 + BS y, c), y = 0 .. NB-1,
+ * in y order, added to (esum, ecmp): the disconnected term Z, the
+ * denominator Dn = d_ia + d_jb + d_kc and W (W - Z) / Dn, or for two W sets
+ * (W_L - Z) W_R / Dn (src/pt.c:700,927).  The loads that depend on a, c or
+ * (a, c) only are made once for the NB elements; b is clamped into the
+ * arrays, so every element's loads are made whether or not the triangle
+ * keeps it, and only the sum is masked.  W values: ew[64 y] (one set; the
+ * right set with two) and ew[64 (y + NB)] (the left set).  The workgroup
+ * has staged in LDS the (b, c) values of i_oovv and t2, sbc[(32 n + BS y)
+ * TC] (sbc points at this lane's b0 and c) for n = G jk, Z jk, G ik, Z ik
+ * (mixed spin: GB, ZB; same spin also G ji, Z ji), the values that depend
+ * on b only, sbv[32 n + BS y] (sbv points at b0) for n = u i, f i, u j,
+ * f j, (same spin: u k, f k,) d1 j, and for the mixed spin case the (b, a)
+ * values of the same-spin blocks for ji, sba[(32 n + BS y) 32] for n = GA,
+ * ZA (sba points at b0 and this lane's a).
+ */
+template <int F, int KIND, int NSET, int NB, int BS, int TC>
+__device__ __forceinline__ void
+epi_block(const pt_launch &p, int i, int j, int k, int a, int c, int b0,
+    const typename Form<F>::AE *ew,
+    const typename Form<F>::ER *sbc, const typename Form<F>::ER *sba,
+    const typename Form<F>::ER *sbv, double &esum, double &ecmp)
+{
+	typedef typename Form<F>::ER ER;
+	const ER s0 = (ER)p.inv_scale[0], s1 = (ER)p.inv_scale[1];
+	const ER *d1 = (const ER *)p.epi.d1;
+	/* this element's term from its Z and Dn */
+	auto term = [&](int y, ER z, ER dn) {
+		if constexpr (NSET == 1) {
+			ER w = (ER)ew[64 * y];
+			if (Form<F>::SPLIT)
+				w *= s0;
+			return w * (w - z) / dn;
+		} else {
+			ER wl = (ER)ew[64 * (y + NB)], wr = (ER)ew[64 * y];
+			if (Form<F>::SPLIT) {
+				wl *= s0;
+				wr *= s1;
+			}
+			return (wl - z) * wr / dn;
+		}
+	};
+	if constexpr (KIND == PT_AAA) {
+		/* src/pt.c:162-175, for (u, G) = (t1 or l1, i_oovv) and
+		 * (f, Z) = (f_ov or f2_ov, t2 or l2) */
+		const int64_t o = p.oa, v = p.va, vv = v * v;
+		const ER *u = (const ER *)p.epi.u1, *f = (const ER *)p.epi.f1;
+		const ER *G = (const ER *)p.epi.GA, *Z = (const ER *)p.epi.ZA;
+		const int64_t jk = ((int64_t)j * o + k) * vv;
+		const int64_t ik = ((int64_t)i * o + k) * vv;
+		const int64_t ji = ((int64_t)j * o + i) * vv;
+		const ER uia = u[i * v + a], uja = u[j * v + a], uka = u[k * v + a];
+		const ER fia = f[i * v + a], fja = f[j * v + a], fka = f[k * v + a];
+		const ER uic = u[i * v + c], ujc = u[j * v + c], ukc = u[k * v + c];
+		const ER fic = f[i * v + c], fjc = f[j * v + c], fkc = f[k * v + c];
+		const int64_t ac = (int64_t)a * v + c;
+		const ER gjkac = G[jk + ac], gikac = G[ik + ac], gjiac = G[ji + ac];
+		const ER zjkac = Z[jk + ac], zikac = Z[ik + ac], zjiac = Z[ji + ac];
+		const ER dia = d1[i * v + a], dkc = d1[k * v + c];
+#pragma unroll 1
+		for (int y = 0; y < NB; ++y) {
+			const int bb = BS * y, b = b0 + bb;
+			const int bq = b < p.na ? b : p.na - 1;
+			const int64_t ba = (int64_t)bq * v + a;
+			const ER uib = sbv[bb], fib = sbv[32 + bb];
+			const ER ujb = sbv[64 + bb], fjb = sbv[96 + bb];
+			const ER ukb = sbv[128 + bb], fkb = sbv[160 + bb];
+			const ER djb = sbv[192 + bb];
+			const ER gjkbc = sbc[bb * TC], zjkbc = sbc[(32 + bb) * TC];
+			const ER gikbc = sbc[(64 + bb) * TC];
+			const ER zikbc = sbc[(96 + bb) * TC];
+			const ER gjibc = sbc[(128 + bb) * TC];
+			const ER zjibc = sbc[(160 + bb) * TC];
+			const ER zu = uia * gjkbc - uja * gikbc -
+			    uka * gjibc - uib * gjkac + ujb * gikac +
+			    ukb * gjiac - uic * G[jk + ba] + ujc * G[ik + ba] +
+			    ukc * G[ji + ba];
+			const ER zf = fia * zjkbc - fja * zikbc -
+			    fka * zjibc - fib * zjkac + fjb * zikac +
+			    fkb * zjiac - fic * Z[jk + ba] + fjc * Z[ik + ba] +
+			    fkc * Z[ji + ba];
+			const ER t = term(y, zu + zf, dia + djb + dkc);
+			if (a > b && b > c)
+				kahan(esum, ecmp, (double)t);
+		}
+	} else {
+		/* src/pt.c:177-185 and :433-442 */
+		const int64_t va = p.va, ob = p.ob, vb = p.vb;
+		const ER *u1 = (const ER *)p.epi.u1, *u2 = (const ER *)p.epi.u2;
+		const ER *f1 = (const ER *)p.epi.f1, *f2 = (const ER *)p.epi.f2;
+		const ER *GB = (const ER *)p.epi.GB, *ZB = (const ER *)p.epi.ZB;
+		const ER *d2 = (const ER *)p.epi.d2;
+		const int64_t jk = ((int64_t)j * ob + k) * va;
+		const int64_t ik = ((int64_t)i * ob + k) * va;
+		const ER uia = u1[i * va + a], fia = f1[i * va + a];
+		const ER uja = u1[j * va + a], fja = f1[j * va + a];
+		const ER u2c = u2[k * vb + c], f2c = f2[k * vb + c];
+		const int64_t jkac = (jk + a) * vb + c, ikac = (ik + a) * vb + c;
+		const ER gjkac = GB[jkac], zjkac = ZB[jkac];
+		const ER gikac = GB[ikac], zikac = ZB[ikac];
+		const ER dia = d1[i * va + a], dkc = d2[k * vb + c];
+#pragma unroll 1
+		for (int y = 0; y < NB; ++y) {
+			const int bb = BS * y, b = b0 + bb;
+			const ER uib = sbv[bb], fib = sbv[32 + bb];
+			const ER ujb = sbv[64 + bb], fjb = sbv[96 + bb];
+			const ER djb = sbv[128 + bb];
+			const ER gjkbc = sbc[bb * TC], zjkbc = sbc[(32 + bb) * TC];
+			const ER gikbc = sbc[(64 + bb) * TC];
+			const ER zikbc = sbc[(96 + bb) * TC];
+			const ER gjiba = sba[bb * 32], zjiba = sba[(32 + bb) * 32];
+			const ER z = (uia * gjkbc + fia * zjkbc)
+			    - (uib * gjkac + fib * zjkac)
+			    - (uja * gikbc + fja * zikbc)
+			    + (ujb * gikac + fjb * zikac)
+			    + (u2c * gjiba + f2c * zjiba);
+			const ER t = term(y, z, dia + djb + dkc);
+			if (a > b)
+				kahan(esum, ecmp, (double)t);
+		}
+	}
+}
+
+/* values the whole wave shares: readfirstlane tells the compiler so, which
+ * keeps them (and everything derived from them) in scalar registers */
+__device__ __forceinline__ int
+uni(int x)
+{
+	return __builtin_amdgcn_readfirstlane(x);
+}
+
+__device__ __forceinline__ int64_t
+uni64(int64_t x)
+{
+	const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+	const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+	return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+/* buffer descriptors: loads at offsets at or beyond the descriptor's byte
+ * count return zero, which handles tile edges, invalid pairs and the kappa
+ * tail without branches */
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t
+brsrc(const void *base, int64_t bytes)
+{
+	const int nrec = bytes <= 0 ? 0 : bytes > 0x7fffffff ? 0x7fffffff :
+	    (int)bytes;
+	return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, nrec,
+	    0x00020000);
+}
+
+#define PT_OOR 0x80000000u  /* an offset every descriptor rejects */
+
+/* buffer store / load of one accumulator value at lane offset vofs plus a
+ * constant offset sofs: the constant goes to a scalar register, so a run of
+ * them costs no vector registers for addresses */
+template <class AE>
+__device__ __forceinline__ void
+bstore_ae(__amdgpu_buffer_rsrc_t r, uint32_t vofs, int sofs, AE v)
+{
+	if constexpr (sizeof(AE) == 8)
+		__builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r,
+		    (int)vofs, sofs, 0);
+	else
+		__builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t,
+		    v), r, (int)vofs, sofs, 0);
+}
+
+template <class AE>
+__device__ __forceinline__ AE
+bload_ae(__amdgpu_buffer_rsrc_t r, uint32_t vofs, int sofs)
+{
+	if constexpr (sizeof(AE) == 8)
+		return __builtin_bit_cast(AE,
+		    __builtin_amdgcn_raw_buffer_load_b64(r, (int)vofs, sofs, 0));
+	else
+		return __builtin_bit_cast(AE,
+		    __builtin_amdgcn_raw_buffer_load_b32(r, (int)vofs, sofs, 0));
+}
+
+
+
+/* ------------------------------------------------------ terms of an item */
+
+/* one term of the item's tile, in LDS, made once per item by one thread
+ * each; every field is read as a wave-uniform value */
+struct TermP {
+	uint64_t q[2];    /* chunk 0 of the two u blocks at the tile's first w */
+	uint64_t s;       /* S element (row 0, kappa 0) */
+	uint32_t dq[2];   /* bytes from one chunk to the next */
+	uint32_t xa, xb;  /* bytes from w to w + 1 and, over 16 w, w + 16 */
+	uint32_t sst;     /* bytes between S rows */
+	uint32_t sbytes;  /* bytes of the S rows from s */
+	int32_t nch;      /* kappa chunks */
+	uint32_t sgn;     /* sign bit to flip in S */
+	int32_t tr;       /* Q rows are w (the plane is packed transposed) */
+	int32_t pad_;
+};
+
+/* the term's addresses for the tile (A0, B0, C0).  A packed slab is
+ * [row block of 16][chunk][column][1 KB fragment]: rows u and columns w, or
+ * (tr) rows w and columns u; tri: columns 0 .. 16 (block + 1) - 1 only. */
+template <int F>
+__device__ __forceinline__ void
+make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
+    int B0, int C0, TermP &o)
+{
+	constexpr int ES = (int)sizeof(typename Form<F>::G);
+	const int na = p.na, nc = p.nc;
+	const int u0 = t.role == PT_ROLE_A ? B0 : A0;
+	const int w0 = t.role == PT_ROLE_C ? B0 : C0;
+	const char *qb = (const char *)p.buf[t.q_buf] + t.q_off[0] * i +
+	    t.q_off[1] * j + t.q_off[2] * k;
+	for (int e = 0; e < 2; ++e) {
+		const int64_t ub = u0 / 16 + e;
+		int64_t off, cols;
+		if (t.tri) {
+			off = t.nch * 8 * ub * (ub + 1) + w0;
+			cols = 16 * (ub + 1);
+		} else if (t.tr) {
+			off = (int64_t)(w0 / 16) * t.nch * t.cols + 16 * ub;
+			cols = t.cols;
+		} else {
+			off = ub * t.nch * t.cols + w0;
+			cols = t.cols;
+		}
+		o.q[e] = (uint64_t)qb + 1024 * (uint64_t)off;
+		o.dq[e] = (uint32_t)(1024 * cols);
+	}
+	o.xa = t.tr ? 16 : 1024;
+	o.xb = t.tr ? (uint32_t)((int64_t)t.nch * t.cols * 1024) : 16 * 1024;
+	o.s = (uint64_t)p.buf[t.s_buf] + ES * (uint64_t)(t.s_off[0] * i +
+	    t.s_off[1] * j + t.s_off[2] * k);
+	o.sst = (uint32_t)(t.s_st * ES);
+	const int64_t sb = (t.role == PT_ROLE_C ? nc : na) * t.s_st * ES;
+	o.sbytes = (uint32_t)(sb > 0x7fffffff ? 0x7fffffff : sb);
+	o.nch = t.nch;
+	o.sgn = t.sign < 0 ? 0x80000000u : 0u;
+	o.tr = t.tr;
+	o.pad_ = 0;
+}
+
+/*
+ * The terms [t0, t1) of one role, over all their kappa chunks, added to the
+ * accumulators.  The wave owns w = w0 + NW x + wave, x = 0 .. NX-1, of the
+ * tile; per chunk it holds the fragments (x, u block e) and the NSB S
+ * blocks; B::id(x, e, s) is the accumulator block of a fragment and an S
+ * block.  mask: the blocks that hold an element of the triangle inside the
+ * extents; they are computed in groups (half of x, e, s), and a group
+ * without any is skipped, so that the tiles cut by the diagonal or by the
+ * end of an index pay for 16 x 16 blocks and not for whole tiles.  The
+ * fragments that serve a block of the mask are a range of x for each e;
+ * those outside it may not exist, so the nearest one of the range is read
+ * in their place (their blocks are never used).
+ *
+ * Step n = (term, chunk).  Each fragment's registers are loaded for step
+ * n + 1 right after its MFMAs of step n, so that a step's loads are always
+ * in flight per wave and every load has one step to arrive; the loads after
+ * the last step are all out of range and return zero.
+ *
+ * One loop serves full and cut tiles: with loop variants chosen by control
+ * flow the accumulators, more than half of the registers, meet at joins
+ * after every variant, and the register allocator then spills dozens of
+ * blocks there and inside the loops.
+ */
+template <int F, int NW, int NX, int NSB, int ROLE, class B, int NACC>
+__device__ __forceinline__ void
+run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
+    int u0, int uext, int s0, int sext, int wave, int ln, int lg,
+    uint32_t mask)
+{
+	static_assert(Form<F>::KC * sizeof(typename Form<F>::G) == 64,
+	    "a chunk of S is 64 bytes per row");
+	constexpr bool QA = ROLE != PT_ROLE_A;
+	constexpr int XB = 16 / NW;      /* x per 16 w */
+	if (t0 >= t1)
+		return;
+	uint64_t q0, q1, sp;
+	uint32_t dq0, dq1, xa, xb, sgn;
+	int sb;
+	int left;
+	bool more = true;
+	uint32_t vo[2], so[NSB];
+	/* the x of each e that may be read (xhi < 0: none), the groups */
+	constexpr int NH = NX / 2;
+	int xlo[2], xhi[2];
+	uint32_t grp = 0;
+#pragma unroll
+	for (int e = 0; e < 2; ++e) {
+		xlo[e] = NX - 1;
+		xhi[e] = -1;
+#pragma unroll
+		for (int x = 0; x < NX; ++x)
+#pragma unroll
+			for (int s = 0; s < NSB; ++s)
+				if (mask >> B::id(x, e, s) & 1) {
+					xlo[e] = x < xlo[e] ? x : xlo[e];
+					xhi[e] = x;
+					grp |= 1u << ((x / NH * 2 + e) * NSB + s);
+				}
+		xlo[e] = uni(xlo[e]);
+		xhi[e] = uni(xhi[e]);
+	}
+	grp = (uint32_t)uni((int)grp);
+	/* scalars and lane offsets of term t */
+	auto term = [&](int t) {
+		const TermP &T = tp[t];
+		q0 = (uint64_t)uni64((int64_t)T.q[0]);
+		q1 = (uint64_t)uni64((int64_t)T.q[1]);
+		sp = (uint64_t)uni64((int64_t)T.s);
+		dq0 = (uint32_t)uni((int)T.dq[0]);
+		dq1 = (uint32_t)uni((int)T.dq[1]);
+		xa = (uint32_t)uni((int)T.xa);
+		xb = (uint32_t)uni((int)T.xb);
+		sb = uni((int)T.sbytes);
+		sgn = (uint32_t)uni((int)T.sgn);
+		left = uni(T.nch);
+		const uint32_t sst = (uint32_t)uni((int)T.sst);
+		const bool tr = uni(T.tr) != 0;
+		q0 += (uint64_t)xa * (uint32_t)wave;
+		q1 += (uint64_t)xa * (uint32_t)wave;
+#pragma unroll
+		for (int e = 0; e < 2; ++e)
+			vo[e] = xhi[e] < 0 ? PT_OOR : !tr ?
+			    (uint32_t)(16 * (16 * lg + ln)) :
+			    u0 + 16 * e + ln < uext ?
+			    (uint32_t)(1024 * ln + 256 * lg) : PT_OOR;
+#pragma unroll
+		for (int e = 0; e < NSB; ++e)
+			so[e] = s0 + 16 * e + ln < sext ?
+			    (uint32_t)(s0 + 16 * e + ln) * sst + 16u * lg : PT_OOR;
+	};
+	/* lanes without data take an offset that every descriptor rejects; the
+	 * scalar offset is never relied on for a range check */
+	auto load_q = [&](int x, int e) {
+		x = x < xlo[e] ? xlo[e] : x > xhi[e] ? xhi[e] : x;
+		const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+		    (void *)(e ? q1 : q0), (short)0, 0x7fffffff, 0x00020000);
+		return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r,
+		    (int)vo[e], (int)((uint32_t)(x % XB) * NW * xa +
+		    (uint32_t)(x / XB) * xb), 0));
+	};
+	auto load_s = [&](int e) {
+		const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+		    (void *)sp, (short)0, sb, 0x00020000);
+		return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r,
+		    (int)so[e], 0, 0));
+	};
+
+	term(t0);
+	int t = t0;
+	v4u q[2 * NX], sr[NSB];
+#pragma unroll
+	for (int e = 0; e < NSB; ++e)
+		sr[e] = load_s(e);
+#pragma unroll
+	for (int x = 0; x < NX; ++x)
+#pragma unroll
+		for (int e = 0; e < 2; ++e)
+			q[2 * x + e] = load_q(x, e);
+	do {
+		SFrag<F> s[NSB];
+#pragma unroll
+		for (int e = 0; e < NSB; ++e)
+			s[e].set(sr[e], sgn);
+		/* on to the next step */
+		if (--left > 0) {
+			q0 += dq0;
+			q1 += dq1;
+			sp += 64;       /* KC elements of S */
+			sb = sb - 64 > 0 ? sb - 64 : 0;
+		} else if (++t < t1) {
+			term(t);
+		} else {
+			more = false;
+			vo[0] = vo[1] = PT_OOR;
+#pragma unroll
+			for (int e = 0; e < NSB; ++e)
+				so[e] = PT_OOR;
+		}
+#pragma unroll
+		for (int e = 0; e < NSB; ++e)
+			sr[e] = load_s(e);
+#pragma unroll
+		for (int h = 0; h < 2; ++h)
+#pragma unroll
+		for (int e = 0; e < 2; ++e) {
+#pragma unroll
+			for (int b = 0; b < NSB; ++b)
+				if (grp >> ((h * 2 + e) * NSB + b) & 1) {
+#pragma unroll
+					for (int m = 0; m < NMF<F>; ++m)
+#pragma unroll
+					for (int x = h * NH; x < (h + 1) * NH; ++x) {
+						const int a = B::id(x, e, b);
+						acc[a] = mma_part<F, QA>(m, q[2 * x + e], s[b],
+						    acc[a]);
+					}
+				}
+#pragma unroll
+			for (int x = h * NH; x < (h + 1) * NH; ++x)
+				q[2 * x + e] = load_q(x, e);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	} while (more);
+}
+
+/* -------------------------------------------------------------- kernel */
+
+/*
+ * Workgroup geometry, per wave count NW (pt_tcw, pt_cw in pt_engine.h give
+ * the same numbers to the host).  Tile 32 a x 32 b x TC c; CW = TC / NW c
+ * per wave in phase 1, BW = 32 / NW b per wave in phase 2, NACC 16 x 16
+ * blocks per wave in either.
+ *   NW = 4: TC = 32 for FP32 and the split forms (32 FP32 blocks of 4
+ *           registers), 16 for FP64 (16 blocks of 8 registers): 128
+ *           accumulator registers, two workgroups per CU (two waves per
+ *           SIMD).
+ *   NW = 8: TC = 32, one workgroup per CU.
+ */
+template <int F, int NSET, int NW>
+struct Geo {
+	static constexpr int TC = NW == 8 || F != PT_FORM_FP64 ? 32 : 16;
+	static constexpr int CW = TC / NW, BW = 32 / NW, NCB = TC / 16;
+	static constexpr int NACC = 4 * CW;
+	static constexpr int THREADS = 64 * NW;
+	static constexpr int WG_PER_CU = NW == 8 ? 1 : 2;
+	/* accumulator block of phase 1 (c of the wave, a block, b block) and
+	 * of phase 2 (b of the wave, a block, c block).  In either, bit 1 is
+	 * the a block, so the transpose of an a block stays in its blocks. */
+	static constexpr int blk1(int x, int ab, int bb)
+	{
+		return (2 * x + ab) * 2 + bb;
+	}
+	static constexpr int blk2(int y, int ab, int cb)
+	{
+		return NCB == 2 ? (2 * y + ab) * 2 + cb :
+		    (2 * (y >> 1) + ab) * 2 + (y & 1);
+	}
+};
+
+/* accumulator block of (x, u block, S block) for each role */
+template <class GM> struct RoleA {
+	static constexpr int id(int x, int e, int s) { return GM::blk1(x, s, e); }
+};
+
+template <class GM> struct RoleB {
+	static constexpr int id(int x, int e, int s) { return GM::blk1(x, e, s); }
+};
+
+template <class GM> struct RoleC {
+	static constexpr int id(int y, int e, int s) { return GM::blk2(y, e, s); }
+};
+
+/*
+ * One work item (ijk, tile) of a spin case: everything between reading the
+ * item and writing its energy to partial[it].  KIND is the spin case,
+ * PT_AAA or PT_AAB.  With two W sets the sets are formed one after the
+ * other; wsv is the item's save area for W of set 0 (4 NACC values per lane
+ * per wave).
+ */
+template <int F, int KIND, int NSET, int NW>
+__device__ __forceinline__ void
+tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
+{
+	typedef Form<F> FM;
+	typedef Geo<F, NSET, NW> GM;
+	typedef typename FM::AE AE;
+	typedef typename FM::ACC ACC;
+	typedef typename FM::ER ER;
+	constexpr int TC = GM::TC, CW = GM::CW, BW = GM::BW, NCB = GM::NCB;
+	constexpr int NACC = GM::NACC, NT = GM::THREADS;
+	constexpr bool same = KIND == PT_AAA;
+
+	/* LDS: the transpose's buffers (two of TRC (a block, register) columns
+	 * each), then the epilogue's W columns and staged operands */
+	constexpr int TRW = TC + 1, TRC = 2;
+	constexpr int TRB = TRC * 4 * 32 * TRW;      /* values per buffer */
+	constexpr int NPB = same ? 6 : 4;            /* (b, c) blocks */
+	constexpr int NBC = NPB * 32 * TC, NBV = (NPB + 1) * 32;
+	constexpr int NBA = same ? 0 : 2 * 32 * 32;
+	constexpr int EBYTES = NW * NSET * BW * 64 * (int)sizeof(AE);
+	constexpr int SB1 = 2 * TRB * (int)sizeof(AE);
+	constexpr int SB2 = EBYTES + (NBC + NBV + NBA) * (int)sizeof(ER);
+	constexpr int SMEM = SB1 > SB2 ? SB1 : SB2;
+	constexpr int NTERM = NSET * (same ? PT_TERMS_SAME : PT_TERMS_MIXED);
+	static_assert((SMEM + NTERM * (int)sizeof(TermP) + 8 * NW + 64) *
+	    GM::WG_PER_CU <= 160 * 1024, "LDS of the workgroups of a CU");
+	static_assert(NBC % NT == 0 && NBV <= NT && NBA % NT == 0 &&
+	    NTERM <= NT, "staging by whole passes of the workgroup");
+	__shared__ __attribute__((aligned(16))) char smem[SMEM];
+	__shared__ double red[NW];
+	__shared__ TermP tp[NTERM];
+
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int wave = uni(tid >> 6);
+	const int ln = lane & 15, lg = lane >> 4;
+
+	const int64_t ijk_id = it / p.n_tiles;
+	const int tile = (int)(it - ijk_id * p.n_tiles);
+	const int i = p.ijk[3 * ijk_id], j = p.ijk[3 * ijk_id + 1];
+	const int k = p.ijk[3 * ijk_id + 2];
+	const int A0 = p.tiles[3 * tile] * 32, B0 = p.tiles[3 * tile + 1] * 32;
+	const int C0 = p.tiles[3 * tile + 2] * TC;
+	const int na = p.na, nc = p.nc;
+
+	if (tid < NTERM)
+		make_term<F>(p, p.terms[tid], i, j, k, A0, B0, C0, tp[tid]);
+
+	/* accumulator blocks that hold an element of the triangle, a bit each:
+	 * a > b, and b > c for the same-spin case */
+	uint32_t m1 = 0, m2 = 0;
+#pragma unroll
+	for (int ab = 0; ab < 2; ++ab) {
+		const int a0 = A0 + 16 * ab, a1 = (a0 + 16 < na ? a0 + 16 : na) - 1;
+#pragma unroll
+		for (int x = 0; x < CW; ++x)
+#pragma unroll
+			for (int bb = 0; bb < 2; ++bb) {
+				const int b0 = B0 + 16 * bb, c = C0 + NW * x + wave;
+				const int b1 = (b0 + 16 < na ? b0 + 16 : na) - 1;
+				if (a0 < na && b0 < na && c < nc && a1 > b0 &&
+				    (!same || b1 > c))
+					m1 |= 1u << GM::blk1(x, ab, bb);
+			}
+#pragma unroll
+		for (int y = 0; y < BW; ++y)
+#pragma unroll
+			for (int cb = 0; cb < NCB; ++cb) {
+				const int b = B0 + NW * y + wave, c0 = C0 + 16 * cb;
+				if (a0 < na && b < na && c0 < nc && a1 > b &&
+				    (!same || b > c0))
+					m2 |= 1u << GM::blk2(y, ab, cb);
+			}
+	}
+	m1 = (uint32_t)uni((int)m1);
+	m2 = (uint32_t)uni((int)m2);
+	ACC acc[NACC];
+#pragma unroll
+	for (int x = 0; x < NACC; ++x)
+		acc[x] = ACC{0, 0, 0, 0};
+#pragma unroll
+	for (int x = 0; x < NACC; ++x)
+		pin(acc[x]);
+	/* save area of W set 0: value (r, x) of (wave, lane) at element
+	 * ((r NACC + x) NW + wave) 64 + lane */
+	constexpr int WST = NW * 64 * (int)sizeof(AE);
+	const __amdgpu_buffer_rsrc_t wr = brsrc(wsv, NSET == 2 ?
+	    (int64_t)4 * NACC * WST : 0);
+	const uint32_t wvo = (uint32_t)((wave * 64 + lane) * sizeof(AE));
+
+	/* terms of one W set: role a, role b, role c; set 1 follows set 0 */
+	const int nset_terms = uni(p.nterm1 + p.nterm2);
+	const int nta = uni(p.nterm_a), nt1 = uni(p.nterm1);
+	__syncthreads();
+
+	/* [a][b]@c -> [a][c]@b: per (a block, register) a 32 b x TC c matrix
+	 * for each of the four lane groups, TRC of them per barrier */
+	auto transpose = [&]() {
+		AE *X = (AE *)smem;
+#pragma unroll
+		for (int g = 0; g < 8 / TRC; ++g) {
+			AE *Y = X + (g & 1) * TRB + lg * 32 * TRW;
+#pragma unroll
+			for (int h = 0; h < TRC; ++h) {
+				const int ab = (g * TRC + h) >> 2, r = (g * TRC + h) & 3;
+#pragma unroll
+				for (int x = 0; x < CW; ++x)
+#pragma unroll
+					for (int bb = 0; bb < 2; ++bb)
+						Y[h * 4 * 32 * TRW + (16 * bb + ln) * TRW +
+						    NW * x + wave] = acc[GM::blk1(x, ab, bb)][r];
+			}
+			__syncthreads();
+#pragma unroll
+			for (int h = 0; h < TRC; ++h) {
+				const int ab = (g * TRC + h) >> 2, r = (g * TRC + h) & 3;
+#pragma unroll
+				for (int y = 0; y < BW; ++y)
+#pragma unroll
+					for (int cb = 0; cb < NCB; ++cb)
+						acc[GM::blk2(y, ab, cb)][r] =
+						    Y[h * 4 * 32 * TRW + (NW * y + wave) * TRW +
+						    16 * cb + ln];
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (int x = 0; x < NACC; ++x)
+			pin(acc[x]);
+	};
+
+#pragma unroll 1
+	for (int s = 0; s < NSET; ++s) {
+		const int ts = s * nset_terms;
+		/* a wave without any block has no terms to walk */
+		const int e1 = m1 ? nt1 : 0, ea = m1 ? nta : 0;
+		run_terms<F, NW, CW, 2, PT_ROLE_A, RoleA<GM>>(acc, tp, ts, ts + ea,
+		    B0, na, A0, na, wave, ln, lg, m1);
+		run_terms<F, NW, CW, 2, PT_ROLE_B, RoleB<GM>>(acc, tp, ts + ea,
+		    ts + e1, A0, na, B0, na, wave, ln, lg, m1);
+		transpose();
+		run_terms<F, NW, BW, NCB, PT_ROLE_C, RoleC<GM>>(acc, tp, ts + nt1,
+		    ts + (m2 ? nset_terms : nt1), A0, na, C0, nc, wave, ln, lg, m2);
+		if (NSET == 2 && s == 0) {
+			/* W of set 0 to the save area, lane-contiguous per (r, x,
+			 * wave); the accumulators restart for set 1 */
+#pragma unroll
+			for (int r = 0; r < 4; ++r)
+#pragma unroll
+				for (int x = 0; x < NACC; ++x) {
+					bstore_ae<AE>(wr, wvo, (r * NACC + x) * WST,
+					    acc[x][r]);
+					acc[x][r] = 0;
+				}
+#pragma unroll
+			for (int x = 0; x < NACC; ++x)
+				pin(acc[x]);
+		}
+	}
+
+	/* epilogue: layout [a][c]@b; the lane holds c = C0 + 16 cb + ln.  Each
+	 * (register, a block, c block) column of BW b goes through the lane's
+	 * own LDS slots, so that the element loop runs with a runtime index. */
+	double esum = 0.0, ecmp = 0.0;
+	AE *E = (AE *)smem + wave * (NSET * BW * 64) + lane;
+	/* the tile's epilogue operands that do not depend on a or c alone,
+	 * staged once in LDS behind the W values: the (b, c) blocks of i_oovv
+	 * and t2, [G jk, Z jk, G ik, Z ik (, G ji, Z ji)][32 b][TC c] (mixed
+	 * spin: the GB, ZB blocks; same spin: GA, ZA with ji), the b vectors
+	 * [u i, f i, u j, f j, (u k, f k,) d1 j][32 b] and, for the mixed spin
+	 * case, the (b, a) blocks of the same-spin ones for ji, [GA, ZA][32
+	 * b][32 a] (rows and columns beyond the arrays repeat the last one; the
+	 * epilogue masks those elements).  The transpose's last barrier ended
+	 * every use of this memory. */
+	ER *const stg = (ER *)(smem + EBYTES);
+	const ER *sbc = stg + wave * TC + ln;
+	const ER *sbv = stg + NBC + wave;
+	const ER *sba = stg + NBC + NBV + wave * 32;
+	{
+		/* block n: (G, Z)[n & 1] of pair n / 2 = jk, ik (, ji); mixed
+		 * spin: rows (jk + b) vb, same spin: jk + b v, v = vb */
+		const ER *G = (const ER *)(same ? p.epi.GA : p.epi.GB);
+		const ER *Z = (const ER *)(same ? p.epi.ZA : p.epi.ZB);
+		const int64_t po = same ? p.oa : p.ob;
+		const int64_t pr = same ? p.va * p.va : p.va;
+		const int64_t pjk = ((int64_t)j * po + k) * pr;
+		const int64_t pik = ((int64_t)i * po + k) * pr;
+		const int64_t pji = ((int64_t)j * p.oa + i) * pr;
+#pragma unroll
+		for (int q = 0; q < NBC / NT; ++q) {
+			const int n = tid + q * NT;
+			const int arr = n / (32 * TC), bl = (n / TC) % 32, cl = n % TC;
+			const int b = B0 + bl < na ? B0 + bl : na - 1;
+			const int c = C0 + cl < nc ? C0 + cl : nc - 1;
+			const int64_t pb = arr < 2 ? pjk : arr < 4 ? pik : pji;
+			const int64_t row = same ? pb + (int64_t)b * p.vb :
+			    (pb + b) * p.vb;
+			stg[n] = ((arr & 1) ? Z : G)[row + c];
+		}
+		/* vector n: (u, f)[n & 1] at occupied index (i, j, k)[n / 2], the
+		 * last one d1 at j */
+		if (tid < NBV) {
+			const int arr = tid / 32, bl = tid % 32;
+			const int b = B0 + bl < na ? B0 + bl : na - 1;
+			const int occ = arr < 2 ? i : arr < 4 || arr == NPB ? j : k;
+			const ER *src = arr == NPB ? (const ER *)p.epi.d1 :
+			    (arr & 1) ? (const ER *)p.epi.f1 : (const ER *)p.epi.u1;
+			stg[NBC + tid] = src[occ * p.va + b];
+		}
+	}
+	if constexpr (!same) {
+		const ER *GA = (const ER *)p.epi.GA, *ZA = (const ER *)p.epi.ZA;
+		const int64_t ji = ((int64_t)j * p.oa + i) * p.va;
+#pragma unroll
+		for (int q = 0; q < NBA / NT; ++q) {
+			const int n = tid + q * NT;
+			const int arr = n / 1024, bl = (n / 32) % 32, al = n % 32;
+			const int b = B0 + bl < na ? B0 + bl : na - 1;
+			const int a = A0 + al < na ? A0 + al : na - 1;
+			stg[NBC + NBV + n] = (arr ? ZA : GA)[(ji + b) * p.va + a];
+		}
+	}
+	__syncthreads();
+#pragma unroll
+	for (int ab = 0; ab < 2; ++ab)
+#pragma unroll
+	for (int r = 0; r < 4; ++r)
+#pragma unroll
+	for (int cb = 0; cb < NCB; ++cb) {
+		uint32_t col = 0;
+#pragma unroll
+		for (int y = 0; y < BW; ++y)
+			col |= 1u << GM::blk2(y, ab, cb);
+		if (!(m2 & col))
+			continue;
+#pragma unroll
+		for (int y = 0; y < BW; ++y) {
+			const int x = GM::blk2(y, ab, cb);
+			E[y * 64] = acc[x][r];
+			if (NSET == 2)
+				E[(BW + y) * 64] = bload_ae<AE>(wr, wvo,
+				    (r * NACC + x) * WST);
+		}
+		const int al = 16 * ab + (FM::ROW_F64 ? (lg + 4 * r) : (4 * lg + r));
+		const int a = A0 + al, c = C0 + 16 * cb + ln;
+		if (a < na && c < nc)
+			epi_block<F, KIND, NSET, BW, NW, TC>(p, i, j, k, a, c,
+			    B0 + wave, E, sbc + 16 * cb, sba + al, sbv, esum, ecmp);
+	}
+
+	/* deterministic workgroup reduction */
+	double e = esum - ecmp;
+#pragma unroll
+	for (int off = 32; off >= 1; off >>= 1)
+		e += __shfl_xor(e, off);
+	if (lane == 0)
+		red[wave] = e;
+	__syncthreads();
+	if (tid == 0) {
+		double t = (red[0] + red[1]) + (red[2] + red[3]);
+		if constexpr (NW == 8)
+			t += (red[4] + red[5]) + (red[6] + red[7]);
+		p.partial[it] = t;
+	}
+}
+/* save area `slot` of wsave (two W sets; pt_wsave_bytes each) */
+template <int F, int NW>
+__device__ __forceinline__ typename Form<F>::AE *
+wsave_of(void *wsave, int64_t slot)
+{
+	constexpr int64_t bytes = (int64_t)NW * Geo<F, 2, NW>::NACC * 4 * 64 *
+	    sizeof(typename Form<F>::AE);
+	return (typename Form<F>::AE *)((char *)wsave + slot * bytes);
+}
+
+/*
+ * One launch over items [item0, item0 + n_chunk) of one spin case (item =
+ * ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
+ * and each XCD gets a contiguous run of the launch's items, so the
+ * workgroups running together on one XCD share operand slices in L2.  With
+ * kgrp > 1 that run is taken in groups of kgrp consecutive ijk, tile-major
+ * within a group: the work list holds (i, j, k) with k fastest, and
+ * consecutive k share the slabs of i and j (six of the eight ovvv terms of
+ * the mixed-spin case), which the kgrp items of one tile then read
+ * together.  Each item still writes its own energy at its place in the
+ * work list, so the energies do not depend on kgrp.  One workgroup per
+ * item, handed out by the dispatcher in order; with two W sets item n of
+ * the launch keeps W of set 0 in save area n (n_chunk <= p.nwsave).
+ */
+/* work-list item of launch position it (kgrp > 1: groups of kgrp ijk,
+ * tile-major within a group) */
+__device__ __forceinline__ int64_t
+item_of(const pt_launch &p, int64_t it)
+{
+	if (p.kgrp <= 1)
+		return p.item0 + it;
+	const int64_t nt = p.n_tiles, G = p.kgrp, m = p.n_chunk / nt;
+	const int64_t grp = it / (G * nt), r = it - grp * G * nt;
+	const int64_t gsz = G < m - grp * G ? G : m - grp * G;
+	const int64_t tile = r / gsz, g = r - tile * gsz;
+	return p.item0 + (grp * G + g) * nt + tile;
+}
+
+template <int F, int KIND, int NSET, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void
+k_tiles(pt_launch p)
+{
+	const int64_t per = (p.n_chunk + 7) / 8;
+	const int64_t x = blockIdx.x & 7;
+	const int64_t it = x * per + (blockIdx.x >> 3);
+	if (it >= p.n_chunk)
+		return;
+	tile_item<F, KIND, NSET, NW>(p, item_of(p, it),
+	    NSET == 2 ? wsave_of<F, NW>(p.wsave, it) : nullptr);
+}
+
+/*
+ * The same items from a persistent grid: workgroup w serves XCD w % 8 and
+ * takes that XCD's run of launch positions, [x per, x per + per), one at a
+ * time from the XCD's counter, in order.  The counter is fetched by one
+ * thread between two barriers that every wave meets outside any divergent
+ * branch (the previous item's partial-energy store is behind the first),
+ * the value is read back as a wave-uniform scalar, and the loop ends for
+ * the whole workgroup when it passes the run's end, which the host bounds;
+ * no workgroup waits on another.  With two W sets each workgroup keeps W of
+ * set 0 in its own save area (slot w).
+ */
+template <int F, int KIND, int NSET, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void
+k_tiles_p(pt_launch p)
+{
+	__shared__ int s_next;
+	const int64_t per = (p.n_chunk + 7) / 8;
+	const int x = blockIdx.x & 7;
+	const int64_t lo = x * per;
+	const int64_t cnt = p.n_chunk - lo < per ? p.n_chunk - lo : per;
+	for (;;) {
+		__syncthreads();
+		if (threadIdx.x == 0)
+			s_next = (int)atomicAdd(p.ctr + x, 1u);
+		__syncthreads();
+		const int64_t r = __builtin_amdgcn_readfirstlane(s_next);
+		if (r >= cnt)
+			break;
+		tile_item<F, KIND, NSET, NW>(p, item_of(p, lo + r),
+		    NSET == 2 ? wsave_of<F, NW>(p.wsave, blockIdx.x) : nullptr);
+	}
+}
+
+/* the 8 item counters of a persistent launch, zeroed on its stream by a
+ * kernel (a graph may record it) */
+__global__ void
+k_zero_ctr(uint32_t *c)
+{
+	if (threadIdx.x < 8)
+		c[threadIdx.x] = 0u;
+}
+
+template <int F, int NSET, int NW>
+int
+launch_kind(const pt_launch *p, hipStream_t s)
+{
+	typedef Geo<F, NSET, NW> GM;
+	if (p->tcw != GM::TC)
+		return (int)hipErrorInvalidValue;
+	dim3 block(GM::THREADS);
+	if (p->ctr) {
+		/* persistent grid: one save area per workgroup */
+		if (p->pgrid <= 0 || p->pgrid % 8 || p->n_chunk > INT32_MAX / 2 ||
+		    (NSET == 2 && (!p->wsave || p->pgrid > p->nwsave)))
+			return (int)hipErrorInvalidValue;
+		k_zero_ctr<<<1, 64, 0, s>>>(p->ctr);
+		dim3 grid((unsigned)p->pgrid);
+		if (p->kind == PT_AAA)
+			k_tiles_p<F, PT_AAA, NSET, NW><<<grid, block, 0, s>>>(*p);
+		else
+			k_tiles_p<F, PT_AAB, NSET, NW><<<grid, block, 0, s>>>(*p);
+		return (int)hipGetLastError();
+	}
+	/* one save area per item */
+	if (NSET == 2 && (!p->wsave || p->n_chunk > p->nwsave))
+		return (int)hipErrorInvalidValue;
+	dim3 grid((unsigned)(8 * ((p->n_chunk + 7) / 8)));
+	if (p->kind == PT_AAA)
+		k_tiles<F, PT_AAA, NSET, NW><<<grid, block, 0, s>>>(*p);
+	else
+		k_tiles<F, PT_AAB, NSET, NW><<<grid, block, 0, s>>>(*p);
+	return (int)hipGetLastError();
+}
+
+template <int F>
+int
+launch_form(const pt_launch *p, hipStream_t s)
+{
+	if (p->nw == 8)
+		return p->nset == 1 ? launch_kind<F, 1, 8>(p, s) :
+		    launch_kind<F, 2, 8>(p, s);
+	return p->nset == 1 ? launch_kind<F, 1, 4>(p, s) :
+	    launch_kind<F, 2, 4>(p, s);
+}
+
+} /* namespace */
+
+#endif

@@ -1,0 +1,8 @@
+/* Tile kernels of form PT_FORM_BF16X3 (pt_tiles.h). */
+#include "pt_tiles.h"
+
+extern "C" int
+pt_launch_tiles_bf16x3(const struct pt_launch *p, void *stream)
+{
+	return launch_form<PT_FORM_BF16X3>(p, (hipStream_t)stream);
+}

@@ -1,0 +1,69 @@
+"""Operand fragments of the tile kernel at the edges of their tiles.
+
+- Sizes on both sides of the 16-row blocks, the 4- and 8-wide parts of the c
+  range, the 32-wide tiles and the kappa chunks (8 or 16), the smallest ones
+  included, in every form: tiles cut by the diagonal and by the end of every
+  index skip the blocks outside the triangle and read only fragments that
+  exist.  Bounds: FP64 as for the other parity tests; FP32 and the split
+  forms by their operand precision (FP32 2^-24, split 2^-16 per product).
+- Without the transposed copies (LIBPT_AMD_VC_TRANSPOSED=0, or too little
+  memory for them) the same values come from the plain copies in scattered
+  pieces: per-ijk energies are equal bit for bit."""
+
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from libpt_amd import api
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"fp64": 1e-12, "fp32": 1e-5, "bf16x3": 1e-4, "f16x3": 1e-4}
+SIZES = [(3, 3), (4, 8), (3, 15), (5, 16), (4, 17), (3, 20), (9, 32), (4, 33),
+         (3, 36), (17, 24), (3, 47), (4, 48), (3, 49), (3, 65)]
+
+
+def _energy(kind, form, dims, dev):
+    with api.Plan(kind, form, dims, dev) as pl:
+        pl.run_all()
+        return pl.energy(), [pl.ijk_energies(sc) for sc in range(pl.ncases)]
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "bf16x3", "f16x3"])
+@pytest.mark.parametrize("dims", SIZES, ids=[f"{o}x{v}" for o, v in SIZES])
+def test_tile_edges_match_the_oracle(dims, form):
+    spec = api.make_spec("rpt", dims, seed=sum(dims), sig_f=1e-2)
+    arr = api.synth_host("rpt", spec)
+    eo = oracle.energy("rpt", dims, arr, mp=form == "fp32")
+    dev = api.to_device("rpt", arr, fp32=form == "fp32")
+    try:
+        e, _ = _energy("rpt", form, dims, dev)
+    finally:
+        dev.close()
+    print(dims, form, e, eo)
+    assert abs(e - eo) <= TOL[form] * abs(eo)
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "bf16x3", "f16x3"])
+@pytest.mark.parametrize("kind,dims", [
+    ("rpt", (5, 45)), ("upt", (4, 33, 5, 20)), ("uft", (4, 18, 3, 37))])
+def test_plain_copies_give_the_same_bits(kind, dims, form):
+    spec = api.make_spec(kind, dims, seed=7, sig_f=1e-2,
+                         omega=0.3 if kind == "uft" else 0.0)
+    dev = api.synth_device(kind, spec, fp32=form == "fp32")
+    old = os.environ.get("LIBPT_AMD_VC_TRANSPOSED")
+    try:
+        e0, ijk0 = _energy(kind, form, dims, dev)
+        os.environ["LIBPT_AMD_VC_TRANSPOSED"] = "0"
+        e1, ijk1 = _energy(kind, form, dims, dev)
+    finally:
+        if old is None:
+            os.environ.pop("LIBPT_AMD_VC_TRANSPOSED", None)
+        else:
+            os.environ["LIBPT_AMD_VC_TRANSPOSED"] = old
+        dev.close()
+    assert e0 == e1
+    for a, b in zip(ijk0, ijk1):
+        assert np.array_equal(a, b)
