@@ -90,9 +90,10 @@ double libpt_amd_plan_factor(const libpt_amd_plan *plan, int sc);
 /* tile-kernel geometry of the plan: out3 = (waves per workgroup, c tile
  * width, ijk per item group).  Default: 4 waves (32 x 32 x 16 tiles for
  * FP64, 32 x 32 x 32 for FP32 and the split forms), unless the tuning
- * cache holds a geometry for the plan's sizes; items taken in groups of 4
- * consecutive ijk (tile-major within a group, so that the items of one
- * tile that share the slabs of i and j run together).  LIBPT_AMD_WAVES=4|8
+ * cache holds a geometry for the plan's sizes; items taken in groups of 32
+ * ijk (tile-major within a group, in an order that puts ijk with common
+ * i, j or k together, so that the items of one tile that share their slabs
+ * run together).  LIBPT_AMD_WAVES=4|8
  * and LIBPT_AMD_KGROUP=n (1 to 64) override them for new plans;
  * LIBPT_AMD_PERSISTENT=1 runs new plans' launches on a persistent grid
  * (one workgroup per CU share, items from per-XCD counters, one (fT)

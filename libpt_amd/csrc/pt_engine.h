@@ -151,8 +151,10 @@ struct pt_launch {
 	int32_t kgrp;                /* > 1: the launch covers whole ijk
 	                                (item0 and n_chunk multiples of
 	                                n_tiles) taken in groups of kgrp
-	                                consecutive ijk, each group's items
-	                                tile-major; 1: items in order */
+	                                ijk, each group's items tile-major;
+	                                1: items in order */
+	const int32_t *perm;         /* kgrp > 1: the ijk of positions item0 /
+	                                n_tiles and on (null: themselves) */
 	uint32_t *ctr;               /* non-null: a persistent grid of pgrid
 	                                workgroups takes the items from these
 	                                8 counters (one per XCD, zeroed by the
@@ -204,6 +206,9 @@ int pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
 int pt_launch_pack(const void *src, void *dst, int64_t R, int64_t K,
     int64_t rows, int64_t cols, int tri, int tr, int form, double scale,
     void *stream);
+/* out = the entries of perm[0..n) in [lo, hi), in order (one workgroup) */
+int pt_launch_filter(const int32_t *perm, int64_t n, int32_t lo, int32_t hi,
+    int32_t *out, void *stream);
 int pt_launch_absmax(const double *src, int64_t n, double *out, void *stream);
 int pt_launch_copy(const double *src, double *dst, int64_t n, void *stream);
 int pt_launch_synth(const void *spec, int tensor, void *dst, int64_t n,

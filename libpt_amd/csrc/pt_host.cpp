@@ -280,6 +280,8 @@ struct Case {
 	pt_term_list terms;
 	pt_term *d_terms = nullptr;
 	int32_t *d_ijk = nullptr, *d_tiles = nullptr;
+	int32_t *d_perm = nullptr;  /* launch order of the whole list, */
+	int32_t *d_part = nullptr;  /* and of a range of it (the last one run) */
 	double *d_partial = nullptr;
 	int64_t n_ijk = 0;
 	int n_tiles = 0;
@@ -303,10 +305,16 @@ struct Arena {
 struct libpt_amd_plan {
 	int call = 0, form = 0;
 	int nw = 4;                 /* waves per workgroup of the tile kernel */
-	int kgrp = 4;               /* ijk per item group of a launch: 4
-	                               measured 10 % ahead of 1 for FP64 and
-	                               4 % for split-BF16 at o=45, v=477 (2, 8
-	                               and 16 within 1 % of 4) */
+	int kgrp = 32;              /* ijk per item group of a launch.  Rates in
+	                               TFLOP/s for 64 / 32 / 16 / 8 (tiles in
+	                               8 x 8 x 2 blocks): rpt v=477 mixed spin
+	                               FP64 56.7 / 59.2 / 60.2 / 57.4, split-BF16
+	                               220 / 235 / 238 / 193, same spin FP64 52 /
+	                               54 / 55 / 43; rft v=300 F16X3 same spin
+	                               162 / 144 / 104 / 100; upt v=200 FP32
+	                               90.9 / 97.2 / 97.4 / 94.8.  More share
+	                               their slabs, fewer crowd the same L2
+	                               channels with one tile. */
 	bool copies = true;         /* transposed operand copies (pt_term.tr
 	                               is set without them) */
 	bool fixed_geometry = false; /* a batch's plan: its launches are
@@ -465,24 +473,28 @@ struct ListBuf {
 
 struct ListUpload {
 	int32_t *buf;
-	int n = 0;
+	int n = 0;             /* ints in the buffer */
 	int64_t done = 0;
 	int32_t *dst;
 	bool ok = true;
 	ListUpload(int32_t *d, int32_t *b) : buf(b), dst(d) {}
+	void put(int a)
+	{
+		buf[n] = a;
+		if (++n == 3 * LIST_CHUNK)
+			flush();
+	}
 	void put(int a, int b, int c)
 	{
-		buf[3 * n] = a;
-		buf[3 * n + 1] = b;
-		buf[3 * n + 2] = c;
-		if (++n == LIST_CHUNK)
-			flush();
+		put(a);
+		put(b);
+		put(c);
 	}
 	bool flush()
 	{
 		if (n > 0 && ok) {
-			hipError_t e = hipMemcpy(dst + 3 * done, buf,
-			    3 * sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice);
+			hipError_t e = hipMemcpy(dst + done, buf,
+			    sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice);
 			if (e != hipSuccess) {
 				set_err("list upload failed: %s", hipGetErrorString(e));
 				ok = false;
@@ -571,6 +583,51 @@ case_tiles(libpt_amd_plan *pl, Case &c, int64_t nc, int tcw)
 	return true;
 }
 
+/*
+ * Launch order of the ijk of one spin case: blocks of 4 x 4 x 4 (i, j, k),
+ * in list order within a block; emit(n) gets each triple's place in the work
+ * list (i, then j > i, then k from 0 or, same spin, from j + 1).  The ijk of
+ * a block share their operand slabs (of the eight ovvv terms of the mixed
+ * case three read a Q slab of i, three of j and two of k), so a group of
+ * consecutive ones running the same tile reads each from HBM once: 32 reads
+ * of a term's tile for 64 ijk, where 64 unrelated ones make 512.  Groups of
+ * 32 in this order against groups of 4 in list order (a share of the
+ * triples): rpt v=477 split-BF16 233 -> 209 ms, FP64 270 -> 254 ms; rft
+ * v=300 F16X3 128 -> 103 ms; uft v=160 FP64 137 -> 127 ms; upt v=200 FP32
+ * 196 -> 189 ms.
+ */
+template <class Emit>
+void
+pt_ijk_order(int same, int o1, int o2, Emit emit)
+{
+	constexpr int W = 4;
+	/* list place of (i, j, first k), counted by the triples before it */
+	auto before_i = [&](int64_t i) {
+		const int64_t n = o1;
+		if (!same) /* pairs (i', j) with i' < i, times o2 */
+			return (i * (2 * n - i - 1) / 2) * (int64_t)o2;
+		const int64_t m = n - i; /* C(n, 3) - C(n - i, 3) */
+		return n * (n - 1) * (n - 2) / 6 - m * (m - 1) * (m - 2) / 6;
+	};
+	auto before_j = [&](int64_t i, int64_t j) {
+		if (!same)
+			return (j - i - 1) * (int64_t)o2;
+		const int64_t a = o1 - i - 1, b = o1 - j; /* C(a,2) - C(b,2) */
+		return a * (a - 1) / 2 - b * (b - 1) / 2;
+	};
+	const int ok = same ? o1 : o2;
+	for (int I = 0; I < o1; I += W)
+	for (int J = I; J < o1; J += W)
+	for (int K = same ? J : 0; K < ok; K += W)
+		for (int i = I; i < I + W && i < o1; ++i)
+		for (int j = std::max(J, i + 1); j < J + W && j < o1; ++j) {
+			const int64_t at = before_i(i) + before_j(i, j);
+			const int k0 = same ? j + 1 : 0;
+			for (int k = std::max(K, k0); k < K + W && k < ok; ++k)
+				emit(at + k - k0);
+		}
+}
+
 /* work list of one spin case: ijk items x (A, B, C) tiles */
 bool
 case_lists(libpt_amd_plan *pl, Case &c, int same, int64_t o1, int64_t o2,
@@ -592,6 +649,14 @@ case_lists(libpt_amd_plan *pl, Case &c, int same, int64_t o1, int64_t o2,
 			for (int64_t k = same ? j + 1 : 0; k < (same ? o1 : o2); ++k)
 				ui.put((int)i, (int)j, (int)k);
 	if (!ui.flush())
+		return false;
+	/* the launch order, and room for that of a range (pt_ijk_order) */
+	if (!plan_alloc(pl, (void **)&c.d_perm, sizeof(int32_t) * (size_t)nijk) ||
+	    !plan_alloc(pl, (void **)&c.d_part, sizeof(int32_t) * (size_t)nijk))
+		return false;
+	ListUpload up(c.d_perm, lb.p);
+	pt_ijk_order(same, (int)o1, (int)o2, [&](int64_t n) { up.put((int)n); });
+	if (!up.flush())
 		return false;
 	return case_tiles(pl, c, nc, tcw);
 }
@@ -1104,30 +1169,34 @@ plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 namespace {
 
 /*
- * The tile launches over items [item_b, item_e) of one spin case: grids of
+ * The tile launches over the ijk [ijk_b, ijk_e) of one spin case: grids of
  * at most 2^22 items, and with two W sets of at most wslots (one save area
- * per item).  With base.kgrp > 1, launches hold whole ijk (the kernel
- * takes them in groups of kgrp consecutive ijk); where a launch cannot
- * hold one whole ijk the items go in order.
+ * per item).  With base.kgrp > 1 launches hold whole ijk, taken in the order
+ * of perm (the ijk_e - ijk_b ijk in launch order; null: list order) in
+ * groups of kgrp; where a launch cannot hold one whole ijk the items go in
+ * list order.
  */
 int
-launch_items(int form, const pt_launch &base, int64_t item_b, int64_t item_e,
-    void *wsave, int64_t wslots, hipStream_t st)
+launch_items(int form, const pt_launch &base, int64_t ijk_b, int64_t ijk_e,
+    const int32_t *perm, void *wsave, int64_t wslots, hipStream_t st)
 {
-	const int64_t nt = base.n_tiles;
+	const int64_t nt = base.n_tiles, n = (ijk_e - ijk_b) * nt;
 	int64_t chunk = base.nset == 2 && !base.ctr ? wslots : (int64_t)1 << 22;
 	int kg = base.kgrp;
 	if (kg > 1) {
-		if (item_b % nt || item_e % nt || chunk < nt)
+		if (chunk < nt)
 			kg = 1;
 		else
 			chunk = chunk / nt * nt;
 	}
-	for (int64_t it = item_b; it < item_e; it += chunk) {
+	if (kg <= 1)
+		perm = nullptr;
+	for (int64_t it = 0; it < n; it += chunk) {
 		pt_launch L = base;
-		L.item0 = it;
-		L.n_chunk = std::min(chunk, item_e - it);
+		L.item0 = it + (perm ? 0 : ijk_b * nt);
+		L.n_chunk = std::min(chunk, n - it);
 		L.kgrp = kg;
+		L.perm = perm;
 		L.wsave = wsave;
 		L.nwsave = (int32_t)wslots;
 		const int rc = pt_launch_tiles(form, &L, st);
@@ -1223,8 +1292,20 @@ libpt_amd_plan_run(libpt_amd_plan *pl, int sc, int64_t b, int64_t e)
 		return 0;
 	if (c.L.nset == 2 && !plan_wsave(pl))
 		return -1;
-	const int rc = launch_items(pl->form, c.L, b * c.n_tiles,
-	    e * c.n_tiles, pl->wsave, pl->wslots, pl->stream);
+	/* a range of more than one group goes in the whole list's launch order
+	 * (within one group the order does not matter) */
+	const int32_t *perm = nullptr;
+	int rc = 0;
+	if (b == 0 && e == c.n_ijk) {
+		perm = c.d_perm;
+	} else if (c.L.kgrp > 1 && e - b > c.L.kgrp) {
+		rc = pt_launch_filter(c.d_perm, c.n_ijk, (int32_t)b, (int32_t)e,
+		    c.d_part, pl->stream);
+		perm = c.d_part;
+	}
+	if (rc == 0)
+		rc = launch_items(pl->form, c.L, b, e, perm, pl->wsave, pl->wslots,
+		    pl->stream);
 	if (rc != 0) {
 		set_err("tile kernel launch failed: %s",
 		    hipGetErrorString((hipError_t)rc));
@@ -1559,7 +1640,8 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 		pt_launch L;
 		int sys, sc;
 		double factor, cost;
-		int64_t items;
+		int64_t nijk, items;
+		const int32_t *perm;
 	};
 	std::vector<Seg> segs;
 	for (int s = 0; s < n; ++s) {
@@ -1579,7 +1661,9 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 			g.sc = sc;
 			g.L = c.L;
 			g.L.item0 = 0;
+			g.nijk = c.n_ijk;
 			g.items = c.n_ijk * c.n_tiles;
+			g.perm = c.d_perm;
 			g.L.n_chunk = g.items;
 			g.sys = s;
 			g.factor = c.factor;
@@ -1644,8 +1728,8 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	    hipSuccess || (set_err("stream capture failed"), false));
 	int rc = 0;
 	for (int g = 0; g < nseg && rc == 0; ++g)
-		rc = launch_items(form, L[g], 0, segs[g].items, b->wsave, b->wslots,
-		    b->stream);
+		rc = launch_items(form, L[g], 0, segs[g].nijk, segs[g].perm,
+		    b->wsave, b->wslots, b->stream);
 	if (rc == 0)
 		rc = pt_launch_reduce_batch(b->d_segs, b->d_begin, nseg, b->d_out,
 		    b->stream);
@@ -1905,9 +1989,9 @@ namespace {
 /* The part of an allocation-free call's scratch that decides whether the
  * call is taken (LIBPT_AMD_NOALLOC_SCRATCH): the operand copies in the sizes
  * of their arrays with kappa padded to whole chunks, the lists, energies
- * and term tables, and one (fT) save area.  The packed rows' padding and
- * the transposed copies come on top of it, out of the rest of the static
- * array. */
+ * and term tables, and one (fT) save area.  The packed rows' padding, the
+ * transposed copies and the launch order come on top of it, out of the rest
+ * of the static array. */
 int64_t
 noalloc_need(const libpt_amd_plan &pl)
 {

@@ -159,6 +159,36 @@ k_pack(const void *src, char *dst, int64_t K, int64_t rows, int64_t cols,
 	}
 }
 
+/* the entries of perm in [lo, hi), in order, by one workgroup: 16 waves
+ * take consecutive runs of 64 entries and add the counts of the waves
+ * before them */
+__global__ __launch_bounds__(1024) void
+k_filter(const int32_t *perm, int64_t n, int32_t lo, int32_t hi, int32_t *out)
+{
+	__shared__ int cnt[2][16];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	int64_t base = 0;
+	for (int64_t t0 = 0, b = 0; t0 < n; t0 += 1024, b ^= 1) {
+		const int64_t t = t0 + threadIdx.x;
+		const int32_t x = t < n ? perm[t] : -1;
+		const bool in = t < n && x >= lo && x < hi;
+		const uint64_t m = __ballot(in);
+		if (lane == 0)
+			cnt[b][wave] = __popcll(m);
+		/* the other buffer's readers have passed this barrier's
+		 * predecessor when it is written again */
+		__syncthreads();
+		int64_t at = base;
+		for (int w = 0; w < 16; ++w) {
+			if (w < wave)
+				at += cnt[b][w];
+			base += cnt[b][w];
+		}
+		if (in)
+			out[at + __popcll(m & ((1ull << lane) - 1))] = x;
+	}
+}
+
 /* hi + lo split of (x * scale) into bf16 or fp16 pairs */
 __global__ void
 k_split(const double *src, uint32_t *dst, int64_t n, int fp16, double scale)
@@ -315,6 +345,16 @@ pt_launch_pack(const void *src, void *dst, int64_t R, int64_t K, int64_t rows,
 			return rc;
 	}
 	return 0;
+}
+
+extern "C" int
+pt_launch_filter(const int32_t *perm, int64_t n, int32_t lo, int32_t hi,
+    int32_t *out, void *stream)
+{
+	if (n <= 0)
+		return 0;
+	k_filter<<<1, 1024, 0, (hipStream_t)stream>>>(perm, n, lo, hi, out);
+	return (int)hipGetLastError();
 }
 
 extern "C" int

@@ -944,19 +944,18 @@ wsave_of(void *wsave, int64_t slot)
 /*
  * One launch over items [item0, item0 + n_chunk) of one spin case (item =
  * ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
- * and each XCD gets a contiguous run of the launch's items, so the
- * workgroups running together on one XCD share operand slices in L2.  With
- * kgrp > 1 that run is taken in groups of kgrp consecutive ijk, tile-major
- * within a group: the work list holds (i, j, k) with k fastest, and
- * consecutive k share the slabs of i and j (six of the eight ovvv terms of
- * the mixed-spin case), which the kgrp items of one tile then read
- * together.  Each item still writes its own energy at its place in the
- * work list, so the energies do not depend on kgrp.  One workgroup per
- * item, handed out by the dispatcher in order; with two W sets item n of
- * the launch keeps W of set 0 in save area n (n_chunk <= p.nwsave).
+ * and each XCD gets a contiguous run of the launch's positions, so the
+ * workgroups running together on one XCD share operand slices in its L2.
+ * With kgrp > 1 the positions take the ijk in groups of kgrp, tile-major
+ * within a group, in the order of the perm list (null: the work list's),
+ * which puts ijk that share slabs next to each other (pt_ijk_order): the 64
+ * workgroups that an XCD runs together are on a tile or two, for ijk that
+ * share their slabs.  Each item still writes its own energy at its place in
+ * the work list, so the energies do not depend on kgrp or perm.  One
+ * workgroup per item, handed out by the dispatcher in order; with two W
+ * sets position n of the launch keeps W of set 0 in save area n (n_chunk <=
+ * p.nwsave).
  */
-/* work-list item of launch position it (kgrp > 1: groups of kgrp ijk,
- * tile-major within a group) */
 __device__ __forceinline__ int64_t
 item_of(const pt_launch &p, int64_t it)
 {
@@ -966,7 +965,8 @@ item_of(const pt_launch &p, int64_t it)
 	const int64_t grp = it / (G * nt), r = it - grp * G * nt;
 	const int64_t gsz = G < m - grp * G ? G : m - grp * G;
 	const int64_t tile = r / gsz, g = r - tile * gsz;
-	return p.item0 + (grp * G + g) * nt + tile;
+	const int64_t pos = p.item0 / nt + grp * G + g;
+	return (p.perm ? (int64_t)p.perm[pos] : pos) * nt + tile;
 }
 
 template <int F, int KIND, int NSET, int NW>
