@@ -140,21 +140,23 @@ struct pt_launch {
 	const int32_t *ijk;          /* [n_ijk][3] */
 	const int32_t *tiles;        /* [n_tiles][3]: blocks (A, B, C), A >= B */
 	int32_t n_tiles, nw;         /* tiles per ijk, waves per workgroup */
-	int64_t item0, n_chunk;      /* items [item0, item0 + n_chunk) */
+	int64_t item0, n_seq;        /* a run of items: n_seq of them, from item0
+	                                (whole ijk); its positions are ordered
+	                                by kgrp and perm */
+	int64_t pos0, n_chunk;       /* the launch's: positions [pos0, pos0 +
+	                                n_chunk) of the run */
 	double *partial;             /* energy of each item */
 	double inv_scale[2];         /* per W set: 1 / (operand scale product) */
 	void *wsave;                 /* two W sets: W of set 0 of each item
 	                                of the launch (pt_wsave_bytes each,
-	                                item item0 + n at slot n), else
+	                                position pos0 + n at slot n), else
 	                                unused */
 	int32_t nwsave;              /* save areas in wsave (>= n_chunk) */
-	int32_t kgrp;                /* > 1: the launch covers whole ijk
-	                                (item0 and n_chunk multiples of
-	                                n_tiles) taken in groups of kgrp
-	                                ijk, each group's items tile-major;
-	                                1: items in order */
-	const int32_t *perm;         /* kgrp > 1: the ijk of positions item0 /
-	                                n_tiles and on (null: themselves) */
+	int32_t kgrp;                /* > 1: the run's ijk are taken in groups
+	                                of kgrp, each group's items
+	                                tile-major; 1: items in order */
+	const int32_t *perm;         /* kgrp > 1: the run's ijk in order (null:
+	                                item0 / n_tiles and on) */
 	uint32_t *ctr;               /* non-null: a persistent grid of pgrid
 	                                workgroups takes the items from these
 	                                8 counters (one per XCD, zeroed by the

@@ -1171,10 +1171,8 @@ namespace {
 /*
  * The tile launches over the ijk [ijk_b, ijk_e) of one spin case: grids of
  * at most 2^22 items, and with two W sets of at most wslots (one save area
- * per item).  With base.kgrp > 1 launches hold whole ijk, taken in the order
- * of perm (the ijk_e - ijk_b ijk in launch order; null: list order) in
- * groups of kgrp; where a launch cannot hold one whole ijk the items go in
- * list order.
+ * per item), over positions in the order of perm (the ijk_e - ijk_b ijk in
+ * launch order; null: list order) and base.kgrp.
  */
 int
 launch_items(int form, const pt_launch &base, int64_t ijk_b, int64_t ijk_e,
@@ -1182,23 +1180,15 @@ launch_items(int form, const pt_launch &base, int64_t ijk_b, int64_t ijk_e,
 {
 	const int64_t nt = base.n_tiles, n = (ijk_e - ijk_b) * nt;
 	int64_t chunk = base.nset == 2 && !base.ctr ? wslots : (int64_t)1 << 22;
-	int kg = base.kgrp;
-	if (kg > 1) {
-		if (chunk < nt)
-			kg = 1;
-		else
-			chunk = chunk / nt * nt;
-	}
-	if (kg <= 1)
-		perm = nullptr;
+	pt_launch L = base;
+	L.perm = base.kgrp > 1 ? perm : nullptr;
+	L.item0 = L.perm ? 0 : ijk_b * nt;
+	L.n_seq = n;
+	L.wsave = wsave;
+	L.nwsave = (int32_t)wslots;
 	for (int64_t it = 0; it < n; it += chunk) {
-		pt_launch L = base;
-		L.item0 = it + (perm ? 0 : ijk_b * nt);
+		L.pos0 = it;
 		L.n_chunk = std::min(chunk, n - it);
-		L.kgrp = kg;
-		L.perm = perm;
-		L.wsave = wsave;
-		L.nwsave = (int32_t)wslots;
 		const int rc = pt_launch_tiles(form, &L, st);
 		if (rc != 0)
 			return rc;
@@ -1660,11 +1650,9 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 			Seg g;
 			g.sc = sc;
 			g.L = c.L;
-			g.L.item0 = 0;
 			g.nijk = c.n_ijk;
 			g.items = c.n_ijk * c.n_tiles;
 			g.perm = c.d_perm;
-			g.L.n_chunk = g.items;
 			g.sys = s;
 			g.factor = c.factor;
 			g.cost = c.flop_per_ijk / c.n_tiles;

@@ -942,8 +942,8 @@ wsave_of(void *wsave, int64_t slot)
 }
 
 /*
- * One launch over items [item0, item0 + n_chunk) of one spin case (item =
- * ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
+ * One launch over n_chunk positions of a run of one spin case's items (item
+ * = ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
  * and each XCD gets a contiguous run of the launch's positions, so the
  * workgroups running together on one XCD share operand slices in its L2.
  * With kgrp > 1 the positions take the ijk in groups of kgrp, tile-major
@@ -959,9 +959,10 @@ wsave_of(void *wsave, int64_t slot)
 __device__ __forceinline__ int64_t
 item_of(const pt_launch &p, int64_t it)
 {
+	it += p.pos0;
 	if (p.kgrp <= 1)
 		return p.item0 + it;
-	const int64_t nt = p.n_tiles, G = p.kgrp, m = p.n_chunk / nt;
+	const int64_t nt = p.n_tiles, G = p.kgrp, m = p.n_seq / nt;
 	const int64_t grp = it / (G * nt), r = it - grp * G * nt;
 	const int64_t gsz = G < m - grp * G ? G : m - grp * G;
 	const int64_t tile = r / gsz, g = r - tile * gsz;
