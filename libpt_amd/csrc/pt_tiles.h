@@ -77,7 +77,7 @@ template <> struct Form<PT_FORM_FP64> {
 	typedef v4d ACC;
 	typedef double ER;  /* epilogue real */
 	static constexpr int KC = 8;    /* kappa per fragment */
-	static constexpr bool ROW_F64 = true, SPLIT = false;
+	static constexpr bool ROW_F64 = true, SPLIT = false, PAN = false;
 };
 
 template <> struct Form<PT_FORM_FP32> {
@@ -86,7 +86,7 @@ template <> struct Form<PT_FORM_FP32> {
 	typedef v4f ACC;
 	typedef float ER;
 	static constexpr int KC = 16;
-	static constexpr bool ROW_F64 = false, SPLIT = false;
+	static constexpr bool ROW_F64 = false, SPLIT = false, PAN = false;
 };
 
 template <> struct Form<PT_FORM_BF16X3> {
@@ -96,6 +96,7 @@ template <> struct Form<PT_FORM_BF16X3> {
 	typedef double ER;
 	static constexpr int KC = 16;
 	static constexpr bool ROW_F64 = false, SPLIT = true;
+	static constexpr bool PAN = true;   /* S staged in LDS panels */
 };
 
 template <> struct Form<PT_FORM_F16X3> : Form<PT_FORM_BF16X3> {};
@@ -465,29 +466,63 @@ make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
  * in flight per wave and every load has one step to arrive; the loads after
  * the last step are all out of range and return zero.
  *
+ * S is the same for all waves, and its rows are scattered 64-byte pieces in
+ * the API layout: loaded by each wave for itself, a 16-row block costs the
+ * vector cache as much as four Q fragments.  FP64 and FP32, whose steps take
+ * 2048 and 4096 MFMA cycles, do that.  In the split forms (1024 cycles) S
+ * was a third of the cache accesses and a sixth of the L2 requests, so there
+ * the waves stage it together in LDS (PAN), in panels of PC
+ * steps: while a panel is used, each wave loads its NI fragments of the next
+ * one into registers; they go to the other of two buffers at the panel's
+ * end, behind the only barrier of the loop.  A fragment is [row][quarter ^
+ * (row / 4)] in 16-byte pieces: the four lanes of a row load 64 contiguous
+ * bytes, and the 16 lanes of a read phase (rows at one quarter) fall on
+ * distinct banks.  rft v=300 F16X3 101 -> 92 ms, rpt v=477 split-BF16 210 ->
+ * 206 ms (128 mixed-spin ijk of it 235 -> 259 TFLOP/s); in FP64 it gave
+ * nothing at v=477 and cost 2 to 4 % at v=64 to 160, where the barriers
+ * couple the waves.
+ *
  * One loop serves full and cut tiles: with loop variants chosen by control
  * flow the accumulators, more than half of the registers, meet at joins
  * after every variant, and the register allocator then spills dozens of
  * blocks there and inside the loops.
  */
+constexpr int PC = 8;               /* steps per S panel */
+constexpr int PANEL = PC * 2 * 1024; /* bytes, for two S blocks */
+
+/* a barrier that waits for this wave's LDS accesses only (the compiler's
+ * waits for every global load in flight too) */
+__device__ __forceinline__ void
+lds_barrier()
+{
+	__asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+	__builtin_amdgcn_s_barrier();
+	__asm__ volatile("" ::: "memory");
+}
+
+/* panels: two panel buffers; par: the one to fill first, updated (the
+ * previous call's last panel may still be read from the other) */
 template <int F, int NW, int NX, int NSB, int ROLE, class B, int NACC>
 __device__ __forceinline__ void
 run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
     int u0, int uext, int s0, int sext, int wave, int ln, int lg,
-    uint32_t mask)
+    uint32_t mask, char *panels, int &par)
 {
 	static_assert(Form<F>::KC * sizeof(typename Form<F>::G) == 64,
 	    "a chunk of S is 64 bytes per row");
 	constexpr bool QA = ROLE != PT_ROLE_A;
 	constexpr int XB = 16 / NW;      /* x per 16 w */
+	/* panel fragments (step, S block) are dealt to the waves in order */
+	constexpr bool PAN = Form<F>::PAN;
+	constexpr int NI = PAN ? PC * NSB / NW : NSB, ND = NW / NSB;
+	static_assert(PC * NSB % NW == 0 && NW % NSB == 0, "panel split");
 	if (t0 >= t1)
 		return;
-	uint64_t q0, q1, sp;
+	uint64_t q0, q1;
 	uint32_t dq0, dq1, xa, xb, sgn;
-	int sb;
 	int left;
 	bool more = true;
-	uint32_t vo[2], so[NSB];
+	uint32_t vo[2];
 	/* the x of each e that may be read (xhi < 0: none), the groups */
 	constexpr int NH = NX / 2;
 	int xlo[2], xhi[2];
@@ -514,15 +549,12 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 		const TermP &T = tp[t];
 		q0 = (uint64_t)uni64((int64_t)T.q[0]);
 		q1 = (uint64_t)uni64((int64_t)T.q[1]);
-		sp = (uint64_t)uni64((int64_t)T.s);
 		dq0 = (uint32_t)uni((int)T.dq[0]);
 		dq1 = (uint32_t)uni((int)T.dq[1]);
 		xa = (uint32_t)uni((int)T.xa);
 		xb = (uint32_t)uni((int)T.xb);
-		sb = uni((int)T.sbytes);
 		sgn = (uint32_t)uni((int)T.sgn);
 		left = uni(T.nch);
-		const uint32_t sst = (uint32_t)uni((int)T.sst);
 		const bool tr = uni(T.tr) != 0;
 		q0 += (uint64_t)xa * (uint32_t)wave;
 		q1 += (uint64_t)xa * (uint32_t)wave;
@@ -532,10 +564,6 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 			    (uint32_t)(16 * (16 * lg + ln)) :
 			    u0 + 16 * e + ln < uext ?
 			    (uint32_t)(1024 * ln + 256 * lg) : PT_OOR;
-#pragma unroll
-		for (int e = 0; e < NSB; ++e)
-			so[e] = s0 + 16 * e + ln < sext ?
-			    (uint32_t)(s0 + 16 * e + ln) * sst + 16u * lg : PT_OOR;
 	};
 	/* lanes without data take an offset that every descriptor rejects; the
 	 * scalar offset is never relied on for a range check */
@@ -547,47 +575,94 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 		    (int)vo[e], (int)((uint32_t)(x % XB) * NW * xa +
 		    (uint32_t)(x / XB) * xb), 0));
 	};
-	auto load_s = [&](int e) {
-		const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-		    (void *)sp, (short)0, sb, 0x00020000);
-		return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r,
-		    (int)so[e], 0, 0));
+	/* S loads.  PAN: panel staging, this wave's S block, and its next step
+	 * as (term st, chunk sc).  Else both blocks of the next step. */
+	const int lane = 16 * lg + ln, se = PAN ? wave % NSB : 0;
+	const int srow = s0 + 16 * se + (PAN ? lane >> 2 : ln);
+	const uint32_t sq = 16u * (PAN ? (lane & 3) ^ (lane >> 4) : lg);
+	int st = t0, sc = PAN ? wave / NSB : 0, snch, sbytes;
+	uint64_t sp;
+	uint32_t so[PAN ? 1 : NSB];
+	auto sterm = [&]() {
+		const TermP &T = tp[st];
+		sp = (uint64_t)uni64((int64_t)T.s);
+		sbytes = uni((int)T.sbytes);
+		snch = uni(T.nch);
+		const uint32_t sst = (uint32_t)uni((int)T.sst);
+#pragma unroll
+		for (int e = 0; e < (PAN ? 1 : NSB); ++e)
+			so[e] = srow + 16 * e < sext ?
+			    (uint32_t)(srow + 16 * e) * sst + sq : PT_OOR;
 	};
+	v4u sr[NI];
+	auto stage_load = [&]() {
+#pragma unroll
+		for (int i = 0; i < NI; ++i) {
+			if (PAN || i == 0)
+				while (sc >= snch && st < t1) {
+					sc -= snch;
+					if (++st < t1) {
+						sterm();
+					} else {
+#pragma unroll
+						for (int e = 0; e < (PAN ? 1 : NSB); ++e)
+							so[e] = PT_OOR;
+					}
+				}
+			const int at = 64 * sc;   /* KC elements of S per chunk */
+			const __amdgpu_buffer_rsrc_t r =
+			    __builtin_amdgcn_make_buffer_rsrc((void *)(sp + at),
+			    (short)0, sbytes > at ? sbytes - at : 0, 0x00020000);
+			sr[i] = __builtin_bit_cast(v4u,
+			    __builtin_amdgcn_raw_buffer_load_b128(r,
+			    (int)so[PAN ? 0 : i], 0, 0));
+			if (PAN)
+				sc += ND;
+		}
+		if (!PAN)
+			++sc;
+	};
+	auto stage_write = [&]() {
+		char *d = panels + par * PANEL + 1024 * wave + 16 * lane;
+#pragma unroll
+		for (int i = 0; i < NI; ++i)
+			*(v4u *)(d + 1024 * NW * i) = sr[i];
+	};
+	const uint32_t rofs = 16u * (4 * ln + (lg ^ (ln >> 2)));
 
 	term(t0);
-	int t = t0;
-	v4u q[2 * NX], sr[NSB];
-#pragma unroll
-	for (int e = 0; e < NSB; ++e)
-		sr[e] = load_s(e);
+	sterm();
+	int t = t0, n = 0;
+	stage_load();
+	v4u q[2 * NX];
 #pragma unroll
 	for (int x = 0; x < NX; ++x)
 #pragma unroll
 		for (int e = 0; e < 2; ++e)
 			q[2 * x + e] = load_q(x, e);
+	if constexpr (PAN) {
+		stage_write();
+		lds_barrier();
+		stage_load();
+	}
 	do {
 		SFrag<F> s[NSB];
 #pragma unroll
 		for (int e = 0; e < NSB; ++e)
-			s[e].set(sr[e], sgn);
+			s[e].set(PAN ? *(const v4u *)(panels + par * PANEL + rofs +
+			    1024 * (NSB * n + e)) : sr[e], sgn);
 		/* on to the next step */
 		if (--left > 0) {
 			q0 += dq0;
 			q1 += dq1;
-			sp += 64;       /* KC elements of S */
-			sb = sb - 64 > 0 ? sb - 64 : 0;
 		} else if (++t < t1) {
 			term(t);
 		} else {
 			more = false;
 			vo[0] = vo[1] = PT_OOR;
-#pragma unroll
-			for (int e = 0; e < NSB; ++e)
-				so[e] = PT_OOR;
 		}
-#pragma unroll
-		for (int e = 0; e < NSB; ++e)
-			sr[e] = load_s(e);
+		if constexpr (!PAN)
+			stage_load();
 #pragma unroll
 		for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -609,7 +684,18 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 				q[2 * x + e] = load_q(x, e);
 			__builtin_amdgcn_sched_barrier(0);
 		}
+		if (PAN && ++n == PC) {
+			n = 0;
+			par ^= 1;
+			if (more) {
+				stage_write();
+				lds_barrier();
+				stage_load();
+			}
+		}
 	} while (more);
+	if (n != 0)
+		par ^= 1;
 }
 
 /* -------------------------------------------------------------- kernel */
@@ -679,8 +765,8 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
 	constexpr int NACC = GM::NACC, NT = GM::THREADS;
 	constexpr bool same = KIND == PT_AAA;
 
-	/* LDS: the transpose's buffers (two of TRC (a block, register) columns
-	 * each), then the epilogue's W columns and staged operands */
+	/* LDS: the S panels; the transpose's buffers (two of TRC (a block,
+	 * register) columns each); the epilogue's W columns and staged operands */
 	constexpr int TRW = TC + 1, TRC = 2;
 	constexpr int TRB = TRC * 4 * 32 * TRW;      /* values per buffer */
 	constexpr int NPB = same ? 6 : 4;            /* (b, c) blocks */
@@ -690,6 +776,7 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
 	constexpr int SB1 = 2 * TRB * (int)sizeof(AE);
 	constexpr int SB2 = EBYTES + (NBC + NBV + NBA) * (int)sizeof(ER);
 	constexpr int SMEM = SB1 > SB2 ? SB1 : SB2;
+	static_assert(SMEM >= 2 * PANEL, "the S panels");
 	constexpr int NTERM = NSET * (same ? PT_TERMS_SAME : PT_TERMS_MIXED);
 	static_assert((SMEM + NTERM * (int)sizeof(TermP) + 8 * NW + 64) *
 	    GM::WG_PER_CU <= 160 * 1024, "LDS of the workgroups of a CU");
@@ -797,18 +884,24 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
 			pin(acc[x]);
 	};
 
+	int par = 0;   /* S panel buffer */
 #pragma unroll 1
 	for (int s = 0; s < NSET; ++s) {
 		const int ts = s * nset_terms;
-		/* a wave without any block has no terms to walk */
-		const int e1 = m1 ? nt1 : 0, ea = m1 ? nta : 0;
-		run_terms<F, NW, CW, 2, PT_ROLE_A, RoleA<GM>>(acc, tp, ts, ts + ea,
-		    B0, na, A0, na, wave, ln, lg, m1);
-		run_terms<F, NW, CW, 2, PT_ROLE_B, RoleB<GM>>(acc, tp, ts + ea,
-		    ts + e1, A0, na, B0, na, wave, ln, lg, m1);
+		/* a wave without any block has no terms to walk (with panels it
+		 * stages its part all the same) */
+		const bool w1 = m1 || FM::PAN, w2 = m2 || FM::PAN;
+		run_terms<F, NW, CW, 2, PT_ROLE_A, RoleA<GM>>(acc, tp, ts,
+		    ts + (w1 ? nta : 0), B0, na, A0, na, wave, ln, lg, m1, smem, par);
+		run_terms<F, NW, CW, 2, PT_ROLE_B, RoleB<GM>>(acc, tp, ts + nta,
+		    ts + (w1 ? nt1 : nta), A0, na, B0, na, wave, ln, lg, m1, smem,
+		    par);
+		if (FM::PAN)
+			lds_barrier();   /* the last panel's reads */
 		transpose();
 		run_terms<F, NW, BW, NCB, PT_ROLE_C, RoleC<GM>>(acc, tp, ts + nt1,
-		    ts + (m2 ? nset_terms : nt1), A0, na, C0, nc, wave, ln, lg, m2);
+		    ts + (w2 ? nset_terms : nt1), A0, na, C0, nc, wave, ln, lg, m2,
+		    smem, par);
 		if (NSET == 2 && s == 0) {
 			/* W of set 0 to the save area, lane-contiguous per (r, x,
 			 * wave); the accumulators restart for set 1 */
@@ -838,8 +931,9 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
 	 * [u i, f i, u j, f j, (u k, f k,) d1 j][32 b] and, for the mixed spin
 	 * case, the (b, a) blocks of the same-spin ones for ji, [GA, ZA][32
 	 * b][32 a] (rows and columns beyond the arrays repeat the last one; the
-	 * epilogue masks those elements).  The transpose's last barrier ended
-	 * every use of this memory. */
+	 * epilogue masks those elements). */
+	if (FM::PAN)
+		lds_barrier();   /* the last panel's reads */
 	ER *const stg = (ER *)(smem + EBYTES);
 	const ER *sbc = stg + wave * TC + ln;
 	const ER *sbv = stg + NBC + wave;
