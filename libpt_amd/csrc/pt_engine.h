@@ -196,7 +196,9 @@ int pt_launch_tiles_f16x3(const struct pt_launch *p, void *stream);
 /* out[s] = fixed-order sum of segment s's partials (as pt_launch_reduce) */
 int pt_launch_reduce_batch(const struct pt_launch *segs,
     const int64_t *begin, int nseg, double *out, void *stream);
-int pt_launch_reduce(const double *x, int64_t n, double *out, void *stream);
+/* out[q] = fixed-order sum of x[q][0..n[q]) for q < cnt <= 4 */
+int pt_launch_reduce(const double *const *x, const int64_t *n, int cnt,
+    double *out, void *stream);
 int pt_launch_segsum(const double *x, int64_t nseg, int64_t seglen,
     double *out, void *stream);
 int pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
@@ -204,9 +206,16 @@ int pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
 /* [R slabs][K][plane] -> packed slabs (pt_slab_frags) of the plane's rows
  * and columns; the source plane is [rows][cols], [cols][rows] (tr), or the
  * packed pairs row > column (tri); the split forms store hi and lo of
- * x * scale */
-int pt_launch_pack(const void *src, void *dst, int64_t R, int64_t K,
-    int64_t rows, int64_t cols, int tri, int tr, int form, double scale,
+ * x * scale.  at: set by the launch. */
+struct pt_pack_job {
+	const char *src;
+	char *dst;
+	int64_t R, K, rows, cols;
+	double scale;
+	int64_t at;
+	int32_t tri, tr;
+};
+int pt_launch_pack(const struct pt_pack_job *jobs, int n, int form,
     void *stream);
 /* out = the entries of perm[0..n) in [lo, hi), in order (one workgroup) */
 int pt_launch_filter(const int32_t *perm, int64_t n, int32_t lo, int32_t hi,

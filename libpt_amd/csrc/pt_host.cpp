@@ -345,13 +345,48 @@ struct libpt_amd_plan {
 
 namespace {
 
+/* Idle streams of finished plans, at most IDLE_STREAMS of them (creating and
+ * destroying one costs 35 us, a tenth of a small call); under g_mu.  A
+ * plan's stream is idle when it is given back (plan_release synchronises
+ * it). */
+enum { IDLE_STREAMS = 8 };
+FixedVec<hipStream_t, IDLE_STREAMS> g_idle;
+
+bool
+stream_get(hipStream_t *st)
+{
+	{
+		std::lock_guard<std::mutex> lk(g_mu);
+		if (!g_idle.empty()) {
+			*st = g_idle[g_idle.size() - 1];
+			g_idle.n--;
+			return true;
+		}
+	}
+	return hipStreamCreateWithFlags(st, hipStreamNonBlocking) == hipSuccess;
+}
+
+void
+stream_put(hipStream_t st)
+{
+	{
+		std::lock_guard<std::mutex> lk(g_mu);
+		if (g_idle.size() < IDLE_STREAMS) {
+			g_idle.push_back(st);
+			return;
+		}
+	}
+	(void)hipStreamDestroy(st);
+}
+
 /* waits for the plan's work, then frees what it owns (not the plan) */
 void
 plan_release(libpt_amd_plan *pl)
 {
 	/* a caller's stream may be the null stream */
+	bool idle = true;
 	if (pl->stream || !pl->own_stream)
-		(void)hipStreamSynchronize(pl->stream);
+		idle = hipStreamSynchronize(pl->stream) == hipSuccess;
 	for (void *p : pl->owned)
 		(void)hipFree(p);
 	pl->owned.clear();
@@ -359,8 +394,12 @@ plan_release(libpt_amd_plan *pl)
 		(void)hipEventDestroy(pl->ev0);
 	if (pl->ev1)
 		(void)hipEventDestroy(pl->ev1);
-	if (pl->stream && pl->own_stream)
-		(void)hipStreamDestroy(pl->stream);
+	if (pl->stream && pl->own_stream) {
+		if (idle)
+			stream_put(pl->stream);
+		else
+			(void)hipStreamDestroy(pl->stream);
+	}
 	pl->ev0 = pl->ev1 = nullptr;
 	pl->stream = nullptr;
 }
@@ -448,40 +487,43 @@ plan_drop(libpt_amd_plan *pl, void *p)
 		}
 }
 
-/* Host lists go to the device in chunks of N triples of ints through one
- * chunk buffer: host scratch from the libpt_set_malloc hooks (as the
- * reference takes its scratch, src/pt.c:208,223), or a stack array for
- * the allocation-free entry point. */
-enum { LIST_CHUNK = 2048 };
+/* Host lists go to the device as one stream of ints, in chunks through one
+ * buffer: host scratch from the libpt_set_malloc hooks (as the reference
+ * takes its scratch, src/pt.c:208,223), or a stack array for the
+ * allocation-free entry point.  A copy costs about 14 us whatever its size,
+ * so a small call's lists go in one. */
+enum { LIST_STACK = 6144, LIST_HEAP = 65536 };
 
 struct ListBuf {
-	int32_t stack_[3 * LIST_CHUNK];
+	int32_t stack_[LIST_STACK];
 	HostBuf<int32_t> heap_;
 	int32_t *p = nullptr;
+	int cap = 0;
 	bool get(const libpt_amd_plan *pl)
 	{
 		if (pl->arena) {
 			p = stack_;
+			cap = LIST_STACK;
 			return true;
 		}
-		if (!heap_.alloc(3 * LIST_CHUNK))
+		if (!heap_.alloc(LIST_HEAP))
 			return false;
 		p = heap_.p;
+		cap = LIST_HEAP;
 		return true;
 	}
 };
 
 struct ListUpload {
-	int32_t *buf;
-	int n = 0;             /* ints in the buffer */
+	int32_t *buf, *dst;
+	int cap, n = 0;        /* ints the buffer takes, and holds */
 	int64_t done = 0;
-	int32_t *dst;
 	bool ok = true;
-	ListUpload(int32_t *d, int32_t *b) : buf(b), dst(d) {}
+	ListUpload(int32_t *d, const ListBuf &b) : buf(b.p), dst(d), cap(b.cap) {}
 	void put(int a)
 	{
 		buf[n] = a;
-		if (++n == 3 * LIST_CHUNK)
+		if (++n == cap)
 			flush();
 	}
 	void put(int a, int b, int c)
@@ -504,6 +546,8 @@ struct ListUpload {
 		n = 0;
 		return ok;
 	}
+	/* ints put so far */
+	int64_t at() const { return done + n; }
 };
 
 /* Tiles in blocks of GA x GB x GC (A, B, C): the workgroups that run at the
@@ -547,7 +591,7 @@ case_set_block(const libpt_amd_plan *pl, Case &c, const TileBlock &tb)
 		set_err("tile order changed the tile count");
 		return false;
 	}
-	ListUpload up(c.d_tiles, lb.p);
+	ListUpload up(c.d_tiles, lb);
 	(void)tile_order(c, tb, [&](int a, int b, int x) { up.put(a, b, x); });
 	if (!up.flush())
 		return false;
@@ -555,31 +599,26 @@ case_set_block(const libpt_amd_plan *pl, Case &c, const TileBlock &tb)
 	return true;
 }
 
-/* tile list of one spin case for c tiles of width tcw, and its item
- * energy slots (n_ijk x tiles, cleared).  A >= B; for the same-spin case
- * (a > b > c) only c tiles that reach below the top of the B block. */
-bool
-case_tiles(libpt_amd_plan *pl, Case &c, int64_t nc, int tcw)
+/* tile geometry of one spin case for c tiles of width tcw.  A >= B; for the
+ * same-spin case (a > b > c) only c tiles that reach below the top of the B
+ * block. */
+void
+case_count(Case &c, int64_t nc, int tcw)
 {
 	c.nC = (int)((nc + tcw - 1) / tcw);
 	c.tcw = tcw;
-	int nt = 0;
-	(void)tile_order(c, c.block, [&](int, int, int) { ++nt; });
-	c.n_tiles = nt;
-	if (!plan_alloc(pl, (void **)&c.d_tiles, 3 * sizeof(int32_t) *
-	    (size_t)nt) ||
-	    !plan_alloc(pl, (void **)&c.d_partial,
-	    sizeof(double) * (size_t)(c.n_ijk * nt)))
+	c.n_tiles = tile_order(c, c.block, [](int, int, int) {});
+}
+
+/* the item energy slots of a spin case (n_ijk x tiles), cleared */
+bool
+case_partial(libpt_amd_plan *pl, Case &c)
+{
+	const size_t bytes = sizeof(double) * (size_t)(c.n_ijk * c.n_tiles);
+	if (!plan_alloc(pl, (void **)&c.d_partial, bytes))
 		return false;
-	ListBuf lb;
-	if (!lb.get(pl))
-		return false;
-	ListUpload ut(c.d_tiles, lb.p);
-	(void)tile_order(c, c.block, [&](int a, int b, int x) { ut.put(a, b, x); });
-	if (!ut.flush())
-		return false;
-	HCHK(hipMemset(c.d_partial, 0, sizeof(double) * (size_t)(c.n_ijk * nt)),
-	    false);
+	HCHK(hipMemset(c.d_partial, 0, bytes), false);
+	c.L.partial = c.d_partial;
 	return true;
 }
 
@@ -628,41 +667,9 @@ pt_ijk_order(int same, int o1, int o2, Emit emit)
 		}
 }
 
-/* work list of one spin case: ijk items x (A, B, C) tiles */
-bool
-case_lists(libpt_amd_plan *pl, Case &c, int same, int64_t o1, int64_t o2,
-    int64_t na, int64_t nc, int tcw)
-{
-	int64_t nijk = same ? o1 * (o1 - 1) * (o1 - 2) / 6 : o1 * (o1 - 1) / 2 * o2;
-	c.same = same;
-	c.nA = (int)((na + PT_TA - 1) / PT_TA);
-	c.n_ijk = nijk;
-	if (!plan_alloc(pl, (void **)&c.d_ijk, 3 * sizeof(int32_t) *
-	    (size_t)nijk))
-		return false;
-	ListBuf lb;
-	if (!lb.get(pl))
-		return false;
-	ListUpload ui(c.d_ijk, lb.p);
-	for (int64_t i = 0; i < o1; ++i)
-		for (int64_t j = i + 1; j < o1; ++j)
-			for (int64_t k = same ? j + 1 : 0; k < (same ? o1 : o2); ++k)
-				ui.put((int)i, (int)j, (int)k);
-	if (!ui.flush())
-		return false;
-	/* the launch order, and room for that of a range (pt_ijk_order) */
-	if (!plan_alloc(pl, (void **)&c.d_perm, sizeof(int32_t) * (size_t)nijk) ||
-	    !plan_alloc(pl, (void **)&c.d_part, sizeof(int32_t) * (size_t)nijk))
-		return false;
-	ListUpload up(c.d_perm, lb.p);
-	pt_ijk_order(same, (int)o1, (int)o2, [&](int64_t n) { up.put((int)n); });
-	if (!up.flush())
-		return false;
-	return case_tiles(pl, c, nc, tcw);
-}
-
-bool
-case_finish(libpt_amd_plan *pl, Case &c, int form, int kind, int nset,
+/* the host side of one spin case: terms, counts and launch parameters */
+void
+case_setup(const libpt_amd_plan *pl, Case &c, int form, int kind, int nset,
     int64_t oa, int64_t va, int64_t ob, int64_t vb)
 {
 	pt_launch &L = c.L;
@@ -687,22 +694,73 @@ case_finish(libpt_amd_plan *pl, Case &c, int form, int kind, int nset,
 	}
 	L.nterm1 = pt_terms_order(c.terms, &L.nterm_a);
 	L.nterm2 = (int32_t)c.terms.size() / nset - L.nterm1;
-	if (!plan_alloc(pl, (void **)&c.d_terms, sizeof(pt_term) *
-	    (size_t)c.terms.size()))
-		return false;
-	HCHK(hipMemcpy(c.d_terms, c.terms.data(),
-	    sizeof(pt_term) * (size_t)c.terms.size(), hipMemcpyHostToDevice),
-	    false);
-	L.terms = c.d_terms;
-	if (!case_lists(pl, c, kind == PT_AAA, oa, ob, va, vb, L.tcw))
-		return false;
-	L.ijk = c.d_ijk;
-	L.tiles = c.d_tiles;
+	c.same = kind == PT_AAA;
+	c.nA = (int)((va + PT_TA - 1) / PT_TA);
+	c.n_ijk = c.same ? oa * (oa - 1) * (oa - 2) / 6 : oa * (oa - 1) / 2 * ob;
+	case_count(c, vb, L.tcw);
 	L.n_tiles = c.n_tiles;
-	L.partial = c.d_partial;
 	c.flop_per_ijk = (kind == PT_AAA ? flop_same((double)oa, (double)va) :
 	    flop_mixed((double)oa, (double)va, (double)ob, (double)vb)) * nset;
-	return true;
+}
+
+/* the device lists of every spin case, in one buffer and one stream of
+ * copies: term table, ijk triples, launch order (pt_ijk_order), (A, B, C)
+ * tiles; then room for the launch order of a range, and the energy slots */
+bool
+plan_lists(libpt_amd_plan *pl)
+{
+	constexpr int TI = (int)(sizeof(pt_term) / sizeof(int32_t));
+	int64_t ints = 0, part = 0;
+	for (const Case &c : pl->cases)
+		if (c.n_ijk > 0) {
+			/* term tables start at multiples of 16 bytes */
+			ints = (ints + 3) / 4 * 4 + (int64_t)TI * c.terms.size() +
+			    4 * c.n_ijk + 3 * c.n_tiles;
+			part += c.n_ijk;
+		}
+	if (ints == 0)
+		return true;
+	int32_t *d;
+	if (!plan_alloc(pl, (void **)&d, sizeof(int32_t) * (size_t)(ints + part)))
+		return false;
+	ListBuf lb;
+	if (!lb.get(pl))
+		return false;
+	ListUpload up(d, lb);
+	int32_t *dp = d + ints;
+	for (Case &c : pl->cases) {
+		if (c.n_ijk == 0)
+			continue;
+		while (up.at() % 4)
+			up.put(0);
+		c.d_terms = (pt_term *)(d + up.at());
+		for (const pt_term &t : c.terms) {
+			int32_t w[TI];
+			memcpy(w, &t, sizeof(t));
+			for (int n = 0; n < TI; ++n)
+				up.put(w[n]);
+		}
+		const int o1 = (int)c.L.oa, o2 = (int)c.L.ob;
+		c.d_ijk = d + up.at();
+		for (int i = 0; i < o1; ++i)
+			for (int j = i + 1; j < o1; ++j)
+				for (int k = c.same ? j + 1 : 0; k < (c.same ? o1 : o2); ++k)
+					up.put(i, j, k);
+		c.d_perm = d + up.at();
+		pt_ijk_order(c.same, o1, o2, [&](int64_t n) { up.put((int)n); });
+		c.d_tiles = d + up.at();
+		(void)tile_order(c, c.block, [&](int a, int b, int x) {
+			up.put(a, b, x);
+		});
+		c.d_part = dp;
+		dp += c.n_ijk;
+		c.L.terms = c.d_terms;
+		c.L.ijk = c.d_ijk;
+		c.L.tiles = c.d_tiles;
+		if (!case_partial(pl, c))
+			return false;
+	}
+	return up.flush();
 }
 
 /* power-of-two scale bringing max |x| of a family to about 2^14 */
@@ -792,11 +850,13 @@ plan_set_geometry(libpt_amd_plan *pl, int nw)
 		L.nw = nw;
 		L.tcw = pt_tcw(pl->form, L.nset, nw);
 		L.pgrid = persist_grid(nw);
-		if (!case_tiles(pl, c, L.nc, L.tcw))
+		case_count(c, L.nc, L.tcw);
+		if (!plan_alloc(pl, (void **)&c.d_tiles, 3 * sizeof(int32_t) *
+		    (size_t)c.n_tiles) || !case_partial(pl, c) ||
+		    !case_set_block(pl, c, c.block))
 			return false;
 		L.tiles = c.d_tiles;
 		L.n_tiles = c.n_tiles;
-		L.partial = c.d_partial;
 	}
 	if (had_wsave && !plan_wsave(pl))
 		return false;
@@ -859,8 +919,8 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 			return false; \
 	} while (0)
 	if (pl->own_stream) {
-		PFAIL(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking) ==
-		    hipSuccess || (set_err("hipStreamCreate failed"), false));
+		PFAIL(stream_get(&pl->stream) ||
+		    (set_err("hipStreamCreate failed"), false));
 		PFAIL((hipEventCreate(&pl->ev0) == hipSuccess &&
 		    hipEventCreate(&pl->ev1) == hipSuccess) ||
 		    (set_err("hipEventCreate failed"), false));
@@ -893,7 +953,9 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		famT[1] = 3; famO[1] = 6; famV[1] = 7;
 	}
 	const int nblk = restricted ? 2 : 4;
-	const double t_prep = now_s();
+	if (pl->own_stream)
+		PFAIL(hipEventRecord(pl->ev0, pl->stream) == hipSuccess ||
+		    (set_err("hipEventRecord failed"), false));
 
 	/* block geometry [R slabs][K kappa][plane rows x cols, or the pairs
 	 * row > column] and element offsets, src/pt.c:460-467 (restricted) and
@@ -972,6 +1034,7 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 	    case_mixed(ob, vb, oa, va);
 	const bool used[4] = {sa || mx, mx, sb || mx, mx};
 	const bool used_t[4] = {sa, mx, sb, mx};   /* transposed */
+	FixedVec<pt_pack_job, 28> jobs;
 	auto pack = [&](int s, int fam, int b, bool tr, const char **out) {
 		const Geo g = geo(fam, b);
 		const int64_t rows = tr ? g.cols : g.rows;
@@ -981,12 +1044,17 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		if (!plan_alloc(pl, &dst, (size_t)(g.R * pt_slab_frags(form, g.K,
 		    rows, cols, g.tri)) * PT_FRAG))
 			return false;
-		const char *src = (const char *)arr[api] + esz * (size_t)g.off;
-		if (pt_launch_pack(src, dst, g.R, g.K, rows, cols, g.tri, tr, form,
-		    pl->scale[2 * s + fam], pl->stream) != 0) {
-			set_err("pack launch failed");
-			return false;
-		}
+		pt_pack_job j = {};
+		j.src = (const char *)arr[api] + esz * (size_t)g.off;
+		j.dst = (char *)dst;
+		j.R = g.R;
+		j.K = g.K;
+		j.rows = rows;
+		j.cols = cols;
+		j.tri = g.tri;
+		j.tr = tr;
+		j.scale = pl->scale[2 * s + fam];
+		jobs.push_back(j);
 		*out = (const char *)dst;
 		return true;
 	};
@@ -1009,9 +1077,12 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 			}
 		}
 	}
-	PFAIL(hipStreamSynchronize(pl->stream) == hipSuccess ||
-	    (set_err("operand preparation failed"), false));
-	pl->prep_s = now_s() - t_prep;
+	if (!jobs.empty())
+		PFAIL(pt_launch_pack(jobs.data(), jobs.size(), form, pl->stream) ==
+		    0 || (set_err("pack launch failed"), false));
+	if (pl->own_stream)
+		PFAIL(hipEventRecord(pl->ev1, pl->stream) == hipSuccess ||
+		    (set_err("hipEventRecord failed"), false));
 
 	/* block pointers (element offsets as in src/pt.c:460-467, 487-512) */
 	auto blk4 = [&](const void *base, int fam, size_t el) {
@@ -1120,26 +1191,29 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		e.ZA = zt.p[same];
 		e.ZB = zt.p[mixB];
 		c.factor = fac;
-		bool empty;
 		if (cs.kind == PT_AAA) {
-			empty = !case_same(o1, v1);
-			if (!empty)
-				PFAIL(case_finish(pl, c, form, PT_AAA, nset, o1, v1, o1,
-				    v1));
+			if (case_same(o1, v1))
+				case_setup(pl, c, form, PT_AAA, nset, o1, v1, o1, v1);
 		} else {
-			empty = !case_mixed(o1, v1, o2, v2);
-			if (!empty)
-				PFAIL(case_finish(pl, c, form, PT_AAB, nset, o1, v1, o2,
-				    v2));
+			if (case_mixed(o1, v1, o2, v2))
+				case_setup(pl, c, form, PT_AAB, nset, o1, v1, o2, v2);
 		}
 		pl->cases.push_back(c);
 	}
+	/* built and copied while the operands are packed */
+	PFAIL(plan_lists(pl));
 	if (ft && own_wsave)
 		PFAIL(plan_wsave(pl));
 	/* list uploads and slot clears ran on the null stream; the plan's
 	 * stream does not wait for it */
 	PFAIL(hipDeviceSynchronize() == hipSuccess ||
-	    (set_err("hipDeviceSynchronize failed"), false));
+	    (set_err("operand preparation failed"), false));
+	if (pl->own_stream) {
+		float ms = 0;
+		PFAIL(hipEventElapsedTime(&ms, pl->ev0, pl->ev1) == hipSuccess ||
+		    (set_err("operand preparation failed"), false));
+		pl->prep_s = 1e-3 * ms;
+	}
 #undef PFAIL
 	return true;
 }
@@ -1322,21 +1396,25 @@ libpt_amd_plan_energy(libpt_amd_plan *pl)
 		return NAN;
 	if (!pl)
 		return NAN;
-	double e = 0.0;
-	for (Case &c : pl->cases) {
-		if (c.n_ijk == 0)
-			continue;
-		if (pt_launch_reduce(c.d_partial, c.n_ijk * c.n_tiles, pl->d_out,
-		    pl->stream) != 0) {
-			set_err("reduce launch failed");
-			return NAN;
-		}
-		double x = 0;
-		HCHK(hipMemcpyAsync(&x, pl->d_out, sizeof(double),
-		    hipMemcpyDeviceToHost, pl->stream), NAN);
-		HCHK(hipStreamSynchronize(pl->stream), NAN);
-		e += c.factor * x;
+	const double *x[4] = {nullptr};
+	int64_t n[4] = {0};
+	const int nc = (int)pl->cases.size();
+	for (int sc = 0; sc < nc; ++sc) {
+		x[sc] = pl->cases[sc].d_partial;
+		n[sc] = pl->cases[sc].n_ijk * pl->cases[sc].n_tiles;
 	}
+	if (pt_launch_reduce(x, n, nc, pl->d_out, pl->stream) != 0) {
+		set_err("reduce launch failed");
+		return NAN;
+	}
+	double sum[4] = {0};
+	HCHK(hipMemcpyAsync(sum, pl->d_out, sizeof(double) * (size_t)nc,
+	    hipMemcpyDeviceToHost, pl->stream), NAN);
+	HCHK(hipStreamSynchronize(pl->stream), NAN);
+	double e = 0.0;
+	for (int sc = 0; sc < nc; ++sc)
+		if (n[sc] > 0)
+			e += pl->cases[sc].factor * sum[sc];
 	return e;
 }
 
@@ -2077,15 +2155,24 @@ pt_noalloc_energy(int call, int form, size_t oa, size_t va, size_t ob,
 namespace {
 
 /*
- * Host-to-device copy of the caller's pageable arrays.  Small inputs go
- * with hipMemcpy.  Large ones are cut into chunks of H2D_CHUNK bytes that
- * H2D_WORKERS host threads take in turn: a worker copies its chunk into
- * one of its two pinned buffers and hands it to its own stream, so that
- * the host copies of several threads and the PCIe transfers overlap.
+ * Host-to-device copy of the caller's pageable arrays.  The smallest inputs
+ * are put together in one buffer and one copy (a copy costs 14 us whatever
+ * its size, seven of them 115 us against 53 us for 0.7 MB), small ones go
+ * with hipMemcpy.  Large ones are cut into chunks of H2D_CHUNK bytes that up
+ * to H2D_WORKERS host threads, one per H2D_PER_WORKER bytes, take in turn: a
+ * worker copies its chunk into one of its two pinned buffers and hands it to
+ * its own stream, so that the host copies of several threads and the PCIe
+ * transfers overlap.  Chunks are small because every byte of pinned memory
+ * is allocated in the call: 613 MB took 52 ms with 16 buffers of 32 MB, most
+ * of it the buffers, and takes 20 to 24 ms with 4 MB.  253 MB take 9.4 ms with
+ * hipMemcpy and 12.5 ms this way, with another 4 ms until the GPU runs on.
  */
 enum { H2D_WORKERS = 8 };
-constexpr size_t H2D_CHUNK = (size_t)32 << 20;
-constexpr size_t H2D_PINNED_FROM = (size_t)256 << 20;
+constexpr size_t H2D_CHUNK = (size_t)4 << 20;
+constexpr size_t H2D_PER_WORKER = (size_t)32 << 20;
+constexpr size_t H2D_PINNED_FROM = (size_t)512 << 20;
+constexpr size_t H2D_ONE_COPY = (size_t)1 << 20;
+constexpr size_t H2D_ONE_ALLOC = (size_t)256 << 20;
 
 bool
 h2d_copy(void *const *dst, const void *const *src, const size_t *bytes,
@@ -2107,8 +2194,8 @@ h2d_copy(void *const *dst, const void *const *src, const size_t *bytes,
 		for (size_t o = 0; o < bytes[q]; o += H2D_CHUNK)
 			chunks.push_back({q, o});
 	const unsigned hw = std::thread::hardware_concurrency();
-	const int nw = (int)std::max(1u, std::min<unsigned>(H2D_WORKERS,
-	    hw > 2 ? hw / 2 : 1));
+	const int nw = (int)std::min<size_t>(total / H2D_PER_WORKER,
+	    std::max(1u, std::min<unsigned>(H2D_WORKERS, hw > 2 ? hw / 2 : 1)));
 	std::atomic<size_t> next(0);
 	std::atomic<bool> failed(false);
 	int dev = 0;
@@ -2205,13 +2292,32 @@ host_call(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 	libpt_amd_plan *pl = nullptr;
 	double t1 = 0, t2 = 0;
 	bool ok = true;
-	size_t nbytes[10];
-	for (int q = 0; q < narr && ok; ++q) {
+	size_t nbytes[10], ofs[10], total = 0;
+	for (int q = 0; q < narr; ++q) {
 		nbytes[q] = el * (size_t)n[q];
-		ok = dev_alloc(&d[q], nbytes[q]);
+		ofs[q] = total;
+		total += (nbytes[q] + 255) & ~(size_t)255;
 	}
-	if (ok)
+	/* inputs of moderate size share one buffer, d[0] */
+	const bool one = total <= H2D_ONE_ALLOC;
+	ok = !one || dev_alloc(&d[0], total);
+	for (int q = 0; q < narr && ok; ++q) {
+		if (one)
+			d[q] = (char *)d[0] + ofs[q];
+		else
+			ok = dev_alloc(&d[q], nbytes[q]);
+	}
+	if (ok && total <= H2D_ONE_COPY) {
+		HostBuf<char> h;
+		ok = h.alloc(total);
+		for (int q = 0; q < narr && ok; ++q)
+			if (nbytes[q] > 0)
+				memcpy(h.p + ofs[q], arrays[q], nbytes[q]);
+		if (ok && total > 0)
+			ok = h2d_copy(&d[0], (const void *const *)&h.p, &total, 1);
+	} else if (ok) {
 		ok = h2d_copy(d, arrays, nbytes, narr);
+	}
 	t1 = now_s();
 	if (ok)
 		pl = libpt_amd_plan_create(call, form, oa, va, ob, vb, d);
@@ -2252,7 +2358,7 @@ host_call(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 		}
 	}
 	plan_free(pl);
-	for (int q = 0; q < narr; ++q)
+	for (int q = 0; q < (one ? 1 : narr); ++q)
 		(void)hipFree(d[q]);
 	if (st)
 		st->wall_s = now_s() - t0;

@@ -41,11 +41,16 @@ reduce_block(const double *x, int64_t n, double *out)
 		out[0] = sh[0];
 }
 
-/* one workgroup, fixed-order compensated sum of x[0..n) */
+/* up to four sums, one workgroup each: fixed-order compensated */
+struct reduce_args {
+	const double *x[4];
+	int64_t n[4];
+};
+
 __global__ __launch_bounds__(1024) void
-k_reduce(const double *x, int64_t n, double *out)
+k_reduce(reduce_args a, double *out)
 {
-	reduce_block(x, n, out);
+	reduce_block(a.x[blockIdx.x], a.n[blockIdx.x], out + blockIdx.x);
 }
 
 /* one workgroup per segment: out[s] = the k_reduce sum of its partials */
@@ -86,19 +91,32 @@ split2(double x, int fp16, uint16_t &hb, uint16_t &lb)
 }
 
 /*
- * Operand packing (pt_slab_frags): one workgroup makes the fragments of one
- * (slab, row block, kappa chunk) for PACK_COLS columns.  It reads the
- * plane along its contiguous index (columns, or rows with TR), lays the
- * fragments out in LDS and writes them as whole 1 KB runs; rows and kappa
- * beyond the extents, and tri pairs with column >= row, are zero.  Bound
- * by HBM (each element read once and written once).
+ * Operand packing (pt_slab_frags): one launch for all operands of a plan;
+ * one workgroup makes the fragments of one (slab, row block, kappa chunk) of
+ * a job for PACK_COLS columns.  It reads the plane along its contiguous index
+ * (columns, or rows with tr), PACK_BATCH loads at a time, lays the fragments
+ * out in LDS and writes them as whole 1 KB runs; rows and kappa beyond the
+ * extents, and tri pairs with column >= row, are zero.  Bound by HBM (each
+ * element read once and written once) or, in small plans, by the launch and
+ * one load latency per batch.
  */
-constexpr int PACK_COLS = 32;
+constexpr int PACK_COLS = 32, PACK_BATCH = 8, PACK_JOBS = 28;
+
+struct pack_args {
+	pt_pack_job job[PACK_JOBS];
+	int n;
+};
+
+__device__ __forceinline__ int64_t
+pack_groups(const pt_pack_job &j)
+{
+	return ((j.tri ? (j.rows + 15) / 16 * 16 : j.cols) + PACK_COLS - 1) /
+	    PACK_COLS;
+}
 
 template <int F>
 __global__ __launch_bounds__(256) void
-k_pack(const void *src, char *dst, int64_t K, int64_t rows, int64_t cols,
-    int tri, int tr, double scale, int64_t nch, int64_t nrb, int64_t ncg)
+k_pack(pack_args args)
 {
 	constexpr bool SPLIT = F == PT_FORM_BF16X3 || F == PT_FORM_F16X3;
 	constexpr int KC = F == PT_FORM_FP64 ? 8 : 16;
@@ -108,52 +126,72 @@ k_pack(const void *src, char *dst, int64_t K, int64_t rows, int64_t cols,
 	 * consecutive pairs of banks */
 	constexpr int FS = PT_FRAG + 8;
 	__shared__ __attribute__((aligned(16))) char lds[PACK_COLS * FS];
-	const int64_t bid = blockIdx.x;
-	const int64_t cg = bid % ncg, ch = bid / ncg % nch;
-	const int64_t rb = bid / (ncg * nch) % nrb, r = bid / (ncg * nch * nrb);
-	const int64_t c0 = cg * PACK_COLS, bcols = tri ? 16 * (rb + 1) : cols;
+	int q = 0;
+	while (q + 1 < args.n && (int64_t)blockIdx.x >= args.job[q + 1].at)
+		++q;
+	const pt_pack_job &J = args.job[q];
+	const int64_t K = J.K, rows = J.rows, cols = J.cols;
+	const bool tri = J.tri, tr = J.tr;
+	const int64_t nch = (K + KC - 1) / KC, nrb = (rows + 15) / 16;
+	const int64_t ncg = pack_groups(J);
+	const uint32_t bid = (uint32_t)(blockIdx.x - J.at);
+	const uint32_t cg = bid % (uint32_t)ncg, b1 = bid / (uint32_t)ncg;
+	const uint32_t ch = b1 % (uint32_t)nch, b2 = b1 / (uint32_t)nch;
+	const uint32_t rb = b2 % (uint32_t)nrb, r = b2 / (uint32_t)nrb;
+	const int64_t c0 = (int64_t)cg * PACK_COLS;
+	const int64_t bcols = tri ? 16 * ((int64_t)rb + 1) : cols;
 	if (c0 >= bcols)
 		return;
 	const int64_t pl = tri ? rows * (rows - 1) / 2 : rows * cols;
-	const T *sp = (const T *)src + (r * K + ch * KC) * pl;
-	for (int n = threadIdx.x; n < 16 * KC * PACK_COLS; n += 256) {
-		int row, kk, col;
-		if (tr) {
-			row = n % 16;
-			col = n / 16 % PACK_COLS;
-			kk = n / (16 * PACK_COLS);
-		} else {
-			col = n % PACK_COLS;
-			row = n / PACK_COLS % 16;
-			kk = n / (16 * PACK_COLS);
+	const T *sp = (const T *)J.src + ((int64_t)r * K + (int64_t)ch * KC) * pl;
+	const int tid = threadIdx.x;
+	/* element n = tid + 256 it of the group: column (or, tr, row) fastest */
+	auto place = [&](int n, int &row, int &col, int &kk) {
+		row = tr ? n % 16 : n / PACK_COLS % 16;
+		col = tr ? n / 16 % PACK_COLS : n % PACK_COLS;
+		kk = n / (16 * PACK_COLS);
+	};
+	static_assert(16 * KC * PACK_COLS % (256 * PACK_BATCH) == 0, "batches");
+	for (int n0 = tid; n0 < 16 * KC * PACK_COLS; n0 += 256 * PACK_BATCH) {
+		T x[PACK_BATCH];
+#pragma unroll
+		for (int b = 0; b < PACK_BATCH; ++b) {
+			int row, col, kk;
+			place(n0 + 256 * b, row, col, kk);
+			const int64_t u = 16 * (int64_t)rb + row, w = c0 + col;
+			x[b] = 0;
+			if ((int64_t)ch * KC + kk < K && u < rows &&
+			    (tri ? w < u : w < cols))
+				x[b] = sp[kk * pl + (tri ? u * (u - 1) / 2 + w : tr ?
+				    w * rows + u : u * cols + w)];
 		}
-		const int64_t u = 16 * rb + row, w = c0 + col;
-		T x = 0;
-		if (ch * KC + kk < K && u < rows && (tri ? w < u : w < cols))
-			x = sp[kk * pl + (tri ? u * (u - 1) / 2 + w : tr ?
-			    w * rows + u : u * cols + w)];
-		constexpr int KQ = KC / 4;
-		const int e = kk % KQ;
-		char *d = lds + col * FS + 16 * (16 * (kk / KQ) + row);
-		if constexpr (SPLIT) {
-			uint16_t hb, lb;
-			split2(x * scale, F == PT_FORM_F16X3, hb, lb);
-			*(uint16_t *)(d + 2 * e) = hb;
-			*(uint16_t *)(d + 8 + 2 * e) = lb;
-		} else {
-			*(T *)(d + e * sizeof(T)) = x;
+#pragma unroll
+		for (int b = 0; b < PACK_BATCH; ++b) {
+			int row, col, kk;
+			place(n0 + 256 * b, row, col, kk);
+			constexpr int KQ = KC / 4;
+			const int e = kk % KQ;
+			char *d = lds + col * FS + 16 * (16 * (kk / KQ) + row);
+			if constexpr (SPLIT) {
+				uint16_t hb, lb;
+				split2(x[b] * J.scale, F == PT_FORM_F16X3, hb, lb);
+				*(uint16_t *)(d + 2 * e) = hb;
+				*(uint16_t *)(d + 8 + 2 * e) = lb;
+			} else {
+				*(T *)(d + e * sizeof(T)) = x[b];
+			}
 		}
 	}
 	__syncthreads();
 	const int64_t f0 = tri ? nch * (r * 8 * nrb * (nrb + 1) +
-	    8 * rb * (rb + 1)) + ch * bcols + c0 :
+	    8 * (int64_t)rb * (rb + 1)) + ch * bcols + c0 :
 	    ((r * nrb + rb) * nch + ch) * cols + c0;
-	for (int n = threadIdx.x; n < 64 * PACK_COLS; n += 256) {
+	for (int n = tid; n < 64 * PACK_COLS; n += 256) {
 		const int col = n / 64, l = n % 64;
 		if (c0 + col >= bcols)
 			break;
 		const uint64_t *s8 = (const uint64_t *)(lds + col * FS + 16 * l);
-		uint64_t *d8 = (uint64_t *)(dst + (f0 + col) * PT_FRAG + 16 * l);
+		uint64_t *d8 = (uint64_t *)(J.dst + (f0 + col) * PT_FRAG + 16 * l);
 		d8[0] = s8[0];
 		d8[1] = s8[1];
 	}
@@ -281,9 +319,19 @@ pt_launch_reduce_batch(const struct pt_launch *segs, const int64_t *begin,
 }
 
 extern "C" int
-pt_launch_reduce(const double *x, int64_t n, double *out, void *stream)
+pt_launch_reduce(const double *const *x, const int64_t *n, int cnt,
+    double *out, void *stream)
 {
-	k_reduce<<<1, 1024, 0, (hipStream_t)stream>>>(x, n, out);
+	if (cnt <= 0)
+		return 0;
+	if (cnt > 4)
+		return (int)hipErrorInvalidValue;
+	reduce_args a = {};
+	for (int q = 0; q < cnt; ++q) {
+		a.x[q] = x[q];
+		a.n[q] = n[q];
+	}
+	k_reduce<<<cnt, 1024, 0, (hipStream_t)stream>>>(a, out);
 	return (int)hipGetLastError();
 }
 
@@ -311,40 +359,64 @@ pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
 }
 
 extern "C" int
-pt_launch_pack(const void *src, void *dst, int64_t R, int64_t K, int64_t rows,
-    int64_t cols, int tri, int tr, int form, double scale, void *stream)
+pt_launch_pack(const struct pt_pack_job *jobs, int n, int form, void *stream)
 {
-	const int64_t nch = pt_chunks(form, K), nrb = (rows + 15) / 16;
-	const int64_t ncg = ((tri ? 16 * nrb : cols) + PACK_COLS - 1) / PACK_COLS;
-	if (R <= 0 || nch <= 0 || nrb <= 0 || ncg <= 0)
-		return 0;
-	/* at most 2^30 workgroups per launch, in whole slabs */
-	const int64_t per = nch * nrb * ncg;
-	const int64_t step = per < ((int64_t)1 << 30) ? ((int64_t)1 << 30) / per : 1;
-	const int64_t pl = tri ? rows * (rows - 1) / 2 : rows * cols;
-	const int64_t slab = pt_slab_frags(form, K, rows, cols, tri) * PT_FRAG;
+	const hipStream_t st = (hipStream_t)stream;
 	const int el = form == PT_FORM_FP32 ? 4 : 8;
-	for (int64_t r = 0; r < R; r += step) {
-		const dim3 grid((unsigned)(per * (step < R - r ? step : R - r)));
-		const void *sp = (const char *)src + r * K * pl * el;
-		char *dp = (char *)dst + r * slab;
-		const hipStream_t st = (hipStream_t)stream;
-#define PACK(F) k_pack<F><<<grid, 256, 0, st>>>(sp, dp, K, rows, cols, tri, \
-    tr, scale, nch, nrb, ncg)
+	/* a launch takes up to PACK_JOBS jobs and 2^30 workgroups; a job of more
+	 * goes in runs of whole slabs */
+	constexpr int64_t MOST = (int64_t)1 << 30;
+	pack_args a;
+	a.n = 0;
+	int64_t blocks = 0;
+	auto go = [&]() {
+		if (a.n == 0)
+			return 0;
+		const dim3 grid((unsigned)blocks);
 		if (form == PT_FORM_FP64)
-			PACK(PT_FORM_FP64);
+			k_pack<PT_FORM_FP64><<<grid, 256, 0, st>>>(a);
 		else if (form == PT_FORM_FP32)
-			PACK(PT_FORM_FP32);
+			k_pack<PT_FORM_FP32><<<grid, 256, 0, st>>>(a);
 		else if (form == PT_FORM_BF16X3)
-			PACK(PT_FORM_BF16X3);
+			k_pack<PT_FORM_BF16X3><<<grid, 256, 0, st>>>(a);
 		else
-			PACK(PT_FORM_F16X3);
-#undef PACK
-		const int rc = (int)hipGetLastError();
-		if (rc != 0)
-			return rc;
+			k_pack<PT_FORM_F16X3><<<grid, 256, 0, st>>>(a);
+		a.n = 0;
+		blocks = 0;
+		return (int)hipGetLastError();
+	};
+	for (int q = 0; q < n; ++q) {
+		const pt_pack_job &j = jobs[q];
+		const int64_t nrb = (j.rows + 15) / 16;
+		const int64_t ncg = ((j.tri ? 16 * nrb : j.cols) + PACK_COLS - 1) /
+		    PACK_COLS;
+		const int64_t per = pt_chunks(form, j.K) * nrb * ncg;
+		if (j.R <= 0 || per <= 0)
+			continue;
+		if (per > MOST)
+			return (int)hipErrorInvalidValue;
+		const int64_t pl = j.tri ? j.rows * (j.rows - 1) / 2 :
+		    j.rows * j.cols;
+		const int64_t slab = pt_slab_frags(form, j.K, j.rows, j.cols, j.tri) *
+		    PT_FRAG;
+		for (int64_t r = 0; r < j.R;) {
+			if (a.n == PACK_JOBS || MOST - blocks < per) {
+				const int rc = go();
+				if (rc != 0)
+					return rc;
+			}
+			const int64_t m = (MOST - blocks) / per < j.R - r ?
+			    (MOST - blocks) / per : j.R - r;
+			pt_pack_job &o = a.job[a.n++];
+			o = j;
+			o.src = j.src + r * j.K * pl * el;
+			o.dst = j.dst + r * slab;
+			o.at = blocks;
+			blocks += per * m;
+			r += m;
+		}
 	}
-	return 0;
+	return go();
 }
 
 extern "C" int
