@@ -34,6 +34,7 @@ enum pt_role { PT_ROLE_A = 0, PT_ROLE_B = 1, PT_ROLE_C = 2 };
 
 #define PT_MAX_TERMS 40
 #define PT_MAX_BUFS 26
+#define PT_MAX_SEGS 4    /* spin cases (segments) of one tile launch */
 
 /* kappa per fragment of the packed Q operands: a fragment is 1 KB, 16 rows
  * of 64 bytes (8 FP64, 16 FP32, or 16 split values: per 4 kappa hi 0-3 and
@@ -149,9 +150,9 @@ struct pt_launch {
 	double inv_scale[2];         /* per W set: 1 / (operand scale product) */
 	void *wsave;                 /* two W sets: W of set 0 of each item
 	                                of the launch (pt_wsave_bytes each,
-	                                position pos0 + n at slot n), else
-	                                unused */
-	int32_t nwsave;              /* save areas in wsave (>= n_chunk) */
+	                                position pos0 + n at slot wslot0 +
+	                                n), else unused */
+	int32_t nwsave, wslot0;      /* save areas in wsave */
 	int32_t kgrp;                /* > 1: the run's ijk are taken in groups
 	                                of kgrp, each group's items
 	                                tile-major; 1: items in order */
@@ -188,11 +189,14 @@ pt_ft_chunk(int form, int nw)
 }
 
 /* kernel launchers (pt_tiles_*.hip, pt_kernel.hip); return hipError_t as int */
-int pt_launch_tiles(int form, const struct pt_launch *p, void *stream);
-int pt_launch_tiles_fp64(const struct pt_launch *p, void *stream);
-int pt_launch_tiles_fp32(const struct pt_launch *p, void *stream);
-int pt_launch_tiles_bf16x3(const struct pt_launch *p, void *stream);
-int pt_launch_tiles_f16x3(const struct pt_launch *p, void *stream);
+/* n <= PT_MAX_SEGS segments (n_chunk > 0) of one geometry and W-set count in
+ * one launch, in order; a persistent grid takes one */
+int pt_launch_tiles(int form, const struct pt_launch *p, int n,
+    void *stream);
+int pt_launch_tiles_fp64(const struct pt_launch *p, int n, void *stream);
+int pt_launch_tiles_fp32(const struct pt_launch *p, int n, void *stream);
+int pt_launch_tiles_bf16x3(const struct pt_launch *p, int n, void *stream);
+int pt_launch_tiles_f16x3(const struct pt_launch *p, int n, void *stream);
 /* out[s] = fixed-order sum of segment s's partials (as pt_launch_reduce) */
 int pt_launch_reduce_batch(const struct pt_launch *segs,
     const int64_t *begin, int nseg, double *out, void *stream);

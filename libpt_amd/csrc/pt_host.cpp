@@ -787,16 +787,17 @@ family_scale(libpt_amd_plan *pl, const double *const *arr, const int64_t *n,
 
 namespace {
 
-/* two W sets: the save areas of one launch's items, sized to the largest
- * spin case (at most pt_ft_chunk); no-op when present */
+/* two W sets: the save areas of one launch's items, sized to all spin
+ * cases (at most pt_ft_chunk); no-op when present */
 bool
 plan_wsave(libpt_amd_plan *pl)
 {
 	if (pl->wsave)
 		return true;
-	int64_t most = 1;
+	int64_t most = 0;
 	for (const Case &d : pl->cases)
-		most = std::max(most, d.n_ijk * d.n_tiles);
+		most += d.n_ijk * d.n_tiles;
+	most = std::max<int64_t>(most, 1);
 	int64_t slots = std::min<int64_t>(pt_ft_chunk(pl->form, pl->nw), most);
 	const int64_t wb = pt_wsave_bytes(pl->form, 2, pl->nw);
 	if (pl->persist)
@@ -1242,32 +1243,98 @@ plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 
 namespace {
 
+/* a run of one spin case: its ijk [b, e), in the order of perm (the e - b
+ * ijk in launch order; null: list order) and base->kgrp */
+struct Run {
+	const pt_launch *base;
+	int64_t b, e;
+	const int32_t *perm;
+	int64_t items() const { return (e - b) * base->n_tiles; }
+};
+
 /*
- * The tile launches over the ijk [ijk_b, ijk_e) of one spin case: grids of
- * at most 2^22 items, and with two W sets of at most wslots (one save area
- * per item), over positions in the order of perm (the ijk_e - ijk_b ijk in
- * launch order; null: list order) and base.kgrp.
+ * The tile launches of some runs of one geometry: grids of at most 2^22
+ * items, and with two W sets of at most wslots (one save area per item).
+ * Small runs share a launch, up to PT_MAX_SEGS of them and MERGE_ITEMS items:
+ * each is a fraction of the GPU or a few rounds of it, and they run side by
+ * side or fill each other's ends (the two launches of a rpt 5/19 call took 50
+ * us each).  Larger ones gain nothing by it, and the kernel that holds both
+ * spin cases is 3 % slower per item (rpt v=477 FP64 245 -> 252 ms).
  */
+constexpr int64_t MERGE_ITEMS = 8192;
+
 int
-launch_items(int form, const pt_launch &base, int64_t ijk_b, int64_t ijk_e,
-    const int32_t *perm, void *wsave, int64_t wslots, hipStream_t st)
+launch_runs(int form, const Run *run, int n, void *wsave, int64_t wslots,
+    hipStream_t st)
 {
-	const int64_t nt = base.n_tiles, n = (ijk_e - ijk_b) * nt;
-	int64_t chunk = base.nset == 2 && !base.ctr ? wslots : (int64_t)1 << 22;
-	pt_launch L = base;
-	L.perm = base.kgrp > 1 ? perm : nullptr;
-	L.item0 = L.perm ? 0 : ijk_b * nt;
-	L.n_seq = n;
-	L.wsave = wsave;
-	L.nwsave = (int32_t)wslots;
-	for (int64_t it = 0; it < n; it += chunk) {
-		L.pos0 = it;
-		L.n_chunk = std::min(chunk, n - it);
-		const int rc = pt_launch_tiles(form, &L, st);
-		if (rc != 0)
-			return rc;
+	pt_launch L[PT_MAX_SEGS];
+	int nl = 0;
+	int64_t held = 0;      /* items in L */
+	auto go = [&]() {
+		const int rc = nl > 0 ? pt_launch_tiles(form, L, nl, st) : 0;
+		nl = 0;
+		held = 0;
+		return rc;
+	};
+	for (int q = 0; q < n; ++q) {
+		const pt_launch &base = *run[q].base;
+		const int64_t items = run[q].items();
+		const int64_t most = base.nset == 2 && !base.ctr ? wslots :
+		    (int64_t)1 << 22;
+		for (int64_t it = 0; it < items;) {
+			if (nl > 0 && (nl == PT_MAX_SEGS || base.ctr || it > 0 ||
+			    held + items > std::min(most, MERGE_ITEMS))) {
+				const int rc = go();
+				if (rc != 0)
+					return rc;
+			}
+			pt_launch &S = L[nl++];
+			S = base;
+			S.perm = base.kgrp > 1 ? run[q].perm : nullptr;
+			S.item0 = S.perm ? 0 : run[q].b * base.n_tiles;
+			S.n_seq = items;
+			S.pos0 = it;
+			S.n_chunk = std::min(most - held, items - it);
+			S.wsave = wsave;
+			S.nwsave = (int32_t)wslots;
+			S.wslot0 = (int32_t)held;
+			held += S.n_chunk;
+			it += S.n_chunk;
+			if (it < items || base.ctr) {
+				const int rc = go();
+				if (rc != 0)
+					return rc;
+			}
+		}
 	}
-	return 0;
+	return go();
+}
+
+/* every ijk of every spin case, the costliest items first */
+int
+plan_run_all(libpt_amd_plan *pl)
+{
+	Run run[4];
+	double cost[4];
+	int n = 0;
+	for (const Case &c : pl->cases) {
+		if (c.n_ijk == 0 || c.n_tiles == 0)
+			continue;
+		const double x = c.flop_per_ijk / c.n_tiles;
+		int at = n++;
+		for (; at > 0 && cost[at - 1] < x; --at) {
+			cost[at] = cost[at - 1];
+			run[at] = run[at - 1];
+		}
+		cost[at] = x;
+		run[at] = {&c.L, 0, c.n_ijk, c.d_perm};
+	}
+	const int rc = launch_runs(pl->form, run, n, pl->wsave, pl->wslots,
+	    pl->stream);
+	if (rc != 0)
+		set_err("tile kernel launch failed: %s",
+		    hipGetErrorString((hipError_t)rc));
+	return rc == 0 ? 0 : -1;
 }
 
 } /* namespace */
@@ -1367,8 +1434,9 @@ libpt_amd_plan_run(libpt_amd_plan *pl, int sc, int64_t b, int64_t e)
 		    c.d_part, pl->stream);
 		perm = c.d_part;
 	}
+	const Run run = {&c.L, b, e, perm};
 	if (rc == 0)
-		rc = launch_items(pl->form, c.L, b, e, perm, pl->wsave, pl->wslots,
+		rc = launch_runs(pl->form, &run, 1, pl->wsave, pl->wslots,
 		    pl->stream);
 	if (rc != 0) {
 		set_err("tile kernel launch failed: %s",
@@ -1762,9 +1830,7 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	for (const libpt_amd_plan *pl : b->plans)
 		wbytes = std::max(wbytes, pt_wsave_bytes(form, 2, pl->nw));
 	if (b->nset == 2 && b->total > 0) {
-		int64_t most = 1;
-		for (const Seg &g : segs)
-			most = std::max(most, g.items);
+		const int64_t most = std::max<int64_t>(1, b->total);
 		b->wslots = std::min<int64_t>(((int64_t)4 << 30) / wbytes, most);
 		/* a persistent grid keeps one area per workgroup */
 		for (const libpt_amd_plan *pl : b->plans)
@@ -1793,9 +1859,19 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	BFAIL(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) ==
 	    hipSuccess || (set_err("stream capture failed"), false));
 	int rc = 0;
-	for (int g = 0; g < nseg && rc == 0; ++g)
-		rc = launch_items(form, L[g], 0, segs[g].nijk, segs[g].perm,
-		    b->wsave, b->wslots, b->stream);
+	std::vector<Run> runs;
+	for (int g = 0; g < nseg; ++g) {
+		/* runs of one geometry and grid at a time */
+		if (g > 0 && rc == 0 && (L[g].nw != L[g - 1].nw)) {
+			rc = launch_runs(form, runs.data(), (int)runs.size(), b->wsave,
+			    b->wslots, b->stream);
+			runs.clear();
+		}
+		runs.push_back({&L[g], 0, segs[g].nijk, segs[g].perm});
+	}
+	if (rc == 0)
+		rc = launch_runs(form, runs.data(), (int)runs.size(), b->wsave,
+		    b->wslots, b->stream);
 	if (rc == 0)
 		rc = pt_launch_reduce_batch(b->d_segs, b->d_begin, nseg, b->d_out,
 		    b->stream);
@@ -2137,11 +2213,7 @@ pt_noalloc_energy(int call, int form, size_t oa, size_t va, size_t ob,
 		pl.copies = copies != 0;
 		double e = NAN;
 		if (plan_init(&pl, call, form, oa, va, ob, vb, dev_arrays, true)) {
-			bool ok = true;
-			for (int sc = 0; sc < pl.cases.size() && ok; ++sc)
-				ok = libpt_amd_plan_run(&pl, sc, 0, pl.cases[sc].n_ijk) ==
-				    0;
-			if (ok)
+			if (plan_run_all(&pl) == 0)
 				e = libpt_amd_plan_energy(&pl);
 		}
 		const bool again = copies && pl.no_room;
@@ -2326,19 +2398,19 @@ host_call(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 		/* LIBPT_AMD_PROGRESS set: each spin case in 16 parts, with a line
 		 * on stderr after each (a synchronisation per part) */
 		const bool progress = getenv("LIBPT_AMD_PROGRESS") != nullptr;
-		const int64_t parts = progress ? 16 : 1;
-		for (int sc = 0; sc < (int)pl->cases.size() && ok; ++sc) {
+		const int64_t parts = 16;
+		if (!progress)
+			ok = plan_run_all(pl) == 0;
+		for (int sc = 0; progress && sc < (int)pl->cases.size() && ok; ++sc) {
 			const int64_t nijk = pl->cases[sc].n_ijk;
 			for (int64_t p = 0; p < parts && ok; ++p) {
 				const int64_t b = nijk * p / parts;
 				const int64_t en = nijk * (p + 1) / parts;
-				ok = libpt_amd_plan_run(pl, sc, b, en) == 0;
-				if (ok && progress) {
-					ok = libpt_amd_plan_sync(pl) == 0;
-					fprintf(stderr, "[libpt_amd] spin case %d: ijk %lld of "
-					    "%lld done, %.1f s\n", sc, (long long)en,
-					    (long long)nijk, now_s() - t2);
-				}
+				ok = libpt_amd_plan_run(pl, sc, b, en) == 0 &&
+				    libpt_amd_plan_sync(pl) == 0;
+				fprintf(stderr, "[libpt_amd] spin case %d: ijk %lld of "
+				    "%lld done, %.1f s\n", sc, (long long)en,
+				    (long long)nijk, now_s() - t2);
 			}
 		}
 		if (ok)

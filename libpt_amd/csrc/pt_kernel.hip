@@ -295,15 +295,13 @@ k_synth(pt_synth_spec spec, int tensor, void *dst, int64_t n, int fp32)
 } /* namespace */
 
 extern "C" int
-pt_launch_tiles(int form, const struct pt_launch *p, void *stream)
+pt_launch_tiles(int form, const struct pt_launch *p, int n, void *stream)
 {
-	if (p->n_chunk <= 0)
-		return 0;
 	switch (form) {
-	case PT_FORM_FP64: return pt_launch_tiles_fp64(p, stream);
-	case PT_FORM_FP32: return pt_launch_tiles_fp32(p, stream);
-	case PT_FORM_BF16X3: return pt_launch_tiles_bf16x3(p, stream);
-	case PT_FORM_F16X3: return pt_launch_tiles_f16x3(p, stream);
+	case PT_FORM_FP64: return pt_launch_tiles_fp64(p, n, stream);
+	case PT_FORM_FP32: return pt_launch_tiles_fp32(p, n, stream);
+	case PT_FORM_BF16X3: return pt_launch_tiles_bf16x3(p, n, stream);
+	case PT_FORM_F16X3: return pt_launch_tiles_f16x3(p, n, stream);
 	}
 	return (int)hipErrorInvalidValue;
 }

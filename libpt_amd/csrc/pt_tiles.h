@@ -746,15 +746,48 @@ template <class GM> struct RoleC {
 };
 
 /*
+ * LDS of one item: the term table, the waves' sums, and one area used in
+ * turn for the S panels, the transpose's two buffers (of TRC (a block,
+ * register) columns each) and the epilogue's W columns and staged operands.
+ */
+template <int F, int KIND, int NSET, int NW>
+struct Lds {
+	typedef Geo<F, NSET, NW> GM;
+	static constexpr bool same = KIND == PT_AAA;
+	static constexpr int TC = GM::TC, AES = (int)sizeof(typename Form<F>::AE);
+	static constexpr int ERS = (int)sizeof(typename Form<F>::ER);
+	static constexpr int NTERM = NSET * (same ? PT_TERMS_SAME :
+	    PT_TERMS_MIXED);
+	static constexpr int TRW = TC + 1, TRC = 2;
+	static constexpr int TRB = TRC * 4 * 32 * TRW;  /* values per buffer */
+	static constexpr int NPB = same ? 6 : 4;        /* (b, c) blocks */
+	static constexpr int NBC = NPB * 32 * TC, NBV = (NPB + 1) * 32;
+	static constexpr int NBA = same ? 0 : 2 * 32 * 32;
+	static constexpr int EBYTES = NW * NSET * GM::BW * 64 * AES;
+	static constexpr int B1 = 2 * TRB * AES;
+	static constexpr int B2 = EBYTES + (NBC + NBV + NBA) * ERS;
+	static constexpr int RED = NTERM * (int)sizeof(TermP);
+	static constexpr int MEM = (RED + 8 * NW + 15) / 16 * 16;
+	static constexpr int BYTES = MEM + (B1 > B2 ? B1 : B2);
+	static_assert(B1 >= 2 * PANEL, "the S panels");
+	static_assert(BYTES * GM::WG_PER_CU <= 160 * 1024 - 256,
+	    "LDS of the workgroups of a CU");
+	static_assert(NBC % GM::THREADS == 0 && NBV <= GM::THREADS &&
+	    NBA % GM::THREADS == 0 && NTERM <= GM::THREADS,
+	    "staging by whole passes of the workgroup");
+};
+
+/*
  * One work item (ijk, tile) of a spin case: everything between reading the
  * item and writing its energy to partial[it].  KIND is the spin case,
  * PT_AAA or PT_AAB.  With two W sets the sets are formed one after the
  * other; wsv is the item's save area for W of set 0 (4 NACC values per lane
- * per wave).
+ * per wave); lds: Lds::BYTES.
  */
 template <int F, int KIND, int NSET, int NW>
 __device__ __forceinline__ void
-tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
+tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
+    char *lds)
 {
 	typedef Form<F> FM;
 	typedef Geo<F, NSET, NW> GM;
@@ -765,26 +798,13 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv)
 	constexpr int NACC = GM::NACC, NT = GM::THREADS;
 	constexpr bool same = KIND == PT_AAA;
 
-	/* LDS: the S panels; the transpose's buffers (two of TRC (a block,
-	 * register) columns each); the epilogue's W columns and staged operands */
-	constexpr int TRW = TC + 1, TRC = 2;
-	constexpr int TRB = TRC * 4 * 32 * TRW;      /* values per buffer */
-	constexpr int NPB = same ? 6 : 4;            /* (b, c) blocks */
-	constexpr int NBC = NPB * 32 * TC, NBV = (NPB + 1) * 32;
-	constexpr int NBA = same ? 0 : 2 * 32 * 32;
-	constexpr int EBYTES = NW * NSET * BW * 64 * (int)sizeof(AE);
-	constexpr int SB1 = 2 * TRB * (int)sizeof(AE);
-	constexpr int SB2 = EBYTES + (NBC + NBV + NBA) * (int)sizeof(ER);
-	constexpr int SMEM = SB1 > SB2 ? SB1 : SB2;
-	static_assert(SMEM >= 2 * PANEL, "the S panels");
-	constexpr int NTERM = NSET * (same ? PT_TERMS_SAME : PT_TERMS_MIXED);
-	static_assert((SMEM + NTERM * (int)sizeof(TermP) + 8 * NW + 64) *
-	    GM::WG_PER_CU <= 160 * 1024, "LDS of the workgroups of a CU");
-	static_assert(NBC % NT == 0 && NBV <= NT && NBA % NT == 0 &&
-	    NTERM <= NT, "staging by whole passes of the workgroup");
-	__shared__ __attribute__((aligned(16))) char smem[SMEM];
-	__shared__ double red[NW];
-	__shared__ TermP tp[NTERM];
+	typedef Lds<F, KIND, NSET, NW> LD;
+	constexpr int TRW = LD::TRW, TRC = LD::TRC, TRB = LD::TRB;
+	constexpr int NPB = LD::NPB, NBC = LD::NBC, NBV = LD::NBV, NBA = LD::NBA;
+	constexpr int EBYTES = LD::EBYTES, NTERM = LD::NTERM;
+	TermP *const tp = (TermP *)lds;
+	double *const red = (double *)(lds + LD::RED);
+	char *const smem = lds + LD::MEM;
 
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int wave = uni(tid >> 6);
@@ -1036,8 +1056,8 @@ wsave_of(void *wsave, int64_t slot)
 }
 
 /*
- * One launch over n_chunk positions of a run of one spin case's items (item
- * = ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
+ * One launch segment: n_chunk positions of a run of one spin case's items
+ * (item = ijk * n_tiles + tile).  XCD-aware order: workgroup n runs on XCD n % 8,
  * and each XCD gets a contiguous run of the launch's positions, so the
  * workgroups running together on one XCD share operand slices in its L2.
  * With kgrp > 1 the positions take the ijk in groups of kgrp, tile-major
@@ -1047,8 +1067,7 @@ wsave_of(void *wsave, int64_t slot)
  * share their slabs.  Each item still writes its own energy at its place in
  * the work list, so the energies do not depend on kgrp or perm.  One
  * workgroup per item, handed out by the dispatcher in order; with two W
- * sets position n of the launch keeps W of set 0 in save area n (n_chunk <=
- * p.nwsave).
+ * sets position n of the segment keeps W of set 0 in save area wslot0 + n.
  */
 __device__ __forceinline__ int64_t
 item_of(const pt_launch &p, int64_t it)
@@ -1068,13 +1087,48 @@ template <int F, int KIND, int NSET, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void
 k_tiles(pt_launch p)
 {
+	__shared__ __attribute__((aligned(16))) char
+	    lds[Lds<F, KIND, NSET, NW>::BYTES];
 	const int64_t per = (p.n_chunk + 7) / 8;
-	const int64_t x = blockIdx.x & 7;
-	const int64_t it = x * per + (blockIdx.x >> 3);
+	const int64_t it = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
 	if (it >= p.n_chunk)
 		return;
-	tile_item<F, KIND, NSET, NW>(p, item_of(p, it),
-	    NSET == 2 ? wsave_of<F, NW>(p.wsave, it) : nullptr);
+	tile_item<F, KIND, NSET, NW>(p, item_of(p, it), NSET == 2 ?
+	    wsave_of<F, NW>(p.wsave, p.wslot0 + it) : nullptr, lds);
+}
+
+/* the segments of one launch, of either spin case: workgroups first[s] ..
+ * first[s + 1] - 1 (first a multiple of 8, so that workgroup n of a segment
+ * is on XCD n % 8) */
+struct seg_args {
+	pt_launch seg[PT_MAX_SEGS];
+	int32_t first[PT_MAX_SEGS];
+	int32_t n;
+};
+
+template <int F, int NSET, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void
+k_tiles_segs(seg_args a)
+{
+	constexpr int B0 = Lds<F, PT_AAA, NSET, NW>::BYTES;
+	constexpr int B1 = Lds<F, PT_AAB, NSET, NW>::BYTES;
+	__shared__ __attribute__((aligned(16))) char lds[B0 > B1 ? B0 : B1];
+	int s = 0;
+	while (s + 1 < a.n && (int)blockIdx.x >= a.first[s + 1])
+		++s;
+	const pt_launch &p = a.seg[s];
+	const int n = (int)blockIdx.x - a.first[s];
+	const int64_t per = (p.n_chunk + 7) / 8;
+	const int64_t it = (n & 7) * per + (n >> 3);
+	if (it >= p.n_chunk)
+		return;
+	const int64_t item = item_of(p, it);
+	typename Form<F>::AE *w = NSET == 2 ?
+	    wsave_of<F, NW>(p.wsave, p.wslot0 + it) : nullptr;
+	if (p.kind == PT_AAA)
+		tile_item<F, PT_AAA, NSET, NW>(p, item, w, lds);
+	else
+		tile_item<F, PT_AAB, NSET, NW>(p, item, w, lds);
 }
 
 /*
@@ -1092,6 +1146,8 @@ template <int F, int KIND, int NSET, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void
 k_tiles_p(pt_launch p)
 {
+	__shared__ __attribute__((aligned(16))) char
+	    lds[Lds<F, KIND, NSET, NW>::BYTES];
 	__shared__ int s_next;
 	const int64_t per = (p.n_chunk + 7) / 8;
 	const int x = blockIdx.x & 7;
@@ -1105,8 +1161,8 @@ k_tiles_p(pt_launch p)
 		const int64_t r = __builtin_amdgcn_readfirstlane(s_next);
 		if (r >= cnt)
 			break;
-		tile_item<F, KIND, NSET, NW>(p, item_of(p, lo + r),
-		    NSET == 2 ? wsave_of<F, NW>(p.wsave, blockIdx.x) : nullptr);
+		tile_item<F, KIND, NSET, NW>(p, item_of(p, lo + r), NSET == 2 ?
+		    wsave_of<F, NW>(p.wsave, blockIdx.x) : nullptr, lds);
 	}
 }
 
@@ -1121,11 +1177,15 @@ k_zero_ctr(uint32_t *c)
 
 template <int F, int NSET, int NW>
 int
-launch_kind(const pt_launch *p, hipStream_t s)
+launch_geo(const pt_launch *p, int n, hipStream_t s)
 {
 	typedef Geo<F, NSET, NW> GM;
-	if (p->tcw != GM::TC)
+	if (n < 1 || n > PT_MAX_SEGS)
 		return (int)hipErrorInvalidValue;
+	for (int q = 0; q < n; ++q)
+		if (p[q].tcw != GM::TC || p[q].nw != NW || p[q].nset != NSET ||
+		    (n > 1 && p[q].ctr))
+			return (int)hipErrorInvalidValue;
 	dim3 block(GM::THREADS);
 	if (p->ctr) {
 		/* persistent grid: one save area per workgroup */
@@ -1140,11 +1200,24 @@ launch_kind(const pt_launch *p, hipStream_t s)
 			k_tiles_p<F, PT_AAB, NSET, NW><<<grid, block, 0, s>>>(*p);
 		return (int)hipGetLastError();
 	}
-	/* one save area per item */
-	if (NSET == 2 && (!p->wsave || p->n_chunk > p->nwsave))
-		return (int)hipErrorInvalidValue;
-	dim3 grid((unsigned)(8 * ((p->n_chunk + 7) / 8)));
-	if (p->kind == PT_AAA)
+	seg_args a;
+	a.n = n;
+	int64_t wgs = 0;
+	for (int q = 0; q < n; ++q) {
+		/* one save area per item */
+		if (NSET == 2 && (!p[q].wsave || p[q].wslot0 < 0 ||
+		    p[q].wslot0 + p[q].n_chunk > p[q].nwsave))
+			return (int)hipErrorInvalidValue;
+		a.seg[q] = p[q];
+		a.first[q] = (int32_t)wgs;
+		wgs += 8 * ((p[q].n_chunk + 7) / 8);
+		if (wgs > INT32_MAX / 2)
+			return (int)hipErrorInvalidValue;
+	}
+	const dim3 grid((unsigned)wgs);
+	if (n > 1)
+		k_tiles_segs<F, NSET, NW><<<grid, block, 0, s>>>(a);
+	else if (p->kind == PT_AAA)
 		k_tiles<F, PT_AAA, NSET, NW><<<grid, block, 0, s>>>(*p);
 	else
 		k_tiles<F, PT_AAB, NSET, NW><<<grid, block, 0, s>>>(*p);
@@ -1153,13 +1226,13 @@ launch_kind(const pt_launch *p, hipStream_t s)
 
 template <int F>
 int
-launch_form(const pt_launch *p, hipStream_t s)
+launch_form(const pt_launch *p, int n, hipStream_t s)
 {
 	if (p->nw == 8)
-		return p->nset == 1 ? launch_kind<F, 1, 8>(p, s) :
-		    launch_kind<F, 2, 8>(p, s);
-	return p->nset == 1 ? launch_kind<F, 1, 4>(p, s) :
-	    launch_kind<F, 2, 4>(p, s);
+		return p->nset == 1 ? launch_geo<F, 1, 8>(p, n, s) :
+		    launch_geo<F, 2, 8>(p, n, s);
+	return p->nset == 1 ? launch_geo<F, 1, 4>(p, n, s) :
+	    launch_geo<F, 2, 4>(p, n, s);
 }
 
 } /* namespace */

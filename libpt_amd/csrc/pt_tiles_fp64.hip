@@ -2,7 +2,7 @@
 #include "pt_tiles.h"
 
 extern "C" int
-pt_launch_tiles_fp64(const struct pt_launch *p, void *stream)
+pt_launch_tiles_fp64(const struct pt_launch *p, int n, void *stream)
 {
-	return launch_form<PT_FORM_FP64>(p, (hipStream_t)stream);
+	return launch_form<PT_FORM_FP64>(p, n, (hipStream_t)stream);
 }
