@@ -29,7 +29,7 @@
  * wave and used by both 16-row blocks of S.  There is nothing to share
  * through LDS, hence no barrier in the step loop: the two waves of a SIMD
  * drift apart and fill each other's waits, and each fragment register is
- * reloaded for the next step right after its MFMAs, one whole step ahead.
+ * reloaded for the next step soon after its MFMAs.
  * Against the kernel that staged the operands in LDS (two slots, a barrier
  * per step, one wave per 16 a x 16 b x TC c): MFMA pipe 84 % busy instead of
  * 67 % at rpt v=477 in FP64, where the card's clock then falls from 2.2 to
@@ -78,6 +78,7 @@ template <> struct Form<PT_FORM_FP64> {
 	typedef double ER;  /* epilogue real */
 	static constexpr int KC = 8;    /* kappa per fragment */
 	static constexpr bool ROW_F64 = true, SPLIT = false, PAN = false;
+	static constexpr int LAG = 1;   /* groups between use and reload */
 };
 
 template <> struct Form<PT_FORM_FP32> {
@@ -87,6 +88,7 @@ template <> struct Form<PT_FORM_FP32> {
 	typedef float ER;
 	static constexpr int KC = 16;
 	static constexpr bool ROW_F64 = false, SPLIT = false, PAN = false;
+	static constexpr int LAG = 1;   /* groups between use and reload */
 };
 
 template <> struct Form<PT_FORM_BF16X3> {
@@ -97,6 +99,7 @@ template <> struct Form<PT_FORM_BF16X3> {
 	static constexpr int KC = 16;
 	static constexpr bool ROW_F64 = false, SPLIT = true;
 	static constexpr bool PAN = true;   /* S staged in LDS panels */
+	static constexpr int LAG = 2;
 };
 
 template <> struct Form<PT_FORM_F16X3> : Form<PT_FORM_BF16X3> {};
@@ -461,10 +464,18 @@ make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
  * those outside it may not exist, so the nearest one of the range is read
  * in their place (their blocks are never used).
  *
- * Step n = (term, chunk).  Each fragment's registers are loaded for step
- * n + 1 right after its MFMAs of step n, so that a step's loads are always
- * in flight per wave and every load has one step to arrive; the loads after
+ * Step n = (term, chunk).  A step's MFMAs go in four groups (half of x, e);
+ * a group's fragments are loaded for the next step LAG groups after their
+ * MFMAs, so 4 - LAG groups of loads are in flight per wave; the loads after
  * the last step are all out of range and return zero.
+ *   How far ahead decides how the workgroups of an XCD share its L2.  With a
+ * whole step to arrive even loads that miss L2 are hidden, and workgroups
+ * that read the same slabs drift apart until each fetches them for itself;
+ * with less, the first one waits for HBM, the ones behind it hit and catch
+ * up, and they run together.  The split forms, bound by L2 and HBM, take
+ * LAG = 2: rpt v=477 split-BF16 209 -> 165 to 177 ms for 0 -> 2 (3: 216 ms, its
+ * hits wait too); rft v=300 F16X3 92 ms for either (3: 116 ms).  FP64 and
+ * FP32 take 1, from 0: within 1 % everywhere (2: v=120 FP64 211 -> 216 ms).
  *
  * S is the same for all waves, and its rows are scattered 64-byte pieces in
  * the API layout: loaded by each wave for itself, a 16-row block costs the
@@ -514,6 +525,7 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 	constexpr int XB = 16 / NW;      /* x per 16 w */
 	/* panel fragments (step, S block) are dealt to the waves in order */
 	constexpr bool PAN = Form<F>::PAN;
+	constexpr int LAG = Form<F>::LAG;
 	constexpr int NI = PAN ? PC * NSB / NW : NSB, ND = NW / NSB;
 	static_assert(PC * NSB % NW == 0 && NW % NSB == 0, "panel split");
 	if (t0 >= t1)
@@ -635,11 +647,15 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 	int t = t0, n = 0;
 	stage_load();
 	v4u q[2 * NX];
+	/* the fragments of group g = (half of x, e) */
+	auto load_g = [&](int g) {
 #pragma unroll
-	for (int x = 0; x < NX; ++x)
+		for (int x = (g >> 1) * NH; x < ((g >> 1) + 1) * NH; ++x)
+			q[2 * x + (g & 1)] = load_q(x, g & 1);
+	};
 #pragma unroll
-		for (int e = 0; e < 2; ++e)
-			q[2 * x + e] = load_q(x, e);
+	for (int g = 0; g < 4 - LAG; ++g)
+		load_g(g);
 	if constexpr (PAN) {
 		stage_write();
 		lds_barrier();
@@ -651,25 +667,14 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 		for (int e = 0; e < NSB; ++e)
 			s[e].set(PAN ? *(const v4u *)(panels + par * PANEL + rofs +
 			    1024 * (NSB * n + e)) : sr[e], sgn);
-		/* on to the next step */
-		if (--left > 0) {
-			q0 += dq0;
-			q1 += dq1;
-		} else if (++t < t1) {
-			term(t);
-		} else {
-			more = false;
-			vo[0] = vo[1] = PT_OOR;
-		}
 		if constexpr (!PAN)
 			stage_load();
 #pragma unroll
-		for (int h = 0; h < 2; ++h)
-#pragma unroll
-		for (int e = 0; e < 2; ++e) {
+		for (int g = 0; g < 4; ++g) {
+			const int h = g >> 1, e = g & 1;
 #pragma unroll
 			for (int b = 0; b < NSB; ++b)
-				if (grp >> ((h * 2 + e) * NSB + b) & 1) {
+				if (grp >> (g * NSB + b) & 1) {
 #pragma unroll
 					for (int m = 0; m < NMF<F>; ++m)
 #pragma unroll
@@ -679,9 +684,19 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 						    acc[a]);
 					}
 				}
-#pragma unroll
-			for (int x = h * NH; x < (h + 1) * NH; ++x)
-				q[2 * x + e] = load_q(x, e);
+			if (g == LAG) {
+				/* on to the next step */
+				if (--left > 0) {
+					q0 += dq0;
+					q1 += dq1;
+				} else if (++t < t1) {
+					term(t);
+				} else {
+					more = false;
+					vo[0] = vo[1] = PT_OOR;
+				}
+			}
+			load_g((g + 4 - LAG) & 3);
 			__builtin_amdgcn_sched_barrier(0);
 		}
 		if (PAN && ++n == PC) {
