@@ -797,12 +797,13 @@ struct Lds {
  * item and writing its energy to partial[it].  KIND is the spin case,
  * PT_AAA or PT_AAB.  With two W sets the sets are formed one after the
  * other; wsv is the item's save area for W of set 0 (4 NACC values per lane
- * per wave); lds: Lds::BYTES.
+ * per wave); lds: Lds::BYTES.  keep false: the energy is not written (and
+ * wsv is null: what goes to the save area is dropped).
  */
 template <int F, int KIND, int NSET, int NW>
 __device__ __forceinline__ void
 tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
-    char *lds)
+    char *lds, bool keep = true)
 {
 	typedef Form<F> FM;
 	typedef Geo<F, NSET, NW> GM;
@@ -821,7 +822,7 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 	double *const red = (double *)(lds + LD::RED);
 	char *const smem = lds + LD::MEM;
 
-	const int tid = threadIdx.x, lane = tid & 63;
+	const int tid = threadIdx.x % NT, lane = tid & 63;
 	const int wave = uni(tid >> 6);
 	const int ln = lane & 15, lg = lane >> 4;
 
@@ -874,7 +875,7 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 	/* save area of W set 0: value (r, x) of (wave, lane) at element
 	 * ((r NACC + x) NW + wave) 64 + lane */
 	constexpr int WST = NW * 64 * (int)sizeof(AE);
-	const __amdgpu_buffer_rsrc_t wr = brsrc(wsv, NSET == 2 ?
+	const __amdgpu_buffer_rsrc_t wr = brsrc(wsv, NSET == 2 && wsv ?
 	    (int64_t)4 * NACC * WST : 0);
 	const uint32_t wvo = (uint32_t)((wave * 64 + lane) * sizeof(AE));
 
@@ -1057,7 +1058,8 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 		double t = (red[0] + red[1]) + (red[2] + red[3]);
 		if constexpr (NW == 8)
 			t += (red[4] + red[5]) + (red[6] + red[7]);
-		p.partial[it] = t;
+		if (keep)
+			p.partial[it] = t;
 	}
 }
 /* save area `slot` of wsave (two W sets; pt_wsave_bytes each) */
@@ -1110,6 +1112,47 @@ k_tiles(pt_launch p)
 		return;
 	tile_item<F, KIND, NSET, NW>(p, item_of(p, it), NSET == 2 ?
 	    wsave_of<F, NW>(p.wsave, p.wslot0 + it) : nullptr, lds);
+}
+
+/*
+ * Two items, next to each other in launch order, per workgroup: four waves
+ * each, the whole CU.  Every item of a launch has the same terms and panels,
+ * so both halves meet the same barriers, and the two items of a CU walk their
+ * slabs in step; mostly they have the same tile and share slabs, and what one
+ * half fetched the other finds in L1 or L2 instead of fetching it again.
+ * That pays where the split forms wait for HBM, i.e. where the slabs that
+ * the workgroups of an XCD use together outgrow its L2; below, two workgroups
+ * that drift apart fill each other's barriers and epilogues.  The change is
+ * gradual (48 ijk of rpt o=10 in split BF16, one item per workgroup -> pairs,
+ * same-spin and mixed-spin ms): v=300 8.03 -> 8.01 and 18.6 -> 19.0, v=352
+ * 12.7 -> 12.3 and 28.9 -> 28.6, v=400 23.1 -> 22.1 and 50.8 -> 50.3, v=477
+ * 46.6 -> 41.2 and 94.8 -> 93.6, v=600 134 -> 101 and 238 -> 230; two W sets
+ * (rft F16X3) v=256 9.1 -> 9.5 and 20.6 -> 21.3, v=350 30.3 -> 30.1 and 76.6
+ * -> 76.5, v=400 56.0 -> 51.6 and 133 -> 134.  At v=8 to 200 pairs cost 2 to
+ * 25 %, and FP64 and FP32 (no barriers to keep two workgroups together or
+ * apart) 2 to 20 % there and 4 % at v=477.
+ */
+constexpr int PAIR_NA = 384;
+
+template <int F, int KIND, int NSET>
+__global__ __launch_bounds__(512, 1) void
+k_tiles_pair(pt_launch p)
+{
+	typedef Lds<F, KIND, NSET, 4> LD;
+	__shared__ __attribute__((aligned(16))) char lds[2 * LD::BYTES];
+	const int half = uni((int)threadIdx.x / 256);
+	const int64_t per = (p.n_chunk + 15) / 16 * 2;
+	const int64_t lo = (blockIdx.x & 7) * per;
+	const int64_t hi = lo + per < p.n_chunk ? lo + per : p.n_chunk;
+	const int64_t i0 = lo + 2 * (int64_t)(blockIdx.x >> 3);
+	if (i0 >= hi)
+		return;
+	/* an odd end: the second half does the first one's item and drops it */
+	const bool keep = i0 + half < hi;
+	const int64_t it = keep ? i0 + half : i0;
+	tile_item<F, KIND, NSET, 4>(p, item_of(p, it), NSET == 2 && keep ?
+	    wsave_of<F, 4>(p.wsave, p.wslot0 + it) : nullptr,
+	    lds + half * LD::BYTES, keep);
 }
 
 /* the segments of one launch, of either spin case: workgroups first[s] ..
@@ -1230,6 +1273,15 @@ launch_geo(const pt_launch *p, int n, hipStream_t s)
 			return (int)hipErrorInvalidValue;
 	}
 	const dim3 grid((unsigned)wgs);
+	if constexpr (Form<F>::PAN && NW == 4)
+		if (n == 1 && p->na >= PAIR_NA) {
+			const dim3 pairs((unsigned)(8 * ((p->n_chunk + 15) / 16)));
+			if (p->kind == PT_AAA)
+				k_tiles_pair<F, PT_AAA, NSET><<<pairs, 512, 0, s>>>(*p);
+			else
+				k_tiles_pair<F, PT_AAB, NSET><<<pairs, 512, 0, s>>>(*p);
+			return (int)hipGetLastError();
+		}
 	if (n > 1)
 		k_tiles_segs<F, NSET, NW><<<grid, block, 0, s>>>(a);
 	else if (p->kind == PT_AAA)
