@@ -17,8 +17,8 @@
  *       disconnected term Z, denominator Dn, energy W (W - Z) / Dn
  *       ((fT): (W_L - Z_L) W_R / Dn), compensated FP64 sum per lane,
  *       one deterministic reduction per workgroup into partial[item];
- *       the Z and Dn operands that depend on b are staged in LDS once
- *       per item, those of a and c alone held in registers per lane.
+ *       the Z and Dn operands are staged in LDS, those of (a, c) held
+ *       in registers per lane.
  *
  * Operands go from the packed copies straight into the registers of the
  * wave that multiplies them.  A packed Q slab is a sequence of fragments of
@@ -210,124 +210,127 @@ kahan(double &s, double &cmp, double x)
 
 /*
  * Energy terms of one lane's NB elements (a, b0 + BS y, c), y = 0 .. NB-1,
- * in y order, added to (esum, ecmp): the disconnected term Z, the
- * denominator Dn = d_ia + d_jb + d_kc and W (W - Z) / Dn, or for two W sets
- * (W_L - Z) W_R / Dn (src/pt.c:700,927).  The loads that depend on a, c or
- * (a, c) only are made once for the NB elements; b is clamped into the
- * arrays, so every element's loads are made whether or not the triangle
- * keeps it, and only the sum is masked.  W values: ew[64 y] (one set; the
- * right set with two) and ew[64 (y + NB)] (the left set).  The workgroup
- * has staged in LDS the (b, c) values of i_oovv and t2, sbc[(32 n + BS y)
- * TC] (sbc points at this lane's b0 and c) for n = G jk, Z jk, G ik, Z ik
- * (mixed spin: GB, ZB; same spin also G ji, Z ji), the values that depend
- * on b only, sbv[32 n + BS y] (sbv points at b0) for n = u i, f i, u j,
- * f j, (same spin: u k, f k,) d1 j, and for the mixed spin case the (b, a)
- * values of the same-spin blocks for ji, sba[(32 n + BS y) 32] for n = GA,
- * ZA (sba points at b0 and this lane's a).
+ * in y order, even y added to (esum, ecmp)[0], odd ones to [1]: the
+ * disconnected term Z, the denominator Dn = d_ia + d_jb + d_kc and W (W - Z) / Dn, or for two W sets
+ * (W_L - Z) W_R / Dn (src/pt.c:700,927).  Everything comes from registers
+ * and LDS; every element's values are made whether or not the triangle keeps
+ * it, and only the sum is masked.  W values: ew[64 y] (one set; the right
+ * set with two) and ew[64 (y + NB)] (the left set).  ac: the (a, c) values
+ * of i_oovv and t2, [G jk, Z jk, G ik, Z ik (, G ji, Z ji)] (mixed spin: GB,
+ * ZB; same spin also ji).  sbc: the same for (b, c), sbc[(32 n + BS y) TC]
+ * (sbc points at this lane's b0 and c).  sav, sbv, scv: the values that
+ * depend on a, b, c only, n = u i, f i, u j, f j, (same spin: u k, f k,)
+ * d1 i (a), d1 j (b), d1 k (c), at sav[32 n], sbv[32 n + BS y], scv[TC n];
+ * mixed spin c: u2 k, f2 k, d2 k.  sba: the (b, a) values; mixed spin: GA, ZA
+ * for ji at sba[(32 n + BS y) 32]; same spin: G, Z (n & 1) for jk, ik, ji
+ * (n / 2) at sba[8 NB (n / 2) + 8 y + 4 (n & 1)].
+ *   Bound by latency: an element is about 20 LDS reads and 30 dependent FP64
+ * operations, with one or two waves per SIMD.  Elements go in pairs, whose
+ * chains interleave, and nothing in the loop comes from global memory.  Against
+ * one element at a time with the same-spin (b, a) values read from global
+ * memory (us or ms, same-spin / mixed-spin items): split BF16 rpt v=96 272 /
+ * 1025 -> 251 / 1010 us, v=256 4.53 / 10.1 -> 4.27 / 9.95 ms; FP32 upt v=200 a
+ * share 189 -> 183 ms, rpt_mp v=101 call 142 -> 136 ms; FP64 rpt v=100 1.03 /
+ * 5.53 -> 0.99 / 5.52 ms, v=120 call 208 -> 206 ms.
  */
 template <int F, int KIND, int NSET, int NB, int BS, int TC>
 __device__ __forceinline__ void
-epi_block(const pt_launch &p, int i, int j, int k, int a, int c, int b0,
-    const typename Form<F>::AE *ew,
-    const typename Form<F>::ER *sbc, const typename Form<F>::ER *sba,
-    const typename Form<F>::ER *sbv, double &esum, double &ecmp)
+epi_block(const pt_launch &p, int a, int c, int b0,
+    const typename Form<F>::AE *ew, const typename Form<F>::ER *ac,
+    const typename Form<F>::ER *sav, const typename Form<F>::ER *sbv,
+    const typename Form<F>::ER *scv, const typename Form<F>::ER *sbc,
+    const typename Form<F>::ER *sba, double (&esum)[2], double (&ecmp)[2])
 {
 	typedef typename Form<F>::ER ER;
 	const ER s0 = (ER)p.inv_scale[0], s1 = (ER)p.inv_scale[1];
-	const ER *d1 = (const ER *)p.epi.d1;
-	/* this element's term from its Z and Dn */
-	auto term = [&](int y, ER z, ER dn) {
+	/* W (W - Z) or the two-set form of element h, over Dn, into the sum */
+	auto add = [&](int y, int h, bool in, ER z, ER dn) {
+		ER t;
 		if constexpr (NSET == 1) {
-			ER w = (ER)ew[64 * y];
+			ER w = (ER)ew[64 * (y + h)];
 			if (Form<F>::SPLIT)
 				w *= s0;
-			return w * (w - z) / dn;
+			t = w * (w - z) / dn;
 		} else {
-			ER wl = (ER)ew[64 * (y + NB)], wr = (ER)ew[64 * y];
+			ER wl = (ER)ew[64 * (y + h + NB)], wr = (ER)ew[64 * (y + h)];
 			if (Form<F>::SPLIT) {
 				wl *= s0;
 				wr *= s1;
 			}
-			return (wl - z) * wr / dn;
+			t = (wl - z) * wr / dn;
 		}
+		double s = esum[h], e = ecmp[h];
+		kahan(s, e, (double)t);
+		esum[h] = in ? s : esum[h];
+		ecmp[h] = in ? e : ecmp[h];
 	};
+	const ER uia = sav[0], fia = sav[32], uja = sav[64], fja = sav[96];
 	if constexpr (KIND == PT_AAA) {
 		/* src/pt.c:162-175, for (u, G) = (t1 or l1, i_oovv) and
 		 * (f, Z) = (f_ov or f2_ov, t2 or l2) */
-		const int64_t o = p.oa, v = p.va, vv = v * v;
-		const ER *u = (const ER *)p.epi.u1, *f = (const ER *)p.epi.f1;
-		const ER *G = (const ER *)p.epi.GA, *Z = (const ER *)p.epi.ZA;
-		const int64_t jk = ((int64_t)j * o + k) * vv;
-		const int64_t ik = ((int64_t)i * o + k) * vv;
-		const int64_t ji = ((int64_t)j * o + i) * vv;
-		const ER uia = u[i * v + a], uja = u[j * v + a], uka = u[k * v + a];
-		const ER fia = f[i * v + a], fja = f[j * v + a], fka = f[k * v + a];
-		const ER uic = u[i * v + c], ujc = u[j * v + c], ukc = u[k * v + c];
-		const ER fic = f[i * v + c], fjc = f[j * v + c], fkc = f[k * v + c];
-		const int64_t ac = (int64_t)a * v + c;
-		const ER gjkac = G[jk + ac], gikac = G[ik + ac], gjiac = G[ji + ac];
-		const ER zjkac = Z[jk + ac], zikac = Z[ik + ac], zjiac = Z[ji + ac];
-		const ER dia = d1[i * v + a], dkc = d1[k * v + c];
+		const ER uka = sav[128], fka = sav[160], dia = sav[192];
+		const ER uic = scv[0], fic = scv[TC], ujc = scv[2 * TC];
+		const ER fjc = scv[3 * TC], ukc = scv[4 * TC], fkc = scv[5 * TC];
+		const ER dkc = scv[6 * TC];
 #pragma unroll 1
-		for (int y = 0; y < NB; ++y) {
-			const int bb = BS * y, b = b0 + bb;
-			const int bq = b < p.na ? b : p.na - 1;
-			const int64_t ba = (int64_t)bq * v + a;
-			const ER uib = sbv[bb], fib = sbv[32 + bb];
-			const ER ujb = sbv[64 + bb], fjb = sbv[96 + bb];
-			const ER ukb = sbv[128 + bb], fkb = sbv[160 + bb];
-			const ER djb = sbv[192 + bb];
-			const ER gjkbc = sbc[bb * TC], zjkbc = sbc[(32 + bb) * TC];
-			const ER gikbc = sbc[(64 + bb) * TC];
-			const ER zikbc = sbc[(96 + bb) * TC];
-			const ER gjibc = sbc[(128 + bb) * TC];
-			const ER zjibc = sbc[(160 + bb) * TC];
-			const ER zu = uia * gjkbc - uja * gikbc -
-			    uka * gjibc - uib * gjkac + ujb * gikac +
-			    ukb * gjiac - uic * G[jk + ba] + ujc * G[ik + ba] +
-			    ukc * G[ji + ba];
-			const ER zf = fia * zjkbc - fja * zikbc -
-			    fka * zjibc - fib * zjkac + fjb * zikac +
-			    fkb * zjiac - fic * Z[jk + ba] + fjc * Z[ik + ba] +
-			    fkc * Z[ji + ba];
-			const ER t = term(y, zu + zf, dia + djb + dkc);
-			if (a > b && b > c)
-				kahan(esum, ecmp, (double)t);
+		for (int y = 0; y < NB; y += 2) {
+			ER zu[2], zf[2], dn[2];
+#pragma unroll
+			for (int h = 0; h < 2; ++h) {
+				const ER *bc = sbc + BS * (y + h) * TC;
+				zu[h] = uia * bc[0] - uja * bc[64 * TC] - uka * bc[128 * TC];
+				zf[h] = fia * bc[32 * TC] - fja * bc[96 * TC] -
+				    fka * bc[160 * TC];
+			}
+#pragma unroll
+			for (int h = 0; h < 2; ++h) {
+				const ER *bv = sbv + BS * (y + h);
+				zu[h] = zu[h] - bv[0] * ac[0] + bv[64] * ac[2] +
+				    bv[128] * ac[4];
+				zf[h] = zf[h] - bv[32] * ac[1] + bv[96] * ac[3] +
+				    bv[160] * ac[5];
+				dn[h] = dia + bv[192] + dkc;
+			}
+#pragma unroll
+			for (int h = 0; h < 2; ++h) {
+				const ER *ba = sba + 8 * (y + h);
+				zu[h] = zu[h] - uic * ba[0] + ujc * ba[8 * NB] +
+				    ukc * ba[16 * NB];
+				zf[h] = zf[h] - fic * ba[4] + fjc * ba[8 * NB + 4] +
+				    fkc * ba[16 * NB + 4];
+			}
+#pragma unroll
+			for (int h = 0; h < 2; ++h) {
+				const int b = b0 + BS * (y + h);
+				add(y, h, a > b && b > c, zu[h] + zf[h], dn[h]);
+			}
 		}
 	} else {
 		/* src/pt.c:177-185 and :433-442 */
-		const int64_t va = p.va, ob = p.ob, vb = p.vb;
-		const ER *u1 = (const ER *)p.epi.u1, *u2 = (const ER *)p.epi.u2;
-		const ER *f1 = (const ER *)p.epi.f1, *f2 = (const ER *)p.epi.f2;
-		const ER *GB = (const ER *)p.epi.GB, *ZB = (const ER *)p.epi.ZB;
-		const ER *d2 = (const ER *)p.epi.d2;
-		const int64_t jk = ((int64_t)j * ob + k) * va;
-		const int64_t ik = ((int64_t)i * ob + k) * va;
-		const ER uia = u1[i * va + a], fia = f1[i * va + a];
-		const ER uja = u1[j * va + a], fja = f1[j * va + a];
-		const ER u2c = u2[k * vb + c], f2c = f2[k * vb + c];
-		const int64_t jkac = (jk + a) * vb + c, ikac = (ik + a) * vb + c;
-		const ER gjkac = GB[jkac], zjkac = ZB[jkac];
-		const ER gikac = GB[ikac], zikac = ZB[ikac];
-		const ER dia = d1[i * va + a], dkc = d2[k * vb + c];
+		const ER dia = sav[128];
+		const ER u2c = scv[0], f2c = scv[TC], dkc = scv[2 * TC];
 #pragma unroll 1
-		for (int y = 0; y < NB; ++y) {
-			const int bb = BS * y, b = b0 + bb;
-			const ER uib = sbv[bb], fib = sbv[32 + bb];
-			const ER ujb = sbv[64 + bb], fjb = sbv[96 + bb];
-			const ER djb = sbv[128 + bb];
-			const ER gjkbc = sbc[bb * TC], zjkbc = sbc[(32 + bb) * TC];
-			const ER gikbc = sbc[(64 + bb) * TC];
-			const ER zikbc = sbc[(96 + bb) * TC];
-			const ER gjiba = sba[bb * 32], zjiba = sba[(32 + bb) * 32];
-			const ER z = (uia * gjkbc + fia * zjkbc)
-			    - (uib * gjkac + fib * zjkac)
-			    - (uja * gikbc + fja * zikbc)
-			    + (ujb * gikac + fjb * zikac)
-			    + (u2c * gjiba + f2c * zjiba);
-			const ER t = term(y, z, dia + djb + dkc);
-			if (a > b)
-				kahan(esum, ecmp, (double)t);
+		for (int y = 0; y < NB; y += 2) {
+			ER z[2], dn[2];
+#pragma unroll
+			for (int h = 0; h < 2; ++h) {
+				const int bb = BS * (y + h);
+				const ER uib = sbv[bb], fib = sbv[32 + bb];
+				const ER ujb = sbv[64 + bb], fjb = sbv[96 + bb];
+				const ER gjkbc = sbc[bb * TC], zjkbc = sbc[(32 + bb) * TC];
+				const ER gikbc = sbc[(64 + bb) * TC];
+				const ER zikbc = sbc[(96 + bb) * TC];
+				const ER gjiba = sba[bb * 32], zjiba = sba[(32 + bb) * 32];
+				z[h] = (uia * gjkbc + fia * zjkbc)
+				    - (uib * ac[0] + fib * ac[1])
+				    - (uja * gikbc + fja * zikbc)
+				    + (ujb * ac[2] + fjb * ac[3])
+				    + (u2c * gjiba + f2c * zjiba);
+				dn[h] = dia + sbv[128 + bb] + dkc;
+			}
+#pragma unroll
+			for (int h = 0; h < 2; ++h)
+				add(y, h, a > b0 + BS * (y + h), z[h], dn[h]);
 		}
 	}
 }
@@ -777,18 +780,20 @@ struct Lds {
 	static constexpr int TRB = TRC * 4 * 32 * TRW;  /* values per buffer */
 	static constexpr int NPB = same ? 6 : 4;        /* (b, c) blocks */
 	static constexpr int NBC = NPB * 32 * TC, NBV = (NPB + 1) * 32;
-	static constexpr int NBA = same ? 0 : 2 * 32 * 32;
+	static constexpr int NCV = (same ? NPB + 1 : 3) * TC;  /* c vectors */
+	static constexpr int NCOL = 24 * GM::BW;  /* a wave's (b, a) values */
+	static constexpr int NBA = same ? NW * NCOL : 2 * 32 * 32;
 	static constexpr int EBYTES = NW * NSET * GM::BW * 64 * AES;
 	static constexpr int B1 = 2 * TRB * AES;
-	static constexpr int B2 = EBYTES + (NBC + NBV + NBA) * ERS;
+	static constexpr int B2 = EBYTES + (NBC + 2 * NBV + NCV + NBA) * ERS;
 	static constexpr int RED = NTERM * (int)sizeof(TermP);
 	static constexpr int MEM = (RED + 8 * NW + 15) / 16 * 16;
 	static constexpr int BYTES = MEM + (B1 > B2 ? B1 : B2);
 	static_assert(B1 >= 2 * PANEL, "the S panels");
 	static_assert(BYTES * GM::WG_PER_CU <= 160 * 1024 - 256,
 	    "LDS of the workgroups of a CU");
-	static_assert(NBC % GM::THREADS == 0 && NBV <= GM::THREADS &&
-	    NBA % GM::THREADS == 0 && NTERM <= GM::THREADS,
+	static_assert(NBC % GM::THREADS == 0 && NTERM <= GM::THREADS &&
+	    (same || NBA % GM::THREADS == 0),
 	    "staging by whole passes of the workgroup");
 };
 
@@ -817,6 +822,7 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 	typedef Lds<F, KIND, NSET, NW> LD;
 	constexpr int TRW = LD::TRW, TRC = LD::TRC, TRB = LD::TRB;
 	constexpr int NPB = LD::NPB, NBC = LD::NBC, NBV = LD::NBV, NBA = LD::NBA;
+	constexpr int NCV = LD::NCV, NCOL = LD::NCOL;
 	constexpr int EBYTES = LD::EBYTES, NTERM = LD::NTERM;
 	TermP *const tp = (TermP *)lds;
 	double *const red = (double *)(lds + LD::RED);
@@ -958,32 +964,36 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 	/* epilogue: layout [a][c]@b; the lane holds c = C0 + 16 cb + ln.  Each
 	 * (register, a block, c block) column of BW b goes through the lane's
 	 * own LDS slots, so that the element loop runs with a runtime index. */
-	double esum = 0.0, ecmp = 0.0;
+	double esum[2] = {0.0, 0.0}, ecmp[2] = {0.0, 0.0};
 	AE *E = (AE *)smem + wave * (NSET * BW * 64) + lane;
-	/* the tile's epilogue operands that do not depend on a or c alone,
-	 * staged once in LDS behind the W values: the (b, c) blocks of i_oovv
-	 * and t2, [G jk, Z jk, G ik, Z ik (, G ji, Z ji)][32 b][TC c] (mixed
-	 * spin: the GB, ZB blocks; same spin: GA, ZA with ji), the b vectors
-	 * [u i, f i, u j, f j, (u k, f k,) d1 j][32 b] and, for the mixed spin
-	 * case, the (b, a) blocks of the same-spin ones for ji, [GA, ZA][32
-	 * b][32 a] (rows and columns beyond the arrays repeat the last one; the
-	 * epilogue masks those elements). */
+	/* the tile's epilogue operands, staged in LDS behind the W values: the
+	 * (b, c) blocks of i_oovv and t2, [G jk, Z jk, G ik, Z ik (, G ji, Z
+	 * ji)][32 b][TC c] (mixed spin: the GB, ZB blocks; same spin: GA, ZA with
+	 * ji), the vectors [u i, f i, u j, f j, (u k, f k,) d1][32] of a (d1 i)
+	 * and b (d1 j), those of c (same spin: the same, d1 k; mixed: u2 k, f2 k,
+	 * d2 k), and the (b, a) blocks: for the mixed spin case those of the
+	 * same-spin arrays for ji, [GA, ZA][32 b][32 a]; the six of the same-spin
+	 * case do not fit, so each wave keeps the values of one (a block,
+	 * register) at a time, [jk, ik, ji][BW b][G, Z][4 a], loaded one ahead.
+	 * Rows and columns beyond the arrays repeat the last one; the epilogue
+	 * masks those elements. */
 	if (FM::PAN)
 		lds_barrier();   /* the last panel's reads */
 	ER *const stg = (ER *)(smem + EBYTES);
+	ER *const sva = stg + NBC + NBV, *const svc = sva + NBV;
+	ER *const sab = svc + NCV;
 	const ER *sbc = stg + wave * TC + ln;
 	const ER *sbv = stg + NBC + wave;
-	const ER *sba = stg + NBC + NBV + wave * 32;
+	/* block n: (G, Z)[n & 1] of pair n / 2 = jk, ik (, ji); mixed spin: rows
+	 * (jk + b) vb, same spin: jk + b v, v = vb */
+	const ER *G = (const ER *)(same ? p.epi.GA : p.epi.GB);
+	const ER *Z = (const ER *)(same ? p.epi.ZA : p.epi.ZB);
+	const int64_t po = same ? p.oa : p.ob;
+	const int64_t pr = same ? p.va * p.va : p.va * p.vb;
+	const int64_t pjk = ((int64_t)j * po + k) * pr;
+	const int64_t pik = ((int64_t)i * po + k) * pr;
+	const int64_t pji = ((int64_t)j * p.oa + i) * pr;
 	{
-		/* block n: (G, Z)[n & 1] of pair n / 2 = jk, ik (, ji); mixed
-		 * spin: rows (jk + b) vb, same spin: jk + b v, v = vb */
-		const ER *G = (const ER *)(same ? p.epi.GA : p.epi.GB);
-		const ER *Z = (const ER *)(same ? p.epi.ZA : p.epi.ZB);
-		const int64_t po = same ? p.oa : p.ob;
-		const int64_t pr = same ? p.va * p.va : p.va;
-		const int64_t pjk = ((int64_t)j * po + k) * pr;
-		const int64_t pik = ((int64_t)i * po + k) * pr;
-		const int64_t pji = ((int64_t)j * p.oa + i) * pr;
 #pragma unroll
 		for (int q = 0; q < NBC / NT; ++q) {
 			const int n = tid + q * NT;
@@ -991,19 +1001,29 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 			const int b = B0 + bl < na ? B0 + bl : na - 1;
 			const int c = C0 + cl < nc ? C0 + cl : nc - 1;
 			const int64_t pb = arr < 2 ? pjk : arr < 4 ? pik : pji;
-			const int64_t row = same ? pb + (int64_t)b * p.vb :
-			    (pb + b) * p.vb;
-			stg[n] = ((arr & 1) ? Z : G)[row + c];
+			stg[n] = ((arr & 1) ? Z : G)[pb + (int64_t)b * p.vb + c];
 		}
 		/* vector n: (u, f)[n & 1] at occupied index (i, j, k)[n / 2], the
-		 * last one d1 at j */
-		if (tid < NBV) {
-			const int arr = tid / 32, bl = tid % 32;
-			const int b = B0 + bl < na ? B0 + bl : na - 1;
-			const int occ = arr < 2 ? i : arr < 4 || arr == NPB ? j : k;
-			const ER *src = arr == NPB ? (const ER *)p.epi.d1 :
-			    (arr & 1) ? (const ER *)p.epi.f1 : (const ER *)p.epi.u1;
-			stg[NBC + tid] = src[occ * p.va + b];
+		 * last one d1 */
+		const ER *u1 = (const ER *)p.epi.u1, *u2 = (const ER *)p.epi.u2;
+		const ER *f1 = (const ER *)p.epi.f1, *f2 = (const ER *)p.epi.f2;
+		const ER *d1 = (const ER *)p.epi.d1, *d2 = (const ER *)p.epi.d2;
+		for (int n = tid; n < 2 * NBV + NCV; n += NT) {
+			const bool of_c = n >= 2 * NBV, of_a = !of_c && n >= NBV;
+			const int m = of_c ? n - 2 * NBV : of_a ? n - NBV : n;
+			const int arr = of_c ? m / TC : m / 32;
+			const int l = of_c ? C0 + m % TC : (of_a ? A0 + 0 : B0 + 0) +
+			    m % 32;
+			const int top = (of_c ? nc - 1 : na - 1), x = l < top ? l : top;
+			const int64_t d1r = of_c ? k + 0 : of_a ? i + 0 : j + 0;
+			const int64_t r1 = arr < 2 ? i + 0 : arr < 4 ? j + 0 : k + 0;
+			const ER *src = (arr & 1) ? f1 + r1 * p.va : u1 + r1 * p.va;
+			if (arr == NPB)
+				src = d1 + d1r * p.va;
+			if (!same && of_c)
+				src = (arr == 0 ? u2 + 0 : arr == 1 ? f2 + 0 : d2 + 0) +
+				    (int64_t)k * p.vb;
+			stg[NBC + n] = src[x];
 		}
 	}
 	if constexpr (!same) {
@@ -1015,39 +1035,86 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 			const int arr = n / 1024, bl = (n / 32) % 32, al = n % 32;
 			const int b = B0 + bl < na ? B0 + bl : na - 1;
 			const int a = A0 + al < na ? A0 + al : na - 1;
-			stg[NBC + NBV + n] = (arr ? ZA : GA)[(ji + b) * p.va + a];
+			sab[n] = (arr ? ZA : GA)[(ji + b) * p.va + a];
 		}
 	}
+	/* row of a lane group in (a block, register) */
+	auto row_a = [&](int ab, int r, int g) {
+		return 16 * ab + (FM::ROW_F64 ? g + 4 * r : 4 * g + r);
+	};
+	/* same spin: the wave's (b, a) values of (a block, register) */
+	constexpr int NCV1 = same ? (NCOL + 63) / 64 : 1;
+	ER cv[NCV1];
+	ER *const scol = sab + wave * NCOL;
+	const ER *cp[NCV1];   /* at a = 0 */
+#pragma unroll
+	for (int q = 0; q < NCV1; ++q) {
+		const int m = lane + 64 * q, y = m / 8 % BW;
+		const int b = B0 + NW * y + wave;
+		const int64_t rb = (int64_t)(b < na ? b : na - 1) * p.vb;
+		const int64_t r0 = rb + pjk, r1 = rb + pik, r2 = rb + pji;
+		const int64_t e = m < 8 * BW ? r0 : m < 16 * BW ? r1 : r2;
+		cp[q] = ((m & 4) ? Z : G) + e;
+		cv[q] = 0;
+	}
+	/* (a, c) values of a column, [G, Z] for jk, ik (, ji) */
+	ER ac[NPB];
+	auto load_ac = [&](int ab, int r, int cb)
+	    __attribute__((always_inline)) {
+		const int a = A0 + row_a(ab, r, lg), c = C0 + 16 * cb + ln;
+		const int64_t e = (int64_t)(a < na ? a : na - 1) * p.vb +
+		    (c < nc ? c : nc - 1);
+#pragma unroll
+		for (int q = 0; q < NPB; ++q)
+			ac[q] = ((q & 1) ? Z : G)[(q < 2 ? pjk : q < 4 ? pik : pji) + e];
+	};
 	__syncthreads();
 #pragma unroll
-	for (int ab = 0; ab < 2; ++ab)
+	for (int n = -1; n < 8; ++n) {
+		const int ab = n >> 2, r = n & 3;
+		if constexpr (same) {
+			if (n >= 0)
 #pragma unroll
-	for (int r = 0; r < 4; ++r)
+				for (int q = 0; q < NCV1; ++q)
+					if (lane + 64 * q < NCOL)
+						scol[lane + 64 * q] = cv[q];
+			if (n < 7) {
+				const int a = A0 + row_a((n + 1) >> 2, (n + 1) & 3, lane & 3);
 #pragma unroll
-	for (int cb = 0; cb < NCB; ++cb) {
-		uint32_t col = 0;
-#pragma unroll
-		for (int y = 0; y < BW; ++y)
-			col |= 1u << GM::blk2(y, ab, cb);
-		if (!(m2 & col))
+				for (int q = 0; q < NCV1; ++q)
+					cv[q] = cp[q][a < na ? a : na - 1];
+			}
+		}
+		if (n < 0)
 			continue;
 #pragma unroll
-		for (int y = 0; y < BW; ++y) {
-			const int x = GM::blk2(y, ab, cb);
-			E[y * 64] = acc[x][r];
-			if (NSET == 2)
-				E[(BW + y) * 64] = bload_ae<AE>(wr, wvo,
-				    (r * NACC + x) * WST);
+		for (int cb = 0; cb < NCB; ++cb) {
+			uint32_t col = 0;
+#pragma unroll
+			for (int y = 0; y < BW; ++y)
+				col |= 1u << GM::blk2(y, ab, cb);
+			if (!(m2 & col))
+				continue;
+			load_ac(ab, r, cb);
+#pragma unroll
+			for (int y = 0; y < BW; ++y) {
+				const int x = GM::blk2(y, ab, cb);
+				E[y * 64] = acc[x][r];
+				if (NSET == 2)
+					E[(BW + y) * 64] = bload_ae<AE>(wr, wvo,
+					    (r * NACC + x) * WST);
+			}
+			const int al = row_a(ab, r, lg);
+			const int a = A0 + al, c = C0 + 16 * cb + ln;
+			if (a < na && c < nc)
+				epi_block<F, KIND, NSET, BW, NW, TC>(p, a, c, B0 + wave, E,
+				    ac, sva + al, sbv, svc + 16 * cb + ln, sbc + 16 * cb,
+				    same ? scol + lg : sab + wave * 32 + al, esum, ecmp);
 		}
-		const int al = 16 * ab + (FM::ROW_F64 ? (lg + 4 * r) : (4 * lg + r));
-		const int a = A0 + al, c = C0 + 16 * cb + ln;
-		if (a < na && c < nc)
-			epi_block<F, KIND, NSET, BW, NW, TC>(p, i, j, k, a, c,
-			    B0 + wave, E, sbc + 16 * cb, sba + al, sbv, esum, ecmp);
 	}
 
 	/* deterministic workgroup reduction */
-	double e = esum - ecmp;
+	double e = (esum[0] - ecmp[0]) + (esum[1] - ecmp[1]);
 #pragma unroll
 	for (int off = 32; off >= 1; off >>= 1)
 		e += __shfl_xor(e, off);
