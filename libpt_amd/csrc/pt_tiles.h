@@ -211,8 +211,9 @@ kahan(double &s, double &cmp, double x)
 /*
  * Energy terms of one lane's NB elements (a, b0 + BS y, c), y = 0 .. NB-1,
  * in y order, even y added to (esum, ecmp)[0], odd ones to [1]: the
- * disconnected term Z, the denominator Dn = d_ia + d_jb + d_kc and W (W - Z) / Dn, or for two W sets
- * (W_L - Z) W_R / Dn (src/pt.c:700,927).  Everything comes from registers
+ * disconnected term Z, the denominator Dn = d_ia + d_jb + d_kc and
+ * W (W - Z) / Dn, or for two W sets (W_L - Z) W_R / Dn
+ * (src/pt.c:700,927).  Everything comes from registers
  * and LDS; every element's values are made whether or not the triangle keeps
  * it, and only the sum is masked.  W values: ew[64 y] (one set; the right
  * set with two) and ew[64 (y + NB)] (the left set).  ac: the (a, c) values
