@@ -61,11 +61,13 @@ double libpt_amd_energy(int call, int form, size_t oa, size_t va, size_t ob,
  * returned, NaN on error (libpt_amd_last_error says why).  The call
  * allocates nothing: every buffer it needs (packed and split operands,
  * work lists, per-item energies, (fT) save areas) comes from one static
- * device array of LIBPT_AMD_NOALLOC_SCRATCH bytes per GPU, which each GPU
- * the library runs on holds until the process ends.  A call whose
- * buffers do not fit is rejected with an error (FP64 restricted (T) fits
- * up to about o=10, v=120).  Calls on one GPU share the array: overlapping
- * calls would race on it, so the library runs them one at a time. */
+ * device array per GPU (1792 MiB), which each GPU the library runs on
+ * holds until the process ends.  A call whose buffers, counted without
+ * the rows' padding and the transposed copies, exceed
+ * LIBPT_AMD_NOALLOC_SCRATCH bytes is rejected with an error (FP64
+ * restricted (T) fits up to about o=10, v=120).  Calls on one GPU share
+ * the array: overlapping calls would race on it, so the library runs them
+ * one at a time. */
 #define LIBPT_AMD_NOALLOC_SCRATCH ((size_t)256 << 20)
 double libpt_amd_energy_noalloc(int call, int form, size_t oa, size_t va,
     size_t ob, size_t vb, const void *const *dev_arrays, void *stream);
@@ -148,7 +150,8 @@ typedef struct libpt_amd_batch libpt_amd_batch;
  * read oa, va); dev_arrays[NA s + t] = its t-th pt.h array in device memory
  * (NA = 7 for rpt/upt, 10 for rft/uft).  Stages every system's operands
  * and records one graph: the tile launches of every (system, spin case)
- * in one chain, largest items first, then one reduction per spin case.
+ * in one chain, largest items first (small ones share a launch), then one
+ * reduction per spin case.
  * NULL on error. */
 libpt_amd_batch *libpt_amd_batch_create(int call, int form, int n,
     const int64_t *dims, const void *const *dev_arrays);

@@ -1849,12 +1849,11 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	}
 
 	/*
-	 * The graph: each segment's items as launches of the spin case's own
-	 * tile kernel (the one plans use), largest items first, in one chain,
-	 * then the batched reduction.  Every launch of a system of this size
-	 * range fills the GPU by itself: two concurrent branches (launches
-	 * dealt by accumulated cost) were measured 2-3 % slower than the chain,
-	 * which runs at the speed of the plans run one after another.
+	 * The graph: each segment's items as the tile launches a plan would
+	 * make, largest items first, in one chain, then the batched reduction.
+	 * Small neighbouring segments share launches (launch_runs); every
+	 * other one fills the GPU by itself, and two concurrent branches were
+	 * slower than the chain.
 	 */
 	BFAIL(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) ==
 	    hipSuccess || (set_err("stream capture failed"), false));

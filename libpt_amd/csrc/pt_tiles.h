@@ -26,18 +26,21 @@
  * a fragment is one coalesced 16-byte load per lane, and since each wave
  * owns its own w (c in phase 1, b in phase 2) and the full range of the
  * other two indices, every Q fragment of a tile is loaded by exactly one
- * wave and used by both 16-row blocks of S.  There is nothing to share
- * through LDS, hence no barrier in the step loop: the two waves of a SIMD
- * drift apart and fill each other's waits, and each fragment register is
- * reloaded for the next step soon after its MFMAs.
- * Against the kernel that staged the operands in LDS (two slots, a barrier
- * per step, one wave per 16 a x 16 b x TC c): MFMA pipe 84 % busy instead of
- * 67 % at rpt v=477 in FP64, where the card's clock then falls from 2.2 to
- * 1.95 GHz (a share of the triples: 289 -> 270 ms); rpt o=20 v=120 331 ->
- * 239 ms, FP32 upt 24/200/20/204 292 -> 196 ms, split-BF16 rpt v=477 253 ->
- * 233 ms, a batch of 8 systems of v 40 to 160 198 -> 120 ms.  Bound by the
- * MFMA pipe and power in FP64 and FP32, by L2 and HBM bandwidth in the split
- * forms.
+ * wave and used by both 16-row blocks of S: there is nothing in Q to share
+ * through LDS.  FP64 and FP32 load S the same way and have no barrier in the
+ * step loop (the two waves of a SIMD drift apart and fill each other's
+ * waits); the split forms stage S in LDS panels, a barrier per eight steps.
+ * Each fragment register is reloaded for the next step soon after its MFMAs.
+ *   Against the kernel that staged all operands in LDS (two slots, a barrier
+ * per step, one wave per 16 a x 16 b x TC c), with the launch order and the
+ * later changes noted below: MFMA pipe 84 % busy instead of 67 % at rpt v=477
+ * in FP64, where the card's clock then falls from 2.2 to about 2 GHz (a share of
+ * the triples: 292 -> 245 ms); rpt o=20 v=120 331 -> 211 ms with 11 ms of
+ * copies, FP32 upt 24/200/20/204 292 -> 184 ms, split BF16 rpt v=477 258 ->
+ * 163 ms, a batch of 8 systems of v 40 to 160 198 -> 120 ms.  Bound by the
+ * MFMA pipe and power in FP64 and FP32, by L1, L2 and HBM bandwidth in the
+ * split forms (a wave's 16 KB of Q per 1024 MFMA cycles is the 64 bytes per
+ * clock that a CU's L1 gives).
  *
  * Forms: FP64 (v_mfma_f64_16x16x4_f64), FP32 (v_mfma_f32_16x16x4_f32),
  * split BF16 / FP16 (hi+lo pairs, hi*hi + lo*hi + hi*lo packed into the
