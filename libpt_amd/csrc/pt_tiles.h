@@ -1199,9 +1199,10 @@ k_tiles(pt_launch p)
  * 12.7 -> 12.3 and 28.9 -> 28.6, v=400 23.1 -> 22.1 and 50.8 -> 50.3, v=477
  * 46.6 -> 41.2 and 94.8 -> 93.6, v=600 134 -> 101 and 238 -> 230; two W sets
  * (rft F16X3) v=256 9.1 -> 9.5 and 20.6 -> 21.3, v=350 30.3 -> 30.1 and 76.6
- * -> 76.5, v=400 56.0 -> 51.6 and 133 -> 134.  At v=8 to 200 pairs cost 2 to
- * 25 %, and FP64 and FP32 (no barriers to keep two workgroups together or
- * apart) 2 to 20 % there and 4 % at v=477.
+ * -> 76.5, v=400 56.0 -> 51.6 and 133 -> 134.  Launches of one to eight ijk
+ * share fewer slabs: from 8 % slower to 20 % faster at v=384 to 600, without
+ * a trend.  At v=48 to 200 pairs cost up to 25 %, and FP64 and FP32 lose by
+ * them (FP64 2 to 20 % at v=64 to 200 and 4 % at v=477, FP32 up to 16 %).
  */
 constexpr int PAIR_NA = 384;
 
