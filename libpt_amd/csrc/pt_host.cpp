@@ -324,6 +324,7 @@ struct libpt_amd_plan {
 	bool no_room = false;       /* an allocation did not fit */
 	bool persist = false;       /* persistent grid (LIBPT_AMD_PERSISTENT) */
 	uint32_t *d_ctr = nullptr;  /* its 8 item counters */
+	std::mutex run_mu;          /* held over the launches of one range */
 	int64_t oa = 0, va = 0, ob = 0, vb = 0;
 	hipStream_t stream = nullptr;
 	bool own_stream = true;     /* created (and destroyed) by the plan */
@@ -1421,6 +1422,10 @@ libpt_amd_plan_run(libpt_amd_plan *pl, int sc, int64_t b, int64_t e)
 		e = c.n_ijk;
 	if (e <= b)
 		return 0;
+	/* The launches of a range go to the stream together: its launch order
+	 * (d_part), the save areas and the persistent grid's counters are the
+	 * plan's, and another thread's range may be on its way. */
+	std::lock_guard<std::mutex> lk(pl->run_mu);
 	if (c.L.nset == 2 && !plan_wsave(pl))
 		return -1;
 	/* a range of more than one group goes in the whole list's launch order

@@ -72,3 +72,38 @@ def test_error_text_is_per_thread():
     t.join(timeout=60)
     assert "form" in got.get("bad", "")
     assert api.last_error() == ""
+
+
+def test_ranges_of_one_plan_from_two_threads():
+    """Two threads run disjoint ranges of one plan, each of more than a
+    group of 32 ijk: a range's launches stay together, so the per-ijk
+    energies are those of one thread."""
+    spec = api.make_spec("rpt", (9, 33), seed=2, sig_f=1e-2)
+    dev = api.synth_device("rpt", spec)
+    errs = []
+    try:
+        with api.Plan("rpt", "fp64", (9, 33), dev) as pl:
+            pl.run_all()
+            ref = [pl.ijk_energies(sc) for sc in range(pl.ncases)]
+        with api.Plan("rpt", "fp64", (9, 33), dev) as pl:
+            def work(first):
+                try:
+                    for sc in range(pl.ncases):
+                        n = pl.nijk(sc)
+                        for q in range(first, 4, 2):
+                            pl.run(sc, n * q // 4, n * (q + 1) // 4)
+                except Exception as exc:  # reported by the main thread
+                    errs.append(repr(exc))
+
+            threads = [threading.Thread(target=work, args=(f,))
+                       for f in range(2)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join(timeout=60)
+            assert not errs, errs
+            got = [pl.ijk_energies(sc) for sc in range(pl.ncases)]
+    finally:
+        dev.close()
+    for a, b in zip(ref, got):
+        assert np.array_equal(a, b)
