@@ -52,6 +52,14 @@ set_err(const char *fmt, ...)
 	va_end(ap);
 }
 
+/* the error text from before an attempt that may be made again another way;
+ * back() after the attempt, whose failure is then none of the caller's */
+struct ErrText {
+	char was[sizeof(g_err)];
+	ErrText() { memcpy(was, g_err, sizeof(was)); }
+	void back() { memcpy(g_err, was, sizeof(was)); }
+};
+
 double
 now_s()
 {
@@ -1227,6 +1235,7 @@ plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 	if (!dev_init())
 		return nullptr;
 	/* without the transposed copies where they leave too little memory */
+	ErrText err;
 	for (int copies = 1; copies >= 0; --copies) {
 		libpt_amd_plan *pl = new libpt_amd_plan;
 		pl->copies = copies != 0;
@@ -1236,6 +1245,7 @@ plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 		plan_free(pl);
 		if (!again)
 			break;
+		err.back();
 	}
 	return nullptr;
 }
@@ -2206,6 +2216,7 @@ pt_noalloc_energy(int call, int form, size_t oa, size_t va, size_t ob,
 	if (!dev_init())
 		return NAN;
 	/* without the transposed copies where they do not fit */
+	ErrText err;
 	for (int copies = 1; copies >= 0; --copies) {
 		Arena ar;
 		ar.base = (char *)scratch;
@@ -2224,6 +2235,7 @@ pt_noalloc_energy(int call, int form, size_t oa, size_t va, size_t ob,
 		plan_release(&pl);
 		if (!again)
 			return e;
+		err.back();
 	}
 	return NAN;
 }

@@ -39,6 +39,14 @@ def lib(tmp_path_factory):
     h.libpt_amd_plan_run.argtypes = [vp, ctypes.c_int, i64, i64]
     h.libpt_amd_plan_ijk_energies.argtypes = [vp, ctypes.c_int, vp]
     h.libpt_amd_last_error.restype = ctypes.c_char_p
+    h.pt_noalloc_energy.restype = ctypes.c_double
+    h.pt_noalloc_energy.argtypes = ([ctypes.c_int] * 2 + [sz] * 4 +
+                                    [vp, vp, sz, vp])
+    h.libpt_rpt.restype = ctypes.c_double
+    h.libpt_rpt.argtypes = [sz] * 2 + [vp] * 7
+    h.fake_region.restype = vp
+    h.fake_region.argtypes = [sz]
+    h.fake_region_free.argtypes = [vp, sz]
     h.fake_count.restype = ctypes.c_long
     h.fake_limit.argtypes = [sz]
     yield h
@@ -59,6 +67,93 @@ def _ijk(lib, plan, sc):
     e = np.zeros(lib.libpt_amd_plan_nijk(plan, sc))
     assert lib.libpt_amd_plan_ijk_energies(plan, sc, e.ctypes.data) == 0
     return e
+
+
+@pytest.fixture
+def region(lib):
+    """1 GiB of scratch for the allocation-free call"""
+    size = 1 << 30
+    p = lib.fake_region(size)
+    yield p, size
+    lib.fake_region_free(p, size)
+
+
+def _noalloc(lib, call, form, dims, scratch, cap):
+    dims = tuple(dims) + (0,) * (4 - len(dims))
+    lib.pt_set_error(None)
+    return lib.pt_noalloc_energy(call, form, *dims, _arrays(), scratch, cap,
+                                 None)
+
+
+def _expected(lib, dims):
+    """the restricted energy of the stand-in: 2 (n (n + 1) / 2) per case"""
+    o = dims[0]
+    n = (o * (o - 1) * (o - 2) // 6, o * (o - 1) // 2 * o)
+    return float(sum(x * (x + 1) for x in n))
+
+
+def test_plan_without_room_for_the_copies(lib):
+    """With less memory than the transposed copies take, the plan is made
+    without them, gives the same energies and leaves no error text."""
+    dims = (6, 40)
+    lib.fake_limit(1 << 40)
+    base = lib.fake_count(0)
+    full = _plan(lib, RPT, FP64, dims)
+    ref = [_ijk(lib, full, 0), _ijk(lib, full, 1)]
+    size = lib.fake_count(0) - base
+    lib.libpt_amd_plan_destroy(full)
+    before = lib.libpt_amd_last_error()
+    lib.fake_limit(base + size - 1)
+    plan = _plan(lib, RPT, FP64, dims)
+    lib.fake_limit(1 << 40)
+    assert plan and lib.fake_count(0) - base < 0.8 * size
+    assert lib.libpt_amd_last_error() == before
+    assert [lib.libpt_amd_plan_run(plan, sc, 0, len(e))
+            for sc, e in enumerate(ref)] == [0, 0]
+    for sc, e in enumerate(ref):
+        assert np.array_equal(_ijk(lib, plan, sc), 1.0 + np.arange(len(e)))
+    lib.libpt_amd_plan_destroy(plan)
+    assert lib.fake_count(0) == base
+
+
+def test_drop_in_call_without_room_for_the_copies(lib):
+    """The same through pt.h, with an energy that is NaN (inputs of the
+    caller): it is returned, and no allocation error ends the program."""
+    o, v = 4, 30
+    n = [o * v] * 3 + [2 * o * o * v * v, 2 * o * o * v * o,
+                       2 * o * o * v * v,
+                       o * v * (v * (v - 1) // 2) + o * v * v * v]
+    arr = [np.zeros(k) for k in n]
+    ptr = [a.ctypes.data for a in arr]
+    base = lib.fake_count(0)
+    lib.fake_limit(1 << 40)
+    assert lib.libpt_rpt(o, v, *ptr) == _expected(lib, (o, v))
+    peak = lib.fake_count(1)
+    for nan in (0, 1):
+        lib.fake_nan(nan)
+        lib.fake_limit(peak - 1)
+        e = lib.libpt_rpt(o, v, *ptr)
+        lib.fake_limit(1 << 40)
+        lib.fake_nan(0)
+        assert np.isnan(e) if nan else e == _expected(lib, (o, v))
+        assert lib.libpt_amd_last_error() == b""
+    assert lib.fake_count(0) == base
+
+
+def test_scratch_without_room_for_the_copies(lib, region):
+    """The allocation-free call drops the copies where its scratch ends."""
+    dims = (6, 40)
+    copies = lib.fake_count(5)
+    assert _noalloc(lib, RPT, FP64, dims, *region) == _expected(lib, dims)
+    assert lib.fake_count(5) > copies
+    copies = lib.fake_count(5)
+    cap = 8 << 20
+    while _noalloc(lib, RPT, FP64, dims, region[0], cap) != _expected(lib,
+                                                                      dims):
+        assert b"scratch" in lib.libpt_amd_last_error()
+        cap += 1 << 20
+    assert lib.fake_count(5) == copies
+    assert lib.libpt_amd_last_error() == b""
 
 
 def test_ranges_of_one_plan_from_two_threads(lib):
