@@ -1038,12 +1038,14 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 	 * mixed ovvv blocks as the mixed-spin case reads its VC operand
 	 * (VC[k, d, c, b] with (u, w) = (b or a, c)) */
 	Blocks qT[2] = {}, qV[2] = {}, qTt[2] = {}, qVt[2] = {};
-	/* blocks that a spin case with any triples reads */
+	/* the blocks that a spin case with any triples reads: its pair spin's
+	 * own block, the mixed block as it is (mixB) and the other one
+	 * transposed (mixC), the own amplitudes transposed in the same-spin case */
 	const bool sa = case_same(oa, va), sb = case_same(ob, vb);
-	const bool mx = case_mixed(oa, va, ob, vb) ||
-	    case_mixed(ob, vb, oa, va);
-	const bool used[4] = {sa || mx, mx, sb || mx, mx};
-	const bool used_t[4] = {sa, mx, sb, mx};   /* transposed */
+	const bool ma = case_mixed(oa, va, ob, vb);
+	const bool mb = case_mixed(ob, vb, oa, va);
+	const bool used[4] = {sa || ma, ma, sb || mb, mb};
+	const bool used_t[4] = {sa, mb, sb, ma};   /* transposed */
 	FixedVec<pt_pack_job, 28> jobs;
 	auto pack = [&](int s, int fam, int b, bool tr, const char **out) {
 		const Geo g = geo(fam, b);
@@ -1073,10 +1075,11 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 			Blocks &q = fam == 0 ? qT[s] : qV[s];
 			Blocks &qt = fam == 0 ? qTt[s] : qVt[s];
 			for (int b = 0; b < nblk; ++b) {
-				if (used[b])
+				const bool t = used_t[b] && (fam == 0 || (b & 1));
+				if (used[b] || (t && !pl->copies))
 					PFAIL(pack(s, fam, b, false, &q.p[b]));
 				qt.p[b] = q.p[b];
-				if (used_t[b] && pl->copies && (fam == 0 || (b & 1)))
+				if (t && pl->copies)
 					PFAIL(pack(s, fam, b, true, &qt.p[b]));
 			}
 			if (restricted) {

@@ -6,6 +6,8 @@
   index skip the blocks outside the triangle and read only fragments that
   exist.  Bounds: FP64 as for the other parity tests; FP32 and the split
   forms by their operand precision (FP32 2^-24, split 2^-16 per product).
+- Open-shell sizes with fewer orbitals than a 16-row block in one spin or
+  both, down to spin cases that do not exist.
 - Without the transposed copies (LIBPT_AMD_VC_TRANSPOSED=0, or too little
   memory for them) the same values come from the plain copies in scattered
   pieces: per-ijk energies are equal bit for bit."""
@@ -44,6 +46,31 @@ def test_tile_edges_match_the_oracle(dims, form):
         dev.close()
     print(dims, form, e, eo)
     assert abs(e - eo) <= TOL[form] * abs(eo)
+
+
+# energies of a few 1e-5 to 1e-1, summed from terms of both signs: the bounds
+# above, on the sum of the per-ijk energies' sizes
+@pytest.mark.parametrize("form", ["fp64", "fp32", "bf16x3", "f16x3"])
+@pytest.mark.parametrize("copies", ["1", "0"])
+@pytest.mark.parametrize("kind,dims", [
+    ("upt", (2, 2, 5, 1)), ("upt", (3, 1, 4, 3)), ("upt", (1, 5, 4, 6)),
+    ("uft", (5, 17, 2, 1)), ("uft", (3, 1, 5, 2)), ("upt", (3, 3, 4, 2)),
+    ("uft", (4, 7, 3, 9)), ("upt", (3, 15, 4, 8)), ("uft", (3, 9, 3, 16)),
+    ("upt", (6, 4, 2, 21))])
+def test_few_orbitals_match_the_oracle(kind, dims, copies, form, monkeypatch):
+    monkeypatch.setenv("LIBPT_AMD_VC_TRANSPOSED", copies)
+    spec = api.make_spec(kind, dims, seed=sum(dims), sig_f=1e-2,
+                         omega=0.3 if kind == "uft" else 0.0)
+    arr = api.synth_host(kind, spec)
+    eo = oracle.energy(kind, dims, arr, mp=form == "fp32")
+    dev = api.to_device(kind, arr, fp32=form == "fp32")
+    try:
+        e, ijk = _energy(kind, form, dims, dev)
+    finally:
+        dev.close()
+    size = sum(float(np.sum(np.abs(x))) for x in ijk)
+    print(kind, dims, form, copies, e, eo, size)
+    assert abs(e - eo) <= TOL[form] * size
 
 
 @pytest.mark.parametrize("form", ["fp64", "fp32", "bf16x3", "f16x3"])

@@ -156,6 +156,21 @@ def test_scratch_without_room_for_the_copies(lib, region):
     assert lib.libpt_amd_last_error() == b""
 
 
+@pytest.mark.parametrize("call,dims,plain,transposed", [
+    (RPT, (4, 5), 4, 3), (RPT, (2, 5), 4, 2), (UPT, (4, 5, 3, 6), 8, 6),
+    # no case reads the second spin's own blocks: its pairs have no orbitals
+    (UPT, (2, 2, 50, 1), 4, 2), (UPT, (1, 5, 4, 6), 4, 3),
+    (UPT, (2, 1, 1, 5), 0, 0), (UFT, (4, 5, 1, 1), 8, 6)])
+def test_only_blocks_that_a_case_reads_are_packed(lib, call, dims, plain,
+                                                  transposed):
+    a, b = lib.fake_count(4), lib.fake_count(5)
+    plan = _plan(lib, call, FP64, dims)
+    assert plan
+    lib.libpt_amd_plan_destroy(plan)
+    assert (lib.fake_count(4) - a, lib.fake_count(5) - b) == (plain,
+                                                              transposed)
+
+
 def test_ranges_of_one_plan_from_two_threads(lib):
     """Both threads make the launch order of their range before either runs
     its tiles, unless a range is one unit."""
