@@ -61,7 +61,7 @@ double libpt_amd_energy(int call, int form, size_t oa, size_t va, size_t ob,
  * returned, NaN on error (libpt_amd_last_error says why).  The call
  * allocates nothing: every buffer it needs (packed and split operands,
  * work lists, per-item energies, (fT) save areas) comes from one static
- * device array per GPU (1792 MiB), which each GPU the library runs on
+ * device array per GPU (1 GiB), which each GPU the library runs on
  * holds until the process ends.  A call whose buffers, counted without
  * the rows' padding and the transposed copies, exceed
  * LIBPT_AMD_NOALLOC_SCRATCH bytes is rejected with an error (FP64

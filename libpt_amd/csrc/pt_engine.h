@@ -39,8 +39,16 @@ enum pt_role { PT_ROLE_A = 0, PT_ROLE_B = 1, PT_ROLE_C = 2 };
 /* kappa per fragment of the packed Q operands: a fragment is 1 KB, 16 rows
  * of 64 bytes (8 FP64, 16 FP32, or 16 split values: per 4 kappa hi 0-3 and
  * lo 0-3), in the lane order of the MFMA operand: lane 16 g + row holds
- * the row's g-th quarter */
+ * the row's g-th quarter.  The fragments of a plane of 1, 2, 4 or 8 rows
+ * (rounded up) hold only these: quarter g of a row at 16 (rows g + row).  A
+ * spin of two orbitals would else pad eightfold. */
 #define PT_FRAG 1024
+static inline int
+pt_frag_rows(int64_t rows)
+{
+	return rows > 8 ? 16 : rows > 4 ? 8 : rows > 2 ? 4 : rows > 1 ? 2 : 1;
+}
+
 static inline int
 pt_kc(int form)
 {
@@ -54,14 +62,15 @@ pt_chunks(int form, int64_t K)
 	return (K + pt_kc(form) - 1) / pt_kc(form);
 }
 
-/* fragments of a packed slab [row block of 16][chunk][column]: rows and
- * columns of the plane; tri: the pairs row > column of a square plane,
+/* bytes of a packed slab [row block of 16][chunk][column] of fragments: rows
+ * and columns of the plane; tri: the pairs row > column of a square plane,
  * block b holding its columns 0 .. 16 (b + 1) - 1 */
 static inline int64_t
-pt_slab_frags(int form, int64_t K, int64_t rows, int64_t cols, int tri)
+pt_slab_bytes(int form, int64_t K, int64_t rows, int64_t cols, int tri)
 {
 	const int64_t nb = (rows + 15) / 16;
-	return pt_chunks(form, K) * (tri ? 8 * nb * (nb + 1) : nb * cols);
+	return pt_chunks(form, K) * (tri ? 8 * nb * (nb + 1) : nb * cols) *
+	    (PT_FRAG / 16 * pt_frag_rows(rows));
 }
 
 /* Workgroup geometry (the kernel's Geo): NW = 4 waves, tile 32 a x 32 b x
@@ -110,9 +119,9 @@ struct pt_term {
 	int32_t s_buf, q_buf;
 	int32_t role, set, sign, K;
 	int32_t nch;       /* kappa chunks */
-	int32_t tri;       /* packed triangle u > w (pt_slab_frags) */
+	int32_t tri;       /* packed triangle u > w (pt_slab_bytes) */
 	int32_t tr;
-	int32_t pad_;
+	int32_t fr;        /* rows of a fragment (pt_frag_rows) */
 };
 
 /* terms of one W set of a spin case */
@@ -207,17 +216,17 @@ int pt_launch_segsum(const double *x, int64_t nseg, int64_t seglen,
     double *out, void *stream);
 int pt_launch_split(const double *src, uint32_t *dst, int64_t n, int fp16,
     double scale, void *stream);
-/* [R slabs][K][plane] -> packed slabs (pt_slab_frags) of the plane's rows
+/* [R slabs][K][plane] -> packed slabs (pt_slab_bytes) of the plane's rows
  * and columns; the source plane is [rows][cols], [cols][rows] (tr), or the
  * packed pairs row > column (tri); the split forms store hi and lo of
- * x * scale.  at: set by the launch. */
+ * x * scale.  at, fr: set by the launch. */
 struct pt_pack_job {
 	const char *src;
 	char *dst;
 	int64_t R, K, rows, cols;
 	double scale;
 	int64_t at;
-	int32_t tri, tr;
+	int32_t tri, tr, fr;
 };
 int pt_launch_pack(const struct pt_pack_job *jobs, int n, int form,
     void *stream);
@@ -228,6 +237,17 @@ int pt_launch_absmax(const double *src, int64_t n, double *out, void *stream);
 int pt_launch_copy(const double *src, double *dst, int64_t n, void *stream);
 int pt_launch_synth(const void *spec, int tensor, void *dst, int64_t n,
     int fp32, void *stream);
+
+/* bytes of the allocation-free call's static array.  LIBPT_AMD_NOALLOC_SCRATCH
+ * of them decide which calls are taken; the packed rows' padding (to 16, or to
+ * a power of two below) brings those to at most 496 MiB, for 13 and 17
+ * virtual orbitals.  The rest is room for the transposed copies (with them
+ * the largest call takes 887 MiB) and for (fT) save areas: a launch holds as
+ * many items as there are areas, and the copies are left out where fewer than
+ * PT_NOALLOC_AREAS, eight rounds of workgroups, would remain (uft 5/17/198/17
+ * FP64, whose copies leave 1100: 2.58 s with them, 2.26 s without) */
+#define PT_NOALLOC_ARENA ((size_t)1 << 30)
+#define PT_NOALLOC_AREAS 4096
 
 /* host engine (pt_host.cpp) for pt_noalloc.hip: the device every call
  * runs on (made current; -1 on error), the calling thread's error text

@@ -447,8 +447,7 @@ plan_alloc(libpt_amd_plan *pl, void **p, size_t bytes)
 		if (need > a.cap - a.used) {
 			set_err("the call needs more than the %zu bytes of static "
 			    "scratch of the allocation-free entry point (%zu in use, "
-			    "%zu more requested)", (size_t)LIBPT_AMD_NOALLOC_SCRATCH,
-			    a.used, need);
+			    "%zu more requested)", a.cap, a.used, need);
 			pl->no_room = true;
 			return false;
 		}
@@ -816,6 +815,13 @@ plan_wsave(libpt_amd_plan *pl)
 		/* what the scratch has left, in whole areas: launches then hold
 		 * fewer items */
 		const int64_t left = (int64_t)(pl->arena->cap - pl->arena->used) / wb;
+		if (pl->copies && left < std::min<int64_t>(slots,
+		    PT_NOALLOC_AREAS)) {
+			set_err("the transposed copies leave the static scratch only "
+			    "%lld save areas", (long long)left);
+			pl->no_room = true;
+			return false;
+		}
 		slots = std::min(slots, left > 0 ? left : 1);
 	}
 	if (!plan_alloc(pl, &pl->wsave, (size_t)slots * (size_t)wb))
@@ -936,8 +942,8 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		    (set_err("hipEventCreate failed"), false));
 	}
 	if (pl->arena && noalloc_need(*pl) > (int64_t)LIBPT_AMD_NOALLOC_SCRATCH) {
-		set_err("the call needs more than the %zu bytes of static scratch of "
-		    "the allocation-free entry point (%lld)",
+		set_err("the call needs more than the %zu bytes of static scratch "
+		    "that the allocation-free entry point allows (%lld)",
 		    (size_t)LIBPT_AMD_NOALLOC_SCRATCH, (long long)noalloc_need(*pl));
 		return false;
 	}
@@ -1053,8 +1059,8 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 		const int64_t cols = tr ? g.rows : g.cols;
 		const int api = fam == 0 ? famT[s] : famV[s];
 		void *dst;
-		if (!plan_alloc(pl, &dst, (size_t)(g.R * pt_slab_frags(form, g.K,
-		    rows, cols, g.tri)) * PT_FRAG))
+		if (!plan_alloc(pl, &dst, (size_t)(g.R * pt_slab_bytes(form, g.K,
+		    rows, cols, g.tri))))
 			return false;
 		pt_pack_job j = {};
 		j.src = (const char *)arr[api] + esz * (size_t)g.off;
@@ -2150,7 +2156,7 @@ namespace {
  * of their arrays with kappa padded to whole chunks, the lists, energies
  * and term tables, and one (fT) save area.  The packed rows' padding, the
  * transposed copies and the launch order come on top of it, out of the rest
- * of the static array. */
+ * of the static array (PT_NOALLOC_ARENA). */
 int64_t
 noalloc_need(const libpt_amd_plan &pl)
 {

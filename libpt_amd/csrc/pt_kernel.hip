@@ -91,12 +91,13 @@ split2(double x, int fp16, uint16_t &hb, uint16_t &lb)
 }
 
 /*
- * Operand packing (pt_slab_frags): one launch for all operands of a plan;
+ * Operand packing (pt_slab_bytes): one launch for all operands of a plan;
  * one workgroup makes the fragments of one (slab, row block, kappa chunk) of
  * a job for PACK_COLS columns.  It reads the plane along its contiguous index
  * (columns, or rows with tr), PACK_BATCH loads at a time, lays the fragments
- * out in LDS and writes them as whole 1 KB runs; rows and kappa beyond the
- * extents, and tri pairs with column >= row, are zero.  Bound by HBM (each
+ * out in LDS and writes them as whole 1 KB runs (64 bytes for each of the
+ * fr rows that the fragments of a plane below 16 rows hold); rows and kappa
+ * beyond the extents, and tri pairs with column >= row, are zero.  Bound by HBM (each
  * element read once and written once) or, in small plans, by the launch and
  * one load latency per batch.
  */
@@ -186,12 +187,15 @@ k_pack(pack_args args)
 	const int64_t f0 = tri ? nch * (r * 8 * nrb * (nrb + 1) +
 	    8 * (int64_t)rb * (rb + 1)) + ch * bcols + c0 :
 	    ((r * nrb + rb) * nch + ch) * cols + c0;
-	for (int n = tid; n < 64 * PACK_COLS; n += 256) {
-		const int col = n / 64, l = n % 64;
+	const int frs = 31 - __clz(J.fr), fb = 64 << frs;
+	for (int n = tid; n < (4 * PACK_COLS) << frs; n += 256) {
+		const int col = n >> (frs + 2), l = n & ((4 << frs) - 1);
 		if (c0 + col >= bcols)
 			break;
-		const uint64_t *s8 = (const uint64_t *)(lds + col * FS + 16 * l);
-		uint64_t *d8 = (uint64_t *)(J.dst + (f0 + col) * PT_FRAG + 16 * l);
+		const int row = l & (J.fr - 1);
+		const uint64_t *s8 = (const uint64_t *)(lds + col * FS +
+		    16 * (16 * (l >> frs) + row));
+		uint64_t *d8 = (uint64_t *)(J.dst + (f0 + col) * fb + 16 * l);
 		d8[0] = s8[0];
 		d8[1] = s8[1];
 	}
@@ -395,8 +399,7 @@ pt_launch_pack(const struct pt_pack_job *jobs, int n, int form, void *stream)
 			return (int)hipErrorInvalidValue;
 		const int64_t pl = j.tri ? j.rows * (j.rows - 1) / 2 :
 		    j.rows * j.cols;
-		const int64_t slab = pt_slab_frags(form, j.K, j.rows, j.cols, j.tri) *
-		    PT_FRAG;
+		const int64_t slab = pt_slab_bytes(form, j.K, j.rows, j.cols, j.tri);
 		for (int64_t r = 0; r < j.R;) {
 			if (a.n == PACK_JOBS || MOST - blocks < per) {
 				const int rc = go();
@@ -410,6 +413,7 @@ pt_launch_pack(const struct pt_pack_job *jobs, int n, int form, void *stream)
 			o.src = j.src + r * j.K * pl * el;
 			o.dst = j.dst + r * slab;
 			o.at = blocks;
+			o.fr = pt_frag_rows(j.rows);
 			blocks += per * m;
 			r += m;
 		}

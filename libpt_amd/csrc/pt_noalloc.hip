@@ -25,12 +25,7 @@
 #include "../../include/libpt_amd.h"
 #include "pt_engine.h"
 
-/* LIBPT_AMD_NOALLOC_SCRATCH bytes decide which calls are taken; the rest is
- * what their packed rows' padding to 16 can add (at most to 1.67 GiB, for
- * two virtual orbitals; below 0.5 GiB from 16 on) and, where it is free,
- * room for the transposed copies */
-constexpr size_t ARENA = (size_t)1792 << 20;
-static __device__ __align__(256) unsigned char scratch[ARENA];
+static __device__ __align__(256) unsigned char scratch[PT_NOALLOC_ARENA];
 
 namespace {
 
@@ -68,5 +63,5 @@ libpt_amd_energy_noalloc(int call, int form, size_t oa, size_t va,
 		g_scratch[dev] = ptr;
 	}
 	return pt_noalloc_energy(call, form, oa, va, ob, vb, dev_arrays,
-	    g_scratch[dev], ARENA, stream);
+	    g_scratch[dev], PT_NOALLOC_ARENA, stream);
 }

@@ -51,8 +51,8 @@ struct TermBuilder {
 		t.q_buf = buf;
 		t.tr = tr;
 		t.cols = tr ? nu : nw;
-		t.q_off[o1] = PT_FRAG * pt_slab_frags(form, t.K, tr ? nw : nu,
-		    t.cols, 0);
+		t.fr = pt_frag_rows(tr ? nw : nu);
+		t.q_off[o1] = pt_slab_bytes(form, t.K, tr ? nw : nu, t.cols, 0);
 		return *this;
 	}
 	/* Q: slab o1 of buf, the packed pairs u > w of extent n */
@@ -60,7 +60,8 @@ struct TermBuilder {
 	{
 		t.q_buf = buf;
 		t.tri = 1;
-		t.q_off[o1] = PT_FRAG * pt_slab_frags(form, t.K, n, n, 1);
+		t.fr = pt_frag_rows(n);
+		t.q_off[o1] = pt_slab_bytes(form, t.K, n, n, 1);
 		return *this;
 	}
 	pt_term done() { return t; }

@@ -411,13 +411,15 @@ struct TermP {
 	uint32_t sbytes;  /* bytes of the S rows from s */
 	int32_t nch;      /* kappa chunks */
 	uint32_t sgn;     /* sign bit to flip in S */
-	int32_t tr;       /* Q rows are w (the plane is packed transposed) */
-	int32_t pad_;
+	uint32_t lst;     /* Q bytes from a lane's u to u + 1, and << 16 from one
+	                     quarter of a row to the next */
+	int32_t lim;      /* u of the tile that have data (above 32: all) */
 };
 
 /* the term's addresses for the tile (A0, B0, C0).  A packed slab is
- * [row block of 16][chunk][column][1 KB fragment]: rows u and columns w, or
- * (tr) rows w and columns u; tri: columns 0 .. 16 (block + 1) - 1 only. */
+ * [row block of 16][chunk][column][fragment of 64 fr bytes]: rows u and
+ * columns w, or (tr) rows w and columns u; tri: columns 0 .. 16 (block + 1) -
+ * 1 only. */
 template <int F>
 __device__ __forceinline__ void
 make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
@@ -427,6 +429,7 @@ make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
 	const int na = p.na, nc = p.nc;
 	const int u0 = t.role == PT_ROLE_A ? B0 : A0;
 	const int w0 = t.role == PT_ROLE_C ? B0 : C0;
+	const int fb = 64 * t.fr;
 	const char *qb = (const char *)p.buf[t.q_buf] + t.q_off[0] * i +
 	    t.q_off[1] * j + t.q_off[2] * k;
 	for (int e = 0; e < 2; ++e) {
@@ -442,11 +445,11 @@ make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
 			off = ub * t.nch * t.cols + w0;
 			cols = t.cols;
 		}
-		o.q[e] = (uint64_t)qb + 1024 * (uint64_t)off;
-		o.dq[e] = (uint32_t)(1024 * cols);
+		o.q[e] = (uint64_t)qb + fb * (uint64_t)off;
+		o.dq[e] = (uint32_t)(fb * cols);
 	}
-	o.xa = t.tr ? 16 : 1024;
-	o.xb = t.tr ? (uint32_t)((int64_t)t.nch * t.cols * 1024) : 16 * 1024;
+	o.xa = t.tr ? 16 : fb;
+	o.xb = t.tr ? (uint32_t)((int64_t)t.nch * t.cols * fb) : 16 * fb;
 	o.s = (uint64_t)p.buf[t.s_buf] + ES * (uint64_t)(t.s_off[0] * i +
 	    t.s_off[1] * j + t.s_off[2] * k);
 	o.sst = (uint32_t)(t.s_st * ES);
@@ -454,8 +457,9 @@ make_term(const pt_launch &p, const pt_term &t, int i, int j, int k, int A0,
 	o.sbytes = (uint32_t)(sb > 0x7fffffff ? 0x7fffffff : sb);
 	o.nch = t.nch;
 	o.sgn = t.sign < 0 ? 0x80000000u : 0u;
-	o.tr = t.tr;
-	o.pad_ = 0;
+	/* lane (u, quarter): row u of the fragment, or (tr) column u */
+	o.lst = (t.tr ? fb : 16) | (uint32_t)(16 * t.fr) << 16;
+	o.lim = t.tr ? na - u0 : t.fr < 16 ? t.fr : 32;
 }
 
 /*
@@ -523,8 +527,8 @@ lds_barrier()
 template <int F, int NW, int NX, int NSB, int ROLE, class B, int NACC>
 __device__ __forceinline__ void
 run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
-    int u0, int uext, int s0, int sext, int wave, int ln, int lg,
-    uint32_t mask, char *panels, int &par)
+    int s0, int sext, int wave, int ln, int lg, uint32_t mask, char *panels,
+    int &par)
 {
 	static_assert(Form<F>::KC * sizeof(typename Form<F>::G) == 64,
 	    "a chunk of S is 64 bytes per row");
@@ -574,15 +578,14 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 		xb = (uint32_t)uni((int)T.xb);
 		sgn = (uint32_t)uni((int)T.sgn);
 		left = uni(T.nch);
-		const bool tr = uni(T.tr) != 0;
+		const uint32_t lst = (uint32_t)uni((int)T.lst);
+		const int lim = uni(T.lim);
 		q0 += (uint64_t)xa * (uint32_t)wave;
 		q1 += (uint64_t)xa * (uint32_t)wave;
 #pragma unroll
 		for (int e = 0; e < 2; ++e)
-			vo[e] = xhi[e] < 0 ? PT_OOR : !tr ?
-			    (uint32_t)(16 * (16 * lg + ln)) :
-			    u0 + 16 * e + ln < uext ?
-			    (uint32_t)(1024 * ln + 256 * lg) : PT_OOR;
+			vo[e] = xhi[e] < 0 || 16 * e + ln >= lim ? PT_OOR :
+			    __umul24(lst & 0xffff, ln) + __umul24(lst >> 16, lg);
 	};
 	/* lanes without data take an offset that every descriptor rejects; the
 	 * scalar offset is never relied on for a range check */
@@ -938,16 +941,15 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 		 * stages its part all the same) */
 		const bool w1 = m1 || FM::PAN, w2 = m2 || FM::PAN;
 		run_terms<F, NW, CW, 2, PT_ROLE_A, RoleA<GM>>(acc, tp, ts,
-		    ts + (w1 ? nta : 0), B0, na, A0, na, wave, ln, lg, m1, smem, par);
+		    ts + (w1 ? nta : 0), A0, na, wave, ln, lg, m1, smem, par);
 		run_terms<F, NW, CW, 2, PT_ROLE_B, RoleB<GM>>(acc, tp, ts + nta,
-		    ts + (w1 ? nt1 : nta), A0, na, B0, na, wave, ln, lg, m1, smem,
-		    par);
+		    ts + (w1 ? nt1 : nta), B0, na, wave, ln, lg, m1, smem, par);
 		if (FM::PAN)
 			lds_barrier();   /* the last panel's reads */
 		transpose();
 		run_terms<F, NW, BW, NCB, PT_ROLE_C, RoleC<GM>>(acc, tp, ts + nt1,
-		    ts + (w2 ? nset_terms : nt1), A0, na, C0, nc, wave, ln, lg, m2,
-		    smem, par);
+		    ts + (w2 ? nset_terms : nt1), C0, nc, wave, ln, lg, m2, smem,
+		    par);
 		if (NSET == 2 && s == 0) {
 			/* W of set 0 to the save area, lane-contiguous per (r, x,
 			 * wave); the accumulators restart for set 1 */

@@ -112,6 +112,12 @@ fake_reset_streams(void)
 	streams.clear();
 }
 
+size_t
+fake_arena(void)
+{
+	return PT_NOALLOC_ARENA;
+}
+
 void *
 fake_region(size_t bytes)
 {

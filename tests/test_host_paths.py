@@ -44,6 +44,7 @@ def lib(tmp_path_factory):
                                     [vp, vp, sz, vp])
     h.libpt_rpt.restype = ctypes.c_double
     h.libpt_rpt.argtypes = [sz] * 2 + [vp] * 7
+    h.fake_arena.restype = sz
     h.fake_region.restype = vp
     h.fake_region.argtypes = [sz]
     h.fake_region_free.argtypes = [vp, sz]
@@ -71,8 +72,8 @@ def _ijk(lib, plan, sc):
 
 @pytest.fixture
 def region(lib):
-    """1 GiB of scratch for the allocation-free call"""
-    size = 1 << 30
+    """scratch of the allocation-free call, as large as its static array"""
+    size = lib.fake_arena()
     p = lib.fake_region(size)
     yield p, size
     lib.fake_region_free(p, size)
@@ -169,6 +170,42 @@ def test_only_blocks_that_a_case_reads_are_packed(lib, call, dims, plain,
     lib.libpt_amd_plan_destroy(plan)
     assert (lib.fake_count(4) - a, lib.fake_count(5) - b) == (plain,
                                                               transposed)
+
+
+# sizes at the limit, from one virtual orbital of a spin up, and what they were
+# taken with before rows were padded: 16-fold for one orbital
+@pytest.mark.parametrize("call,form,dims", [
+    (UPT, FP64, (2, 2, 5770, 1)), (UFT, FP64, (1825, 1, 69, 19)),
+    (UFT, FP64, (3641, 1, 36, 2)), (UFT, FP64, (1, 1, 1896, 2)),
+    (UFT, FP32, (2, 2, 5752, 1)), (UPT, BF16X3, (1, 3, 257, 3)),
+    (UFT, FP64, (1, 13, 206, 17)), (UFT, FP64, (1, 33, 179, 17)),
+    (RPT, FP32, (259, 8)), (RPT, FP64, (8, 134)), (RFT, F16X3, (31, 64))])
+def test_sizes_at_the_limit_fit_the_scratch(lib, region, call, form, dims):
+    e = _noalloc(lib, call, form, dims, *region)
+    assert lib.libpt_amd_last_error() == b"" and np.isfinite(e)
+
+
+@pytest.mark.parametrize("call,form,dims", [
+    (UPT, FP64, (2, 2, 5771, 1)), (UFT, FP64, (1, 13, 207, 17)),
+    (RPT, FP64, (9, 134)), (RFT, F16X3, (32, 64))])
+def test_sizes_beyond_the_limit_are_refused(lib, region, call, form, dims):
+    assert np.isnan(_noalloc(lib, call, form, dims, *region))
+    assert b"%d bytes of static scratch" % (256 << 20) in \
+        lib.libpt_amd_last_error()
+
+
+def test_copies_leave_room_for_save_areas(lib, region):
+    """(fT): a launch holds as many items as there are save areas, so the
+    copies are left out where they would take the room of these: more
+    scratch never means more launches."""
+    most = None
+    for cap in list(range(60 << 20, 400 << 20, 4 << 20)) + [region[1]]:
+        tiles = lib.fake_count(7)
+        if not np.isnan(_noalloc(lib, RFT, FP64, (6, 64), region[0], cap)):
+            launches = lib.fake_count(7) - tiles
+            assert most is None or launches <= most, cap
+            most = launches
+    assert most == 1
 
 
 def test_ranges_of_one_plan_from_two_threads(lib):
