@@ -2169,12 +2169,20 @@ noalloc_need(const libpt_amd_plan &pl)
 	const int64_t el = form == PT_FORM_FP64 ? 8 : 4;
 	auto r = [](int64_t b) { return (b + 255) / 256 * 256; };
 	int64_t n[10], need = 512;
-	(void)api_sizes(pl.call, oa, va, ob, vb, n);
 	const int64_t R[4] = {oa, oa, ob, ob}, KT[4] = {oa, ob, ob, oa};
 	const int64_t KV[4] = {va, vb, vb, va};
 	const int64_t T[4] = {va * va, va * vb, vb * vb, vb * va};
 	const int64_t V[4] = {va * (va - 1) / 2, va * vb, vb * (vb - 1) / 2,
 	    vb * va};
+	/* sizes whose blocks alone are too large end here: counting their tiles
+	 * can take hours, and their products may not fit 64 bits */
+	double blocks = 0;
+	for (int b = 0; b < (restricted ? 2 : 4); ++b)
+		blocks += (double)(nset * el * R[b]) * ((double)KT[b] *
+		    (double)T[b] + (double)KV[b] * (double)V[b]);
+	if (blocks > (double)LIBPT_AMD_NOALLOC_SCRATCH)
+		return (int64_t)std::min(blocks, 9e18);
+	(void)api_sizes(pl.call, oa, va, ob, vb, n);
 	for (int s = 0; s < nset; ++s) {
 		if (form == PT_FORM_BF16X3 || form == PT_FORM_F16X3)
 			need += r(4 * n[3]) + r(4 * n[ft ? 6 : 4]);

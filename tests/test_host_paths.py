@@ -7,6 +7,7 @@ import ctypes
 import os
 import subprocess
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -192,6 +193,15 @@ def test_sizes_beyond_the_limit_are_refused(lib, region, call, form, dims):
     assert np.isnan(_noalloc(lib, call, form, dims, *region))
     assert b"%d bytes of static scratch" % (256 << 20) in \
         lib.libpt_amd_last_error()
+
+
+@pytest.mark.parametrize("call,dims", [(RPT, (10, 100000)),
+                                       (UFT, (1 << 20, 1 << 20, 9, 7))])
+def test_far_too_large_sizes_are_refused_at_once(lib, region, call, dims):
+    t0 = time.monotonic()
+    assert np.isnan(_noalloc(lib, call, FP64, dims, *region))
+    assert time.monotonic() - t0 < 1.0
+    assert b"static scratch" in lib.libpt_amd_last_error()
 
 
 def test_copies_leave_room_for_save_areas(lib, region):
