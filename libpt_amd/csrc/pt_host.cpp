@@ -1237,20 +1237,25 @@ plan_init(libpt_amd_plan *pl, int call, int form, size_t oa_, size_t va_,
 	return true;
 }
 
+/* may_copy: try with the transposed copies first; no_room (may be null): a
+ * plan that fails does so because its buffers do not fit */
 libpt_amd_plan *
 plan_create(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
-    const void *const *arr, bool own_wsave)
+    const void *const *arr, bool own_wsave, bool may_copy = true,
+    bool *no_room = nullptr)
 {
 	if (!dev_init())
 		return nullptr;
 	/* without the transposed copies where they leave too little memory */
 	ErrText err;
-	for (int copies = 1; copies >= 0; --copies) {
+	for (int copies = may_copy; copies >= 0; --copies) {
 		libpt_amd_plan *pl = new libpt_amd_plan;
 		pl->copies = copies != 0;
 		if (plan_init(pl, call, form, oa, va, ob, vb, arr, own_wsave))
 			return pl;
 		const bool again = copies && pl->no_room;
+		if (no_room)
+			*no_room = pl->no_room;
 		plan_free(pl);
 		if (!again)
 			break;
@@ -1764,18 +1769,11 @@ batch_free(libpt_amd_batch *b)
 	delete b;
 }
 
-} /* namespace */
-
-extern "C" libpt_amd_batch *
-libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
-    const void *const *dev_arrays)
+/* copies, no_room: as for plan_create */
+libpt_amd_batch *
+batch_build(int call, int form, int n, const int64_t *dims,
+    const void *const *dev_arrays, bool copies, bool *no_room)
 {
-	if (!dev_init())
-		return nullptr;
-	if (n <= 0 || !dims || !dev_arrays) {
-		set_err("empty batch");
-		return nullptr;
-	}
 	const bool ft = call == LIBPT_AMD_RFT || call == LIBPT_AMD_UFT;
 	const int na = ft ? 10 : 7;
 	libpt_amd_batch *b = new libpt_amd_batch;
@@ -1808,7 +1806,7 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 		const int64_t *d = dims + 4 * s;
 		libpt_amd_plan *pl = plan_create(call, form, (size_t)d[0],
 		    (size_t)d[1], (size_t)d[2], (size_t)d[3], dev_arrays + na * s,
-		    false);
+		    false, copies, no_room);
 		BFAIL(pl != nullptr);
 		pl->fixed_geometry = true;
 		b->plans.push_back(pl);
@@ -1845,9 +1843,13 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	for (int g = 0; g < nseg; ++g)
 		b->seg_of[(size_t)segs[g].sys * 4 + segs[g].sc] = g;
 	b->total = begin[nseg];
-	BFAIL(dev_alloc((void **)&b->d_segs, sizeof(pt_launch) * (nseg + 1)));
-	BFAIL(dev_alloc((void **)&b->d_begin, sizeof(int64_t) * (nseg + 1)));
-	BFAIL(dev_alloc((void **)&b->d_out, sizeof(double) * (nseg + 1)));
+	auto alloc = [&](void **p, size_t bytes) {
+		*no_room = !dev_alloc(p, bytes);
+		return !*no_room;
+	};
+	BFAIL(alloc((void **)&b->d_segs, sizeof(pt_launch) * (nseg + 1)));
+	BFAIL(alloc((void **)&b->d_begin, sizeof(int64_t) * (nseg + 1)));
+	BFAIL(alloc((void **)&b->d_out, sizeof(double) * (nseg + 1)));
 	/* systems may differ in geometry (recorded by the tuner): save
 	 * areas of the largest */
 	int64_t wbytes = 1;
@@ -1861,7 +1863,7 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 			if (pl->persist)
 				b->wslots = std::max<int64_t>(b->wslots,
 				    persist_grid(pl->nw));
-		BFAIL(dev_alloc(&b->wsave, (size_t)b->wslots * (size_t)wbytes));
+		BFAIL(alloc(&b->wsave, (size_t)b->wslots * (size_t)wbytes));
 	}
 	if (nseg > 0) {
 		BFAIL(hipMemcpy(b->d_segs, L.data(), sizeof(pt_launch) * nseg,
@@ -1905,6 +1907,31 @@ libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
 	BFAIL(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0) ==
 	    hipSuccess || (set_err("graph instantiation failed"), false));
 #undef BFAIL
+	return b;
+}
+
+} /* namespace */
+
+extern "C" libpt_amd_batch *
+libpt_amd_batch_create(int call, int form, int n, const int64_t *dims,
+    const void *const *dev_arrays)
+{
+	if (!dev_init())
+		return nullptr;
+	if (n <= 0 || !dims || !dev_arrays) {
+		set_err("empty batch");
+		return nullptr;
+	}
+	/* the copies of the first systems may leave too little memory for the
+	 * last ones or the save areas: then none of the systems has them */
+	ErrText err;
+	bool no_room = false;
+	libpt_amd_batch *b = batch_build(call, form, n, dims, dev_arrays, true,
+	    &no_room);
+	if (!b && no_room) {
+		err.back();
+		b = batch_build(call, form, n, dims, dev_arrays, false, &no_room);
+	}
 	return b;
 }
 

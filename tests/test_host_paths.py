@@ -40,6 +40,10 @@ def lib(tmp_path_factory):
     h.libpt_amd_plan_run.argtypes = [vp, ctypes.c_int, i64, i64]
     h.libpt_amd_plan_ijk_energies.argtypes = [vp, ctypes.c_int, vp]
     h.libpt_amd_last_error.restype = ctypes.c_char_p
+    h.libpt_amd_batch_create.restype = vp
+    h.libpt_amd_batch_create.argtypes = [ctypes.c_int] * 3 + [vp] * 2
+    h.libpt_amd_batch_destroy.argtypes = [vp]
+    h.libpt_amd_batch_energies.argtypes = [vp] * 2
     h.pt_noalloc_energy.restype = ctypes.c_double
     h.pt_noalloc_energy.argtypes = ([ctypes.c_int] * 2 + [sz] * 4 +
                                     [vp, vp, sz, vp])
@@ -51,8 +55,13 @@ def lib(tmp_path_factory):
     h.fake_region_free.argtypes = [vp, sz]
     h.fake_count.restype = ctypes.c_long
     h.fake_limit.argtypes = [sz]
-    yield h
-    h.fake_limit(1 << 40)
+    return h
+
+
+@pytest.fixture(autouse=True)
+def _memory(lib):
+    yield
+    lib.fake_limit(1 << 40)
 
 
 def _arrays(n=10):
@@ -156,6 +165,48 @@ def test_scratch_without_room_for_the_copies(lib, region):
         cap += 1 << 20
     assert lib.fake_count(5) == copies
     assert lib.libpt_amd_last_error() == b""
+
+
+def _batch(lib, call, form, sizes):
+    dims = np.array([(o, v, o, v) for o, v in sizes], dtype=np.int64)
+    return lib.libpt_amd_batch_create(call, form, len(sizes),
+                                      dims.ctypes.data,
+                                      _arrays(10 * len(sizes)))
+
+
+@pytest.mark.parametrize("call,form", [(RPT, FP64), (RFT, F16X3)])
+def test_batch_without_room_for_the_copies(lib, monkeypatch, call, form):
+    """Wherever memory ends, a batch that fits without the transposed copies
+    is made; one that does not is refused, and nothing stays allocated."""
+    sizes = [(5, 40), (4, 33), (6, 64), (3, 20)]
+    base = lib.fake_count(0)
+
+    def size():
+        lib.fake_limit(1 << 40)
+        b = _batch(lib, call, form, sizes)
+        used = lib.fake_count(0) - base
+        lib.libpt_amd_batch_destroy(b)
+        return used
+
+    full = size()
+    monkeypatch.setenv("LIBPT_AMD_VC_TRANSPOSED", "0")
+    bare = size()
+    monkeypatch.delenv("LIBPT_AMD_VC_TRANSPOSED")
+    assert bare < 0.9 * full
+    for q in range(21):
+        before = lib.libpt_amd_last_error()
+        lib.fake_limit(base + bare + (full - bare) * q // 20)
+        b = _batch(lib, call, form, sizes)
+        assert b and lib.libpt_amd_last_error() == before, q
+        e = np.zeros(len(sizes))
+        assert lib.libpt_amd_batch_energies(b, e.ctypes.data) == 0
+        assert list(e) == [_expected(lib, s) for s in sizes]
+        lib.libpt_amd_batch_destroy(b)
+    lib.fake_limit(base + bare - 1)
+    assert not _batch(lib, call, form, sizes)
+    assert b"hipMalloc" in lib.libpt_amd_last_error()
+    lib.fake_limit(1 << 40)
+    assert lib.fake_count(0) == base
 
 
 @pytest.mark.parametrize("call,dims,plain,transposed", [
