@@ -357,7 +357,8 @@ namespace {
 /* Idle streams of finished plans, at most IDLE_STREAMS of them (creating and
  * destroying one costs 35 us, a tenth of a small call); under g_mu.  A
  * plan's stream is idle when it is given back (plan_release synchronises
- * it). */
+ * it).  A program may have reset the device since, which ends its streams, so
+ * a handle is asked about before it is used again. */
 enum { IDLE_STREAMS = 8 };
 FixedVec<hipStream_t, IDLE_STREAMS> g_idle;
 
@@ -366,10 +367,12 @@ stream_get(hipStream_t *st)
 {
 	{
 		std::lock_guard<std::mutex> lk(g_mu);
-		if (!g_idle.empty()) {
+		while (!g_idle.empty()) {
 			*st = g_idle[g_idle.size() - 1];
 			g_idle.n--;
-			return true;
+			if (hipStreamQuery(*st) == hipSuccess)
+				return true;
+			(void)hipGetLastError(); /* a later launch check would see it */
 		}
 	}
 	return hipStreamCreateWithFlags(st, hipStreamNonBlocking) == hipSuccess;

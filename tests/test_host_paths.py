@@ -47,6 +47,8 @@ def lib(tmp_path_factory):
     h.pt_noalloc_energy.restype = ctypes.c_double
     h.pt_noalloc_energy.argtypes = ([ctypes.c_int] * 2 + [sz] * 4 +
                                     [vp, vp, sz, vp])
+    h.libpt_amd_energy.restype = ctypes.c_double
+    h.libpt_amd_energy.argtypes = [ctypes.c_int] * 2 + [sz] * 4 + [vp] * 2
     h.libpt_rpt.restype = ctypes.c_double
     h.libpt_rpt.argtypes = [sz] * 2 + [vp] * 7
     h.fake_arena.restype = sz
@@ -149,6 +151,29 @@ def test_drop_in_call_without_room_for_the_copies(lib):
         assert np.isnan(e) if nan else e == _expected(lib, (o, v))
         assert lib.libpt_amd_last_error() == b""
     assert lib.fake_count(0) == base
+
+
+def test_calls_after_a_device_reset(lib):
+    """Streams kept from earlier calls end with the device's other state: a
+    later call notices and makes its own."""
+    o, v = 3, 8
+    n = [o * v] * 3 + [2 * o * o * v * v, 2 * o * o * v * o,
+                       2 * o * o * v * v,
+                       o * v * (v * (v - 1) // 2) + o * v * v * v]
+    arr = [np.zeros(k) for k in n]
+    ptr = (ctypes.c_void_p * 7)(*[a.ctypes.data for a in arr])
+
+    def call():
+        e = lib.libpt_amd_energy(RPT, FP64, o, v, o, v, ptr, None)
+        assert e == _expected(lib, (o, v)), lib.libpt_amd_last_error()
+
+    call()
+    made, bad = lib.fake_count(2), lib.fake_count(3)
+    call()
+    assert lib.fake_count(2) == made
+    lib.fake_reset_streams()
+    call()
+    assert lib.fake_count(2) == made + 1 and lib.fake_count(3) == bad
 
 
 def test_scratch_without_room_for_the_copies(lib, region):
