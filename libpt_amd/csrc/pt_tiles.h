@@ -522,6 +522,18 @@ lds_barrier()
 	__asm__ volatile("" ::: "memory");
 }
 
+/* the x next to x in lo .. hi; of an empty range (lo > hi = -1) its lo: the
+ * scalar offset of a load is made from it, and must not be negative */
+constexpr int
+near_x(int x, int lo, int hi)
+{
+	return (x > hi ? hi : x) < lo ? lo : x > hi ? hi : x;
+}
+
+static_assert(near_x(0, 3, -1) == 3 && near_x(3, 3, -1) == 3, "empty range");
+static_assert(near_x(0, 1, 2) == 1 && near_x(3, 1, 2) == 2 &&
+    near_x(2, 1, 3) == 2, "nearest");
+
 /* panels: two panel buffers; par: the one to fill first, updated (the
  * previous call's last panel may still be read from the other) */
 template <int F, int NW, int NX, int NSB, int ROLE, class B, int NACC>
@@ -590,7 +602,7 @@ run_terms(typename Form<F>::ACC (&acc)[NACC], const TermP *tp, int t0, int t1,
 	/* lanes without data take an offset that every descriptor rejects; the
 	 * scalar offset is never relied on for a range check */
 	auto load_q = [&](int x, int e) {
-		x = x < xlo[e] ? xlo[e] : x > xhi[e] ? xhi[e] : x;
+		x = near_x(x, xlo[e], xhi[e]);
 		const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
 		    (void *)(e ? q1 : q0), (short)0, 0x7fffffff, 0x00020000);
 		return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r,
