@@ -534,6 +534,15 @@ static_assert(near_x(0, 3, -1) == 3 && near_x(3, 3, -1) == 3, "empty range");
 static_assert(near_x(0, 1, 2) == 1 && near_x(3, 1, 2) == 2 &&
     near_x(2, 1, 3) == 2, "nearest");
 
+/* orders LDS accesses of the lanes of a wave (which runs them in program
+ * order: no instruction, but the compiler keeps to it) */
+__device__ __forceinline__ void
+wave_sync()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
 /* panels: two panel buffers; par: the one to fill first, updated (the
  * previous call's last panel may still be read from the other) */
 template <int F, int NW, int NX, int NSB, int ROLE, class B, int NACC>
@@ -1091,11 +1100,15 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 	for (int n = -1; n < 8; ++n) {
 		const int ab = n >> 2, r = n & 3;
 		if constexpr (same) {
-			if (n >= 0)
+			/* other lanes of the wave read these, and read the last ones */
+			if (n >= 0) {
+				wave_sync();
 #pragma unroll
 				for (int q = 0; q < NCV1; ++q)
 					if (lane + 64 * q < NCOL)
 						scol[lane + 64 * q] = cv[q];
+				wave_sync();
+			}
 			if (n < 7) {
 				const int a = A0 + row_a((n + 1) >> 2, (n + 1) & 3, lane & 3);
 #pragma unroll
