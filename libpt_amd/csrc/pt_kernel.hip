@@ -365,9 +365,9 @@ pt_launch_pack(const struct pt_pack_job *jobs, int n, int form, void *stream)
 {
 	const hipStream_t st = (hipStream_t)stream;
 	const int el = form == PT_FORM_FP32 ? 4 : 8;
-	/* a launch takes up to PACK_JOBS jobs and 2^30 workgroups; a job of more
-	 * goes in runs of whole slabs */
-	constexpr int64_t MOST = (int64_t)1 << 30;
+	/* a launch takes up to PACK_JOBS jobs and fewer than 2^32 threads; a job
+	 * of more goes in runs of whole slabs */
+	constexpr int64_t MOST = ((int64_t)1 << 24) - 1;
 	pack_args a;
 	a.n = 0;
 	int64_t blocks = 0;

@@ -12,6 +12,7 @@
   memory for them) the same values come from the plain copies in scattered
   pieces: per-ijk energies are equal bit for bit."""
 
+import ctypes
 import os
 
 import numpy as np
@@ -94,3 +95,42 @@ def test_plain_copies_give_the_same_bits(kind, dims, form):
     assert e0 == e1
     for a, b in zip(ijk0, ijk1):
         assert np.array_equal(a, b)
+
+
+class _PackJob(ctypes.Structure):
+    """struct pt_pack_job of the engine"""
+    _fields_ = ([("src", ctypes.c_void_p), ("dst", ctypes.c_void_p)] +
+                [(n, ctypes.c_int64) for n in ("R", "K", "rows", "cols")] +
+                [("scale", ctypes.c_double), ("at", ctypes.c_int64)] +
+                [(n, ctypes.c_int32) for n in ("tri", "tr", "fr")])
+
+
+def test_more_slabs_than_one_launch_packs():
+    """More workgroups than a launch can hold (2^24 of 256 threads): the job
+    goes in runs, and the slabs at the ends of these arrive."""
+    lib = api.lib()
+    slabs, rows = (1 << 24) + 70, 2
+    src = lib.libpt_amd_dev_alloc(8 * slabs * rows)
+    dst = lib.libpt_amd_dev_alloc(64 * slabs * rows)
+    assert src and dst
+    try:
+        first = [0, (1 << 24) - 8, slabs - 8]
+        for s in first:
+            x = (1.0 + np.arange(8 * rows)) + 1000.0 * s
+            assert lib.libpt_amd_memcpy(src + 8 * rows * s, x.ctypes.data,
+                                        x.nbytes, 1) == 0
+        job = _PackJob(src=src, dst=dst, R=slabs, K=1, rows=rows, cols=1,
+                       scale=1.0)
+        print("pack", slabs, "slabs", flush=True)
+        assert lib.pt_launch_pack(ctypes.byref(job), 1, 0, None) == 0
+        for s in first:
+            # a fragment: four quarters of 2 rows, the first kappa of the
+            # first quarter is the only one
+            got = api.from_device(dst + 64 * rows * s, 8 * 8 * rows)
+            want = np.zeros((8, 4, rows, 2))
+            want[:, 0, :, 0] = (1.0 + np.arange(8 * rows) + 1000.0 * s
+                                ).reshape(8, rows)
+            assert np.array_equal(got, want.ravel()), s
+    finally:
+        lib.libpt_amd_dev_free(src)
+        lib.libpt_amd_dev_free(dst)
