@@ -1291,6 +1291,28 @@ struct Run {
  */
 constexpr int64_t MERGE_ITEMS = 8192;
 
+/*
+ * Does a range of m ijk of a case go in the list's launch order?  The order
+ * of a range is picked out of the whole list by one small kernel (0.6 ns an
+ * entry), so that work is weighed against the range's flops.  Us per range,
+ * list order -> launch order, at flops per list entry: split forms, bound by
+ * L2 and HBM, rft 40/60 F16X3 mixed spin 197 -> 219 at 4.9e5, 240 -> 256 at
+ * 7.8e5, 453 -> 437 at 1.6e6, 809 -> 746 at 3.1e6, rpt 45/100 BF16 878 ->
+ * 896 at 1.8e6, 1575 -> 1512 at 3.6e6, 5852 -> 5339 at 1.4e7; FP64 and FP32
+ * gain less: rpt 45/80 FP64 1495 -> 1527 at 1.6e6, 1772 -> 1761 at 4.7e6,
+ * 3470 -> 3447 at 9.4e6, 24/160 4562 -> 4447 at 3.8e7, 45/100 FP32 4543 ->
+ * 4559 at 7.2e6.  Short ranges of long lists lose by it: 64 ijk of the
+ * 495000 of 100/8 FP64 71 -> 332.
+ */
+bool
+range_ordered(int form, const Case &c, int64_t m)
+{
+	const double per_entry = form == PT_FORM_FP64 || form == PT_FORM_FP32 ?
+	    8e6 : 2e6;
+	return c.L.kgrp > 1 && m > c.L.kgrp &&
+	    (double)m * c.flop_per_ijk >= per_entry * (double)c.n_ijk;
+}
+
 int
 launch_runs(int form, const Run *run, int n, void *wsave, int64_t wslots,
     hipStream_t st)
@@ -1455,13 +1477,12 @@ libpt_amd_plan_run(libpt_amd_plan *pl, int sc, int64_t b, int64_t e)
 	std::lock_guard<std::mutex> lk(pl->run_mu);
 	if (c.L.nset == 2 && !plan_wsave(pl))
 		return -1;
-	/* a range of more than one group goes in the whole list's launch order
-	 * (within one group the order does not matter) */
+	/* within one group the order does not matter */
 	const int32_t *perm = nullptr;
 	int rc = 0;
 	if (b == 0 && e == c.n_ijk) {
 		perm = c.d_perm;
-	} else if (c.L.kgrp > 1 && e - b > c.L.kgrp) {
+	} else if (range_ordered(pl->form, c, e - b)) {
 		rc = pt_launch_filter(c.d_perm, c.n_ijk, (int32_t)b, (int32_t)e,
 		    c.d_part, pl->stream);
 		perm = c.d_part;

@@ -78,14 +78,15 @@ def test_ranges_of_one_plan_from_two_threads():
     """Two threads run disjoint ranges of one plan, each of more than a
     group of 32 ijk: a range's launches stay together, so the per-ijk
     energies are those of one thread."""
-    spec = api.make_spec("rpt", (9, 33), seed=2, sig_f=1e-2)
+    dims = (9, 64)
+    spec = api.make_spec("rpt", dims, seed=2, sig_f=1e-2)
     dev = api.synth_device("rpt", spec)
     errs = []
     try:
-        with api.Plan("rpt", "fp64", (9, 33), dev) as pl:
+        with api.Plan("rpt", "fp64", dims, dev) as pl:
             pl.run_all()
             ref = [pl.ijk_energies(sc) for sc in range(pl.ncases)]
-        with api.Plan("rpt", "fp64", (9, 33), dev) as pl:
+        with api.Plan("rpt", "fp64", dims, dev) as pl:
             def work(first):
                 try:
                     for sc in range(pl.ncases):

@@ -294,6 +294,27 @@ def test_copies_leave_room_for_save_areas(lib, region):
     assert most == 1
 
 
+@pytest.mark.parametrize("form,dims,width,ordered", [
+    (FP64, (12, 200), 64, 1), (BF16X3, (12, 64), 40, 1),
+    (FP64, (12, 200), 32, 0),              # one group
+    (FP64, (60, 8), 256, 0), (FP32, (60, 24), 500, 0),
+    (BF16X3, (45, 48), 40, 0), (BF16X3, (45, 48), 2000, 1)])
+def test_short_ranges_of_long_lists_go_in_list_order(lib, form, dims, width,
+                                                     ordered):
+    """Picking a range's launch order walks the whole list: only where the
+    range's work outweighs that.  Either way each ijk runs once."""
+    plan = _plan(lib, RPT, form, dims)
+    n, made = lib.libpt_amd_plan_nijk(plan, 1), lib.fake_count(6)
+    b = n // 3 + 1
+    assert lib.libpt_amd_plan_run(plan, 1, b, b + width) == 0
+    got = _ijk(lib, plan, 1)
+    lib.libpt_amd_plan_destroy(plan)
+    assert lib.fake_count(6) - made == ordered
+    want = np.zeros(n)
+    want[b:b + width] = 1.0 + np.arange(b, b + width)
+    assert np.array_equal(got, want)
+
+
 def test_ranges_of_one_plan_from_two_threads(lib):
     """Both threads make the launch order of their range before either runs
     its tiles, unless a range is one unit."""
