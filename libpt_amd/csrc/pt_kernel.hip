@@ -237,19 +237,8 @@ k_split(const double *src, uint32_t *dst, int64_t n, int fp16, double scale)
 {
 	for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
 	    t += (int64_t)gridDim.x * blockDim.x) {
-		double x = src[t] * scale;
 		uint16_t hb, lb;
-		if (fp16) {
-			_Float16 h = (_Float16)x;
-			_Float16 l = (_Float16)(x - (double)h);
-			hb = __builtin_bit_cast(uint16_t, h);
-			lb = __builtin_bit_cast(uint16_t, l);
-		} else {
-			__bf16 h = (__bf16)(float)x;
-			__bf16 l = (__bf16)(float)(x - (double)(float)h);
-			hb = __builtin_bit_cast(uint16_t, h);
-			lb = __builtin_bit_cast(uint16_t, l);
-		}
+		split2(src[t] * scale, fp16, hb, lb);
 		dst[t] = (uint32_t)hb | ((uint32_t)lb << 16);
 	}
 }
