@@ -38,9 +38,11 @@
  * the triples: 292 -> 245 ms); rpt o=20 v=120 331 -> 211 ms with 11 ms of
  * copies, FP32 upt 24/200/20/204 292 -> 184 ms, split BF16 rpt v=477 258 ->
  * 163 ms, a batch of 8 systems of v 40 to 160 198 -> 120 ms.  Bound by the
- * MFMA pipe and power in FP64 and FP32, by L1, L2 and HBM bandwidth in the
- * split forms (a wave's 16 KB of Q per 1024 MFMA cycles is the 64 bytes per
- * clock that a CU's L1 gives).
+ * MFMA pipe and power in FP64 and FP32, by L2 and HBM bandwidth in the split
+ * forms: at full MFMA rate a CU's four SIMDs would take 64 bytes of Q per
+ * clock (16 KB per wave and 1024 MFMA cycles), all that its L1 can give; L2
+ * delivers 30 to 32 bytes per clock and CU (16 to 17 TB/s), which is the .44
+ * that the pipe is busy.
  *
  * Forms: FP64 (v_mfma_f64_16x16x4_f64), FP32 (v_mfma_f32_16x16x4_f32),
  * split BF16 / FP16 (hi+lo pairs, hi*hi + lo*hi + hi*lo packed into the
@@ -1039,17 +1041,15 @@ tile_item(const pt_launch &p, int64_t it, typename Form<F>::AE *wsv,
 			const bool of_c = n >= 2 * NBV, of_a = !of_c && n >= NBV;
 			const int m = of_c ? n - 2 * NBV : of_a ? n - NBV : n;
 			const int arr = of_c ? m / TC : m / 32;
-			const int l = of_c ? C0 + m % TC : (of_a ? A0 + 0 : B0 + 0) +
-			    m % 32;
+			const int l = of_c ? C0 + m % TC : (of_a ? A0 : B0) + m % 32;
 			const int top = (of_c ? nc - 1 : na - 1), x = l < top ? l : top;
-			const int64_t d1r = of_c ? k + 0 : of_a ? i + 0 : j + 0;
-			const int64_t r1 = arr < 2 ? i + 0 : arr < 4 ? j + 0 : k + 0;
+			const int64_t d1r = of_c ? k : of_a ? i : j;
+			const int64_t r1 = arr < 2 ? i : arr < 4 ? j : k;
 			const ER *src = (arr & 1) ? f1 + r1 * p.va : u1 + r1 * p.va;
 			if (arr == NPB)
 				src = d1 + d1r * p.va;
 			if (!same && of_c)
-				src = (arr == 0 ? u2 + 0 : arr == 1 ? f2 + 0 : d2 + 0) +
-				    (int64_t)k * p.vb;
+				src = (arr == 0 ? u2 : arr == 1 ? f2 : d2) + (int64_t)k * p.vb;
 			stg[NBC + n] = src[x];
 		}
 	}
@@ -1225,8 +1225,12 @@ k_tiles(pt_launch p)
  * same-spin and mixed-spin ms): v=300 8.03 -> 8.01 and 18.6 -> 19.0, v=352
  * 12.7 -> 12.3 and 28.9 -> 28.6, v=400 23.1 -> 22.1 and 50.8 -> 50.3, v=477
  * 46.6 -> 41.2 and 94.8 -> 93.6, v=600 134 -> 101 and 238 -> 230; two W sets
- * (rft F16X3) v=256 9.1 -> 9.5 and 20.6 -> 21.3, v=350 30.3 -> 30.1 and 76.6
- * -> 76.5, v=400 56.0 -> 51.6 and 133 -> 134.  Launches of one to eight ijk
+ * (rft F16X3, other sets of ijk) v=256 9.1 -> 9.5 and 20.6 -> 21.3, v=350 30.3
+ * -> 30.1 and 76.6 -> 76.5, v=384 42.5 -> 34.7 and 77.9 -> 77.6, v=400 52.0 ->
+ * 43.9 and 102 -> 101, v=440 82.2 -> 62.2 and 143 -> 142, v=477 110 -> 82.6 and
+ * 188 -> 184, v=600 216 -> 182 and 459 -> 449; rft BF16X3 v=420 72.8 -> 56.3 and
+ * 135 -> 132, uft BF16X3 450/440 72.7 -> 66.5 and 58.8 -> 54.9).  Launches of
+ * one to eight ijk
  * share fewer slabs: from 8 % slower to 20 % faster at v=384 to 600, without
  * a trend.  At v=48 to 200 pairs cost up to 25 %, and FP64 and FP32 lose by
  * them (FP64 2 to 20 % at v=64 to 200 and 4 % at v=477, FP32 up to 16 %).
