@@ -104,7 +104,7 @@ double libpt_amd_plan_factor(const libpt_amd_plan *plan, int sc);
 int libpt_amd_plan_geometry(const libpt_amd_plan *plan, int *out3);
 
 /* enqueue ijk items [ijk_begin, ijk_end) of spin case sc on the plan's
- * stream; 0 on success */
+ * stream; 0 on success.  Several threads may run ranges of one plan. */
 int libpt_amd_plan_run(libpt_amd_plan *plan, int sc, int64_t ijk_begin,
     int64_t ijk_end);
 int libpt_amd_plan_sync(libpt_amd_plan *plan);
