@@ -798,18 +798,31 @@ family_scale(libpt_amd_plan *pl, const double *const *arr, const int64_t *n,
 
 namespace {
 
-/* two W sets: the save areas of one launch's items, sized to all spin
- * cases (at most pt_ft_chunk); no-op when present */
+/* items that share a tile launch (launch_runs) */
+constexpr int64_t MERGE_ITEMS = 8192;
+
+/* two W sets: the items of the largest launch, which runs one spin case
+ * (largest) or small ones together (all: the items of all of them) */
+int64_t
+launch_items(int64_t largest, int64_t all)
+{
+	return std::max<int64_t>(1, std::max(largest, std::min(all, MERGE_ITEMS)));
+}
+
+/* two W sets: the save areas of one launch's items (at most pt_ft_chunk);
+ * no-op when present */
 bool
 plan_wsave(libpt_amd_plan *pl)
 {
 	if (pl->wsave)
 		return true;
-	int64_t most = 0;
-	for (const Case &d : pl->cases)
-		most += d.n_ijk * d.n_tiles;
-	most = std::max<int64_t>(most, 1);
-	int64_t slots = std::min<int64_t>(pt_ft_chunk(pl->form, pl->nw), most);
+	int64_t largest = 0, all = 0;
+	for (const Case &d : pl->cases) {
+		largest = std::max(largest, d.n_ijk * d.n_tiles);
+		all += d.n_ijk * d.n_tiles;
+	}
+	int64_t slots = std::min<int64_t>(pt_ft_chunk(pl->form, pl->nw),
+	    launch_items(largest, all));
 	const int64_t wb = pt_wsave_bytes(pl->form, 2, pl->nw);
 	if (pl->persist)
 		/* one area per workgroup of the grid, whatever the item count */
@@ -1281,17 +1294,6 @@ struct Run {
 };
 
 /*
- * The tile launches of some runs of one geometry: grids of at most 2^22
- * items, and with two W sets of at most wslots (one save area per item).
- * Small runs share a launch, up to PT_MAX_SEGS of them and MERGE_ITEMS items:
- * each is a fraction of the GPU or a few rounds of it, and they run side by
- * side or fill each other's ends (the two launches of a rpt 5/19 call took 50
- * us each).  Larger ones gain nothing by it, and the kernel that holds both
- * spin cases is 3 % slower per item (rpt v=477 FP64 245 -> 252 ms).
- */
-constexpr int64_t MERGE_ITEMS = 8192;
-
-/*
  * Does a range of m ijk of a case go in the list's launch order?  The order
  * of a range is picked out of the whole list by one small kernel (0.6 ns an
  * entry), so that work is weighed against the range's flops.  Us per range,
@@ -1313,6 +1315,15 @@ range_ordered(int form, const Case &c, int64_t m)
 	    (double)m * c.flop_per_ijk >= per_entry * (double)c.n_ijk;
 }
 
+/*
+ * The tile launches of some runs of one geometry: grids of at most 2^22
+ * items, and with two W sets of at most wslots (one save area per item).
+ * Small runs share a launch, up to PT_MAX_SEGS of them and MERGE_ITEMS items:
+ * each is a fraction of the GPU or a few rounds of it, and they run side by
+ * side or fill each other's ends (the two launches of a rpt 5/19 call took 50
+ * us each).  Larger ones gain nothing by it, and the kernel that holds both
+ * spin cases is 3 % slower per item (rpt v=477 FP64 245 -> 252 ms).
+ */
 int
 launch_runs(int form, const Run *run, int n, void *wsave, int64_t wslots,
     hipStream_t st)
@@ -1880,8 +1891,11 @@ batch_build(int call, int form, int n, const int64_t *dims,
 	for (const libpt_amd_plan *pl : b->plans)
 		wbytes = std::max(wbytes, pt_wsave_bytes(form, 2, pl->nw));
 	if (b->nset == 2 && b->total > 0) {
-		const int64_t most = std::max<int64_t>(1, b->total);
-		b->wslots = std::min<int64_t>(((int64_t)4 << 30) / wbytes, most);
+		int64_t largest = 0;
+		for (const Seg &g : segs)
+			largest = std::max(largest, g.items);
+		b->wslots = std::min<int64_t>(((int64_t)4 << 30) / wbytes,
+		    launch_items(largest, b->total));
 		/* a persistent grid keeps one area per workgroup */
 		for (const libpt_amd_plan *pl : b->plans)
 			if (pl->persist)

@@ -234,6 +234,22 @@ def test_batch_without_room_for_the_copies(lib, monkeypatch, call, form):
     assert lib.fake_count(0) == base
 
 
+def test_save_areas_of_a_batch_fit_its_largest_launch(lib):
+    """24 small (fT) systems: spin cases share launches of up to 8192 items, so
+    that many areas of 128 KB beside the systems' own 75 MB each, and not one
+    for each of the batch's items."""
+    sizes = [(6, 64)] * 24
+    base = lib.fake_count(0)
+    tiles = lib.fake_count(7)
+    b = _batch(lib, RFT, FP64, sizes)
+    assert b and lib.fake_count(7) > tiles
+    assert lib.fake_count(0) - base < (8192 << 17) + 24 * (76 << 20)
+    e = np.zeros(len(sizes))
+    assert lib.libpt_amd_batch_energies(b, e.ctypes.data) == 0
+    assert list(e) == [_expected(lib, s) for s in sizes]
+    lib.libpt_amd_batch_destroy(b)
+
+
 @pytest.mark.parametrize("call,dims,plain,transposed", [
     (RPT, (4, 5), 4, 3), (RPT, (2, 5), 4, 2), (UPT, (4, 5, 3, 6), 8, 6),
     # no case reads the second spin's own blocks: its pairs have no orbitals
