@@ -2506,9 +2506,10 @@ host_call(int call, int form, size_t oa, size_t va, size_t ob, size_t vb,
 				const int64_t en = nijk * (p + 1) / parts;
 				ok = libpt_amd_plan_run(pl, sc, b, en) == 0 &&
 				    libpt_amd_plan_sync(pl) == 0;
-				fprintf(stderr, "[libpt_amd] spin case %d: ijk %lld of "
-				    "%lld done, %.1f s\n", sc, (long long)en,
-				    (long long)nijk, now_s() - t2);
+				if (ok)
+					fprintf(stderr, "[libpt_amd] spin case %d: ijk %lld of "
+					    "%lld done, %.1f s\n", sc, (long long)en,
+					    (long long)nijk, now_s() - t2);
 			}
 		}
 		if (ok)

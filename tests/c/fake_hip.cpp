@@ -34,7 +34,7 @@ long next_handle = 1;
 long created = 0, bad = 0;           /* streams made; uses of a dead one */
 long packs[2] = {0, 0};              /* pack jobs: plain, transposed */
 long filters = 0, tiles = 0;
-bool energy_nan = false;
+bool energy_nan = false, tiles_fail = false;
 
 /* filters in flight of a test with two threads: the first waits for the
  * second one, or 0.3 s */
@@ -94,6 +94,12 @@ void
 fake_nan(int on)
 {
 	energy_nan = on != 0;
+}
+
+void
+fake_fail_tiles(int on)
+{
+	tiles_fail = on != 0;
 }
 
 void
@@ -298,8 +304,8 @@ pt_launch_tiles(int form, const struct pt_launch *p, int n, void *stream)
 {
 	(void)form;
 	const hipError_t e = use((hipStream_t)stream);
-	if (e != hipSuccess)
-		return (int)e;
+	if (e != hipSuccess || tiles_fail)
+		return e ? (int)e : (int)hipErrorUnknown;
 	for (int q = 0; q < n; ++q)
 		for (int64_t t = 0; t < p[q].n_chunk; ++t) {
 			const int64_t it = item_of(p[q], t);

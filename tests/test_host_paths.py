@@ -176,6 +176,24 @@ def test_calls_after_a_device_reset(lib):
     assert lib.fake_count(2) == made + 1 and lib.fake_count(3) == bad
 
 
+def test_progress_lines_name_what_was_done(lib, monkeypatch, capfd):
+    o, v = 4, 8
+    n = [o * v] * 3 + [2 * o * o * v * v, 2 * o * o * v * o,
+                       2 * o * o * v * v,
+                       o * v * (v * (v - 1) // 2) + o * v * v * v]
+    arr = [np.zeros(k) for k in n]
+    ptr = (ctypes.c_void_p * 7)(*[a.ctypes.data for a in arr])
+    monkeypatch.setenv("LIBPT_AMD_PROGRESS", "1")
+    for fail in (0, 1):
+        lib.fake_fail_tiles(fail)
+        e = lib.libpt_amd_energy(RPT, FP64, o, v, o, v, ptr, None)
+        lib.fake_fail_tiles(0)
+        lines = capfd.readouterr().err.count("done")
+        # 16 parts a spin case; of 4 ijk the first three parts are empty
+        assert (np.isnan(e), lines) == ((True, 3) if fail else
+                                        (False, 32)), lines
+
+
 def test_scratch_without_room_for_the_copies(lib, region):
     """The allocation-free call drops the copies where its scratch ends."""
     dims = (6, 40)
